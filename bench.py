@@ -108,7 +108,14 @@ def spmv_only(args):
         ops.rec_pack(cl[0], z64, r1)
         cases["matfree_rec_f64_cheb"] = lambda: ops.matfree_rec(r0, r1, r2, cl[1], rent, A.plus_i, s1=0.1, c0=2.0,
                                                                 c2=1.0, acc=acc_r, mu=0.01)
-        out["bytes_per_launch"]["k_matfree_rec<true>"] = int(kernel_bytes("mf64rec", A, "cheb"))
+        out["bytes_per_launch"]["k_matfree_rec<true>"] = 4 * rent.numel() + 8 * cl[1].numel() + 144 * cl[0].numel()
+    if A.tiles() is not None:
+        T = A.tiles()
+        t0, t1, t2 = T.buffers(3)
+        tacc = torch.zeros(3 * T.slots, dtype=torch.float64, device="cuda")
+        cases["matfree_tile_f64_cheb"] = lambda: T.product(t0, t1, t2, A.plus_i, s1=0.1, c0=2.0, c2=1.0, acc=tacc,
+                                                           mu=0.1)
+        out["bytes_per_launch"][kernel_key("mf64rec", A)] = int(kernel_bytes("mf64rec", A, "cheb"))
     for name, fn in cases.items():
         for _ in range(3):
             fn()
@@ -517,12 +524,16 @@ def kernel_bytes(kind, A, epi):
     nnzb, n_atoms = A.nnzb, A.n_atoms
     nd = 3 * n_atoms
     if kind == "mf64rec":
-        # record form: lists (slot words) + cluster pointers, every slot's record (coordinates
-        # and x, 48 B) read, and per slot 24 B of z read, 24 B of output written, 48 B of the
-        # accumulator read and written
+        # slot order: every slot's record (coordinates and x, 48 B) read, and per slot 24 B of z
+        # read, 24 B of output written, 48 B of the accumulator read and written; the tile
+        # form's lists (union words, wave headers, pair blocks) or the record form's (slot
+        # words, cluster pointers)
+        if A.tiles() is not None:
+            T = A.tiles()
+            lists = 4 * int(T.ulen.sum()) + 4 * T.ulen.numel() + 4 * T.waves.numel() + T.pairs.numel()
+            return lists + (144 if epi == "cheb" else 72) * T.slots
         _, ptr, _, ent = A.clusters()
-        slots = 4 * (ptr.numel() - 1)
-        return 4 * ent.numel() + 8 * ptr.numel() + (144 if epi == "cheb" else 72) * slots
+        return 4 * ent.numel() + 8 * ptr.numel() + (144 if epi == "cheb" else 72) * 4 * (ptr.numel() - 1)
     if kind == "f32":
         s, sv = 4, 4 if epi == "cheb" else 8
         return 9 * s * nnzb + (5 if epi == "cheb" else 2) * nd * sv
@@ -540,14 +551,15 @@ def kernel_bytes(kind, A, epi):
 KERNEL_DESC = {"f32": "block SpMV, fp32 values, Chebyshev epilogue",
                "f64": "block SpMV, fp64 values, Chebyshev epilogue",
                "mf64": "matrix-free fp64 ANM product, Chebyshev epilogue",
-               "mf64rec": "matrix-free fp64 ANM product on cluster-order records, Chebyshev epilogue"}
+               "mf64rec": "matrix-free fp64 ANM product in slot order, Chebyshev epilogue"}
 
 
 def kernel_key(kind, A):
     """Template name of the operator kernel the autotuner picked for this matrix."""
     from inching_amd.autotune import best_config
     if kind == "mf64rec":
-        return "k_matfree_rec<true>"
+        T = A.tiles()
+        return "k_matfree_rec<true>" if T is None else "k_matfree_tile<%d,%d,false>" % T.shape
     cfg = best_config(A, kind)
     if kind == "mf64":
         c, f = cfg % 1000, cfg // 1000

@@ -51,6 +51,13 @@ SIGNATURES = {
     "inch_anm_records": (_STATUS, [_i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "inch_anm_matfree_rec": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _vp, _vp, _dbl, _dbl, _dbl, _dbl, _vp, _dbl, _i32,
                                        _vp]),
+    "inch_anm_tile_order": (_STATUS, [_i64, _vp, _dbl, _i32, _vp, _vp, _vp, _vp]),
+    "inch_anm_tiles": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _dbl, _dbl, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
+                                 _i32, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
+    "inch_anm_matfree_tile": (_STATUS, [_i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp, _dbl,
+                                        _dbl, _dbl, _dbl, _dbl, _dbl, _vp, _dbl, _vp]),
+    "inch_anm_chebyshev_tile": (_STATUS, [_i64, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _dbl, _dbl, _vp, _vp, _i32, _i32,
+                                          _vp, _vp, _dbl, _dbl, _dbl, _vp, _vp]),
     "inch_rec_pack": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _dbl, _vp]),
     "inch_rec_unpack": (_STATUS, [_i64, _vp, _vp, _vp, _vp]),
     "inch_anm_matfree_cl": (_STATUS, [_i64, _vp, _i64, _vp, _vp, _vp, _vp, _dbl, _i32, _vp, _vp, _dbl, _dbl, _vp,

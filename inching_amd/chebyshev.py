@@ -349,7 +349,7 @@ class KPMCounter:
     come from degree / 2 operator launches (fused Chebyshev steps) by the doubling relations
     mu_2k = 2 <T_k v, T_k v> - mu_0 and mu_2k-1 = 2 <T_k v, T_k-1 v> - mu_1 (two dots per
     step; an odd degree takes one more launch). With the matrix-free operator the recurrence
-    runs on the cluster-order records (the probe is drawn in the matrix's order, as otherwise,
+    runs on records in slot order (the probe is drawn in the matrix's order, as otherwise,
     and packed) and the dots on their slot-order outputs, whose padding slots are zero."""
 
     def __init__(self, A, bound, degree=64, probes=1, seed=0, precision="mf64"):
@@ -365,7 +365,7 @@ class KPMCounter:
         g = torch.Generator(device=dev)
         g.manual_seed(int(seed))
         ws = ops.Workspace(1, dev)
-        rec = A.records() if precision == "mf64" and getattr(A, "images", None) is None else None
+        rec = A.slot_form() if precision == "mf64" else None
         if rec is not None:
             self._dots_on_records(A, rec, g, probes, half, dots, ws)
         else:
@@ -386,10 +386,8 @@ class KPMCounter:
     def _dots_on_records(self, A, rec, g, probes, half, dots, ws):
         """dots[p, 2k] = <T_k v, T_k v>, dots[p, 2k - 1] = <T_k v, T_k-1 v> for probe p, the
         recurrence on three record buffers in turn, T_k v in slot order from each step."""
-        recs, rent = rec
-        atoms, ptr = A.clusters()[:2]
-        ncl = ptr.numel() - 1
-        ys = [torch.empty(12 * ncl, dtype=torch.float64, device=A.device) for _ in range(2)]
+        recs, atoms = rec.buffers(3), rec.atoms
+        ys = [torch.empty(3 * rec.slots, dtype=torch.float64, device=A.device) for _ in range(2)]
         for p in range(probes):
             v = torch.randn(self.n, generator=g, dtype=torch.float64, device=A.device)
             v /= torch.linalg.norm(v)
@@ -399,9 +397,9 @@ class KPMCounter:
                 nxt = free.pop(0)
                 y, y_prev = ys[k % 2], ys[(k - 1) % 2]
                 if k == 1:
-                    ops.matfree_rec(cur, None, nxt, ptr, rent, A.plus_i, s1=1.0 / self.dd, c0=self.cc, y=y)
+                    rec.product(cur, None, nxt, A.plus_i, s1=1.0 / self.dd, c0=self.cc, y=y)
                 else:
-                    ops.matfree_rec(cur, prev, nxt, ptr, rent, A.plus_i, s1=2.0 / self.dd, c0=self.cc, c2=1.0, y=y)
+                    rec.product(cur, prev, nxt, A.plus_i, s1=2.0 / self.dd, c0=self.cc, c2=1.0, y=y)
                 ops.multidot(y.view(1, -1), 1, y, dots[p, 2 * k:2 * k + 1], ws)
                 ops.multidot(y_prev.view(1, -1), 1, y, dots[p, 2 * k - 1:2 * k], ws)
                 if prev is not None:
@@ -495,13 +493,13 @@ def spectrum_bound(A, n_tridiag=300, seed=0, precision="f64", stop_rel=None, inf
         A.ensure(precision)
     n = A.shape[0]
     dev = A.device
-    # with the matrix-free operator the run can stay in the record layout's slot order (the
-    # Ritz values do not depend on the numbering): vectors of 12 ncl entries, zero on
+    # with the matrix-free operator the run can stay in slot order (the
+    # Ritz values do not depend on the numbering): vectors of 3 entries per slot, zero on
     # padding slots (whose rows are zero), one pack into a record per product
-    rec = A.records() if precision == "mf64" and getattr(A, "images", None) is None else None
+    rec = A.slot_form() if precision == "mf64" else None
     if rec is not None:
-        atoms, ptr = A.clusters()[:2]
-        n = 3 * atoms.numel()
+        atoms, n = rec.atoms, 3 * rec.slots
+        buf = rec.buffers(1)[0]
     g = torch.Generator(device=dev)
     g.manual_seed(int(seed))
     v = torch.rand(n, generator=g, dtype=torch.float64, device=dev) - 0.5
@@ -522,8 +520,8 @@ def spectrum_bound(A, n_tridiag=300, seed=0, precision="f64", stop_rel=None, inf
 
     def av(x, y):
         if rec is not None:
-            ops.rec_pack(None, x, rec[0][0], ncl=ptr.numel() - 1)
-            ops.matfree_rec(rec[0][0], None, None, ptr, rec[1], A.plus_i, y=y)
+            ops.rec_pack(None, x, buf, ncl=rec.slots // ops.CLUSTER_ATOMS)
+            rec.product(buf, None, None, A.plus_i, y=y)
         elif vals is None:
             A.matfree_spmv(x, y, config=cfg)
         else:

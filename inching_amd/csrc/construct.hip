@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "scan.h"
+#include "tile.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -714,6 +715,312 @@ __global__ void __launch_bounds__(256) k_rec_lists(int64_t ncl, const int64_t *_
   for (int e = threadIdx.x; e < len; e += blockDim.x) out[e0 + e] = key[e];
 }
 
+// ---- tile form of the matrix-free operator (the operator's Chebyshev recurrence) ----
+// Atoms are numbered by slots: sorted along columns of side x side in x and y (boustrophedon
+// over the columns and along z, so that consecutive tiles stay close across a turn), every
+// column cut into equal tiles of at most TA atoms, inside a tile by falling row length (a wave
+// of the product runs as many passes as its longest row needs). A tile that spans two columns
+// would be long and its union large (up to 1.6 times, and beyond the limit where a column
+// crosses several parts of an assembly); the equal shares leave 3% of the slots empty in a
+// 300,000-atom globule. A tile lists the union of its atoms' neighbours once; each atom then
+// lists its own as 16-bit offsets into that union.
+
+// Order of the atoms: (column, place along it) in 64 bits, sorted stably with the atom index.
+__global__ void k_tile_keys(int64_t n, const double *__restrict__ xyz, CGrid g, double zscale,
+                            uint64_t *__restrict__ key, int32_t *__restrict__ atom) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t cx = cell_coord(xyz[3 * i], g.lo[0], g.inv[0], g.dim[0]);
+  int64_t cy = cell_coord(xyz[3 * i + 1], g.lo[1], g.inv[1], g.dim[1]);
+  if (cx & 1) cy = g.dim[1] - 1 - cy;
+  const int64_t c = cx * g.dim[1] + cy;
+  const double f = (xyz[3 * i + 2] - g.lo[2]) * zscale;   // 0 .. 2^32 - 1
+  uint32_t z = f < 4294967295.0 ? (uint32_t)f : 0xffffffffu;
+  if (c & 1) z = ~z;
+  key[i] = ((uint64_t)c << 32) | z;
+  atom[i] = (int32_t)i;
+}
+
+// head[i] = 1 where a new column begins in the sorted keys
+__global__ void k_tile_heads(int64_t n, const uint64_t *__restrict__ key, int32_t *__restrict__ head) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < n) head[i] = i == 0 || (key[i] >> 32) != (key[i - 1] >> 32);
+}
+
+// first[c] = where column c begins (first[columns] = n); cidx: exclusive scan of head
+__global__ void k_tile_first(int64_t n, const int32_t *__restrict__ head, const int32_t *__restrict__ cidx,
+                             int32_t *__restrict__ first) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < n && head[i]) first[cidx[i]] = (int32_t)i;
+  if (i == 0) first[cidx[n]] = (int32_t)n;
+}
+
+// tiles of column c (0 beyond the last column)
+__global__ void k_tile_column(int64_t n, int TA, const int32_t *__restrict__ cidx, const int32_t *__restrict__ first,
+                              int32_t *__restrict__ tiles) {
+  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (c < n) tiles[c] = c < cidx[n] ? (first[c + 1] - first[c] + TA - 1) / TA : 0;
+}
+
+// tile_start of every tile of column c: the column's atoms in equal shares
+__global__ void k_tile_cut(int64_t n, const int32_t *__restrict__ cidx, const int32_t *__restrict__ first,
+                           const int32_t *__restrict__ base, int32_t *__restrict__ tile_start) {
+  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (c >= cidx[n]) return;
+  const int64_t b = first[c], len = first[c + 1] - b, t0 = base[c], K = base[c + 1] - t0;
+  for (int64_t k = 0; k < K; ++k) tile_start[t0 + k] = (int32_t)(b + len * k / K);
+  if (c == cidx[n] - 1) tile_start[t0 + K] = (int32_t)n;
+}
+
+// The image masks of an entry with a term: bits of the images at a nonzero distance (open
+// boundaries: bit 4, the unshifted one). far |= 1 when a distance leaves the range in which
+// the product's float32 reciprocal seed is normal.
+template <bool PBC>
+__device__ __forceinline__ uint32_t tile_images(const double *__restrict__ xyz, int64_t i, int64_t j,
+                                                const uint16_t *__restrict__ images, int64_t e, double bx, double by,
+                                                int &far) {
+  uint32_t m = PBC ? (uint32_t)images[e] & 511u : 16u, keep = 0;
+  while (m) {
+    const int bit = __ffs(m) - 1;
+    m &= m - 1;
+    const double sx = PBC ? (double)(bit / 3 - 1) * bx : 0.0, sy = PBC ? (double)(bit % 3 - 1) * by : 0.0;
+    const double d0 = (xyz[3 * j] + sx) - xyz[3 * i], d1 = (xyz[3 * j + 1] + sy) - xyz[3 * i + 1];
+    const double d2 = xyz[3 * j + 2] - xyz[3 * i + 2];
+    const double r2 = __builtin_fma(d2, d2, __builtin_fma(d1, d1, d0 * d0));
+    if (r2 > 0.0) {
+      keep |= 1u << bit;
+      if (!(r2 > 1e-30 && r2 < 1e30)) far = 1;
+    }
+  }
+  return keep;
+}
+
+// cnt[i] = terms of atom i (entries times their images); one 16-lane group per row. Flags:
+// bit 3 a column outside [0, n), bit 4 a distance outside the float32 seed's range.
+template <bool PBC>
+__global__ void __launch_bounds__(256) k_tile_count(int64_t n, const double *__restrict__ xyz,
+                                                    const int64_t *__restrict__ rowptr,
+                                                    const int32_t *__restrict__ col,
+                                                    const uint16_t *__restrict__ images, double bx, double by,
+                                                    int32_t *__restrict__ cnt, int32_t *__restrict__ flags) {
+  const int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 4;
+  const int lane = threadIdx.x & 15;
+  if (i >= n) return;
+  int32_t c = 0;
+  int far = 0;
+  for (int64_t e = rowptr[i] + lane; e < rowptr[i + 1]; e += 16) {
+    const int32_t j = col[e];
+    if (j < 0 || j >= n) {
+      atomicOr(flags, 8);
+      continue;
+    }
+    c += __popc(tile_images<PBC>(xyz, i, j, images, e, bx, by, far));
+  }
+  if (far) atomicOr(flags, 16);
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) c += __shfl_xor(c, off, 16);
+  if (lane == 0) cnt[i] = c;
+}
+
+// One 64-thread block per tile: its atoms by falling term count (ties by place), the slot of
+// every atom, and per wave of 64 / G atoms its passes (terms of its longest row / G) and its
+// blocks of 8 passes.
+__global__ void __launch_bounds__(64) k_tile_slots(int TA, int G, const int32_t *__restrict__ sorted,
+                                                   const int32_t *__restrict__ tile_start,
+                                                   const int32_t *__restrict__ cnt, int32_t *__restrict__ tile_atoms,
+                                                   int32_t *__restrict__ slot_of, int32_t *__restrict__ passes,
+                                                   int32_t *__restrict__ blocks) {
+  __shared__ int32_t ca[64], cc[64];
+  const int64_t t = blockIdx.x;
+  const int q = threadIdx.x;
+  const int64_t at = (int64_t)tile_start[t] + q;
+  int32_t a = -1, c = -1;
+  if (q < TA && at < tile_start[t + 1]) {
+    a = sorted[at];
+    c = cnt[a];
+  }
+  ca[q] = c;
+  __syncthreads();
+  int r = 0;
+  if (q < TA) {
+    for (int p = 0; p < TA; ++p) r += ca[p] > c || (ca[p] == c && p < q);
+    tile_atoms[t * TA + r] = a;
+    if (a >= 0) slot_of[a] = (int32_t)(t * TA + r);
+    cc[r] = c;
+  }
+  __syncthreads();
+  const int AW = 64 / G, NW = TA / AW;
+  if (q < NW) {
+    const int32_t top = cc[q * AW];           // falling: the wave's first atom has the most terms
+    const int32_t p = top > 0 ? (top + G - 1) / G : 0;
+    passes[t * NW + q] = p;
+    blocks[t * NW + q] = (p + 7) / 8;
+  }
+}
+
+// waves[w] = (first block, passes) of wave w
+__global__ void k_tile_waves(int64_t nw, const int32_t *__restrict__ ptr, const int32_t *__restrict__ passes,
+                             int2 *__restrict__ waves) {
+  const int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (w < nw) waves[w] = make_int2(ptr[w], passes[w]);
+}
+
+constexpr int kTileHash = 4096;   // slots of the union's hash table: at least 3 x the largest union
+
+// One block per tile. The (neighbour slot, image) words of its rows go into an LDS hash
+// table; the distinct ones, sorted, are the tile's union (written as 48 slot | image: the
+// byte offset of the neighbour's record, the image in its low 4 bits). Then a wave per row
+// writes its terms as 16-bit byte offsets 48 p of their places p in the union, term number q
+// of an atom at pass q / G, lane q % G of its G lanes, 8 passes to a block of 64 lanes x 16
+// bytes. Passes that a row does not fill name the atom's own dummy record 48 (union + atom),
+// whose term is zero. flags bit 0: the union exceeds ucap.
+template <bool PBC>
+__global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, const double *__restrict__ xyz,
+                                                   const int64_t *__restrict__ rowptr,
+                                                   const int32_t *__restrict__ col,
+                                                   const uint16_t *__restrict__ images, double bx, double by,
+                                                   const int32_t *__restrict__ tile_atoms,
+                                                   const int32_t *__restrict__ slot_of, const int2 *__restrict__ waves,
+                                                   int ucap, int32_t *__restrict__ ulen, uint32_t *__restrict__ ulist,
+                                                   uint16_t *__restrict__ pairs, int32_t *__restrict__ flags,
+                                                   int32_t *__restrict__ umax) {
+  __shared__ uint32_t hkey[kTileHash];
+  __shared__ uint16_t hpos[kTileHash];
+  __shared__ uint32_t list[2048];
+  __shared__ int s_n;
+  const int64_t t = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  constexpr uint32_t kEmpty = 0xffffffffu;
+  for (int q = tid; q < kTileHash; q += 256) hkey[q] = kEmpty;
+  if (tid == 0) s_n = 0;
+  __syncthreads();
+  auto place = [](uint32_t k) { return (k * 2654435761u) >> 20; };   // 12 bits
+  int far = 0;
+  for (int a = w; a < TA; a += 4) {
+    const int32_t i = tile_atoms[t * TA + a];
+    if (i < 0) continue;
+    for (int64_t e = rowptr[i] + lane; e < rowptr[i + 1]; e += 64) {
+      const int32_t j = col[e];
+      uint32_t m = tile_images<PBC>(xyz, i, j, images, e, bx, by, far);
+      while (m) {
+        const int bit = __ffs(m) - 1;
+        m &= m - 1;
+        const uint32_t k = ((uint32_t)slot_of[j] << 4) | (uint32_t)bit;
+        uint32_t h = place(k);
+        // the table never fills: a thread stops once more than ucap words are in, so at most
+        // ucap + 256 < kTileHash are
+        while (*(volatile int *)&s_n <= ucap) {
+          const uint32_t old = atomicCAS(&hkey[h], kEmpty, k);
+          if (old == k) break;
+          if (old == kEmpty) {
+            atomicAdd(&s_n, 1);
+            break;
+          }
+          h = (h + 1) & (kTileHash - 1);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const int ul = s_n;
+  if (ul > ucap) {   // uniform
+    if (tid == 0) {
+      atomicOr(flags, 1);
+      ulen[t] = 0;
+    }
+    return;
+  }
+  __syncthreads();
+  if (tid == 0) s_n = 0;
+  __syncthreads();
+  for (int q = tid; q < kTileHash; q += 256)
+    if (hkey[q] != kEmpty) list[atomicAdd(&s_n, 1)] = hkey[q];
+  int p2 = 1;
+  while (p2 < ul) p2 <<= 1;
+  __syncthreads();
+  for (int q = ul + tid; q < p2; q += 256) list[q] = kEmpty;
+  __syncthreads();
+  for (int k = 2; k <= p2; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int q = tid; q < p2 / 2; q += 256) {
+        const int lo = 2 * j * (q / j) + q % j, hi = lo + j;
+        const uint32_t x = list[lo], y = list[hi];
+        if ((x > y) == ((lo & k) == 0)) {
+          list[lo] = y;
+          list[hi] = x;
+        }
+      }
+      __syncthreads();
+    }
+  for (int q = tid; q < ul; q += 256) {
+    const uint32_t k = list[q];
+    uint32_t h = place(k);
+    while (hkey[h] != k) h = (h + 1) & (kTileHash - 1);
+    hpos[h] = (uint16_t)q;
+    ulist[t * ucap + q] = 48u * (k >> 4) | (k & 15u);
+  }
+  if (tid == 0) {
+    ulen[t] = ul;
+    atomicMax(umax, ul);
+  }
+  __syncthreads();
+  const int AW = 64 / G, NW = TA / AW;
+  for (int a = w; a < TA; a += 4) {
+    const int32_t i = tile_atoms[t * TA + a];
+    const int2 wv = waves[t * NW + a / AW];
+    uint16_t *out = pairs + 512 * (int64_t)wv.x;
+    const int l0 = (a % AW) * G, room = 8 * G * ((wv.y + 7) / 8);
+    auto put = [&](int q, uint32_t p) {   // term q of the atom
+      const int pass = q / G;
+      out[((pass >> 3) * 64 + l0 + q % G) * 8 + (pass & 7)] = (uint16_t)(48u * p);
+    };
+    int done = 0;
+    if (i >= 0) {
+      const int64_t e1 = rowptr[i + 1];
+      for (int64_t e0 = rowptr[i]; e0 < e1; e0 += 64) {
+        const int64_t e = e0 + lane;
+        uint32_t m = 0;
+        uint32_t s = 0;
+        if (e < e1) {
+          const int32_t j = col[e];
+          m = tile_images<PBC>(xyz, i, j, images, e, bx, by, far);
+          s = (uint32_t)slot_of[j];
+        }
+        int c = __popc(m), inc = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const int v = __shfl_up(inc, off, 64);
+          if (lane >= off) inc += v;
+        }
+        int q = done + inc - c;
+        while (m) {
+          const int bit = __ffs(m) - 1;
+          m &= m - 1;
+          const uint32_t k = (s << 4) | (uint32_t)bit;
+          uint32_t h = place(k);
+          while (hkey[h] != k) h = (h + 1) & (kTileHash - 1);
+          if (q < room) put(q, hpos[h]);   // always, by the count that sized the blocks
+          ++q;
+        }
+        done += __shfl(inc, 63, 64);
+      }
+    }
+    for (int q = done + lane; q < room; q += 64) put(q, (uint32_t)(ul + a));
+  }
+}
+
+// rec[6 q .. 6 q + 2] = coordinates of slot q (zeros for a padding slot), rec[6 q + 3 ..] = 0
+__global__ void k_tile_coords(int64_t slots, const int32_t *__restrict__ tile_atoms, const double *__restrict__ xyz,
+                              double *__restrict__ rec) {
+  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (q >= slots) return;
+  const int32_t at = tile_atoms[q];
+  for (int k = 0; k < 3; ++k) {
+    rec[6 * q + k] = at >= 0 ? xyz[3 * (int64_t)at + k] : 0.0;
+    rec[6 * q + 3 + k] = 0.0;
+  }
+}
+
 struct DevBuf {
   void *p = nullptr;
   ~DevBuf() {
@@ -1165,5 +1472,152 @@ extern "C" inch_status inch_anm_records(int64_t n, const double *xyz, int64_t nc
   k_rec_lists<<<(unsigned)ncl, 256, 0, st>>>(ncl, cl_ptr, base, entries, (const int32_t *)slot_of.p, rec_entries);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));   // slot_of is freed on return
+  return INCH_OK;
+}
+
+extern "C" inch_status inch_anm_tile_order(int64_t n, const double *xyz, double side, int32_t tile, int32_t *order,
+                                           int32_t *tile_start, int64_t *ntile_out, void *stream) {
+  INCH_REQUIRE(n > 0 && n < (int64_t)1 << 31 && xyz && order && tile_start && ntile_out && side > 0 && tile > 0,
+               "inch_anm_tile_order: bad args");
+  hipStream_t st = (hipStream_t)stream;
+  const int bs = 256;
+  const int nb = 256;
+  DevBuf part;
+  HIP_TRY(hipMalloc(&part.p, nb * 6 * sizeof(double)));
+  k_minmax<<<nb, 256, 0, st>>>(n, xyz, (double *)part.p);
+  HIP_TRY(hipGetLastError());
+  std::vector<double> hp(nb * 6);
+  HIP_TRY(hipMemcpyAsync(hp.data(), part.p, nb * 6 * sizeof(double), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  CGrid g;
+  double hi[3];
+  for (int a = 0; a < 3; ++a) {
+    g.lo[a] = INFINITY;
+    hi[a] = -INFINITY;
+    bool nan = false;   // std::min/max would drop a NaN partial
+    for (int b = 0; b < nb; ++b) {
+      nan |= std::isnan(hp[b * 6 + a]) || std::isnan(hp[b * 6 + 3 + a]);
+      g.lo[a] = std::min(g.lo[a], hp[b * 6 + a]);
+      hi[a] = std::max(hi[a], hp[b * 6 + 3 + a]);
+    }
+    if (nan || !std::isfinite(g.lo[a]) || !std::isfinite(hi[a])) INCH_FAIL(INCH_ERR_NAN, "inch_anm_tile_order: non-finite coordinates");
+  }
+  // columns (coarser ones where their numbers would not fit 31 bits)
+  for (double s = side;; s *= 2.0) {
+    double cells = 1.0;
+    for (int a = 0; a < 2; ++a) {
+      g.inv[a] = 1.0 / s;
+      const double d = std::floor((hi[a] - g.lo[a]) * g.inv[a]) + 1.0;
+      cells *= d;
+      g.dim[a] = d < 2147483647.0 ? std::max<int64_t>(1, (int64_t)d) : (int64_t)1 << 31;
+    }
+    if (cells < 2147483647.0) break;
+  }
+  const double zspan = hi[2] - g.lo[2], zscale = zspan > 0.0 ? 4294967295.0 / zspan : 0.0;
+  DevBuf key, key2, at, head, cidx, first, tiles, base, tmp;
+  HIP_TRY(hipMalloc(&key.p, n * sizeof(uint64_t)));
+  HIP_TRY(hipMalloc(&key2.p, n * sizeof(uint64_t)));
+  HIP_TRY(hipMalloc(&at.p, n * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&head.p, n * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&cidx.p, (n + 1) * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&first.p, (n + 1) * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&base.p, (n + 1) * sizeof(int32_t)));
+  const unsigned gb = (unsigned)((n + bs - 1) / bs);
+  k_tile_keys<<<gb, bs, 0, st>>>(n, xyz, g, zscale, (uint64_t *)key.p, (int32_t *)at.p);
+  HIP_TRY(hipGetLastError());
+  int top = 33;
+  while (top < 64 && ((uint64_t)(g.dim[0] * g.dim[1]) >> (top - 32))) ++top;
+  size_t tmp_bytes = 0;
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, (const uint64_t *)key.p, (uint64_t *)key2.p,
+                                             (const int32_t *)at.p, order, (int)n, 0, top, st));
+  HIP_TRY(hipMalloc(&tmp.p, tmp_bytes));
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, (const uint64_t *)key.p, (uint64_t *)key2.p,
+                                             (const int32_t *)at.p, order, (int)n, 0, top, st));
+  k_tile_heads<<<gb, bs, 0, st>>>(n, (const uint64_t *)key2.p, (int32_t *)head.p);
+  HIP_TRY(hipGetLastError());
+  SCAN_TRY(n, (const int32_t *)head.p, (int32_t *)cidx.p);
+  k_tile_first<<<gb, bs, 0, st>>>(n, (const int32_t *)head.p, (const int32_t *)cidx.p, (int32_t *)first.p);
+  k_tile_column<<<gb, bs, 0, st>>>(n, tile, (const int32_t *)cidx.p, (const int32_t *)first.p, (int32_t *)head.p);
+  HIP_TRY(hipGetLastError());
+  SCAN_TRY(n, (const int32_t *)head.p, (int32_t *)base.p);
+  k_tile_cut<<<gb, bs, 0, st>>>(n, (const int32_t *)cidx.p, (const int32_t *)first.p, (const int32_t *)base.p, tile_start);
+  HIP_TRY(hipGetLastError());
+  int32_t nt = 0;
+  HIP_TRY(hipMemcpyAsync(&nt, (const int32_t *)base.p + n, sizeof(nt), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  *ntile_out = nt;
+  return INCH_OK;
+}
+
+extern "C" inch_status inch_anm_tiles(int64_t n, const double *xyz, const int64_t *rowptr, const int32_t *col,
+                                      const uint16_t *images, double box_x, double box_y, int64_t ntile,
+                                      int32_t tile, int32_t lanes, const int32_t *order, const int32_t *tile_start,
+                                      int32_t *tile_atoms, int32_t *slot_of, int32_t *waves, int64_t *blocks_out,
+                                      int32_t ucap, int32_t *ulen, uint32_t *ulist, uint16_t *pairs,
+                                      int64_t pair_blocks, double *rec, int32_t *umax_out, void *stream) {
+  INCH_REQUIRE(n > 0 && xyz && rowptr && col && tile_atoms && slot_of && waves && ntile > 0, "inch_anm_tiles: bad args");
+  INCH_REQUIRE(inch_tile_shape_ok(tile, lanes), "inch_anm_tiles: no tile shape of %d atoms x %d lanes", tile, lanes);
+  const int64_t slots = ntile * tile, nw = slots * lanes / 64;
+  if (48 * slots > (int64_t)UINT32_MAX)
+    INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tiles: %lld atoms exceed the 32-bit record offsets", (long long)n);
+  hipStream_t st = (hipStream_t)stream;
+  const int bs = 256;
+  DevBuf flags;
+  HIP_TRY(hipMalloc(&flags.p, 2 * sizeof(int32_t)));
+  HIP_TRY(hipMemsetAsync(flags.p, 0, 2 * sizeof(int32_t), st));
+  int32_t *umax = (int32_t *)flags.p + 1;
+  int32_t fl[2] = {0, 0};
+  auto check = [&]() -> inch_status {
+    HIP_TRY(hipMemcpyAsync(fl, flags.p, sizeof(fl), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    if (fl[0] & 8) INCH_FAIL(INCH_ERR_INVALID, "inch_anm_tiles: a column lies outside [0, n)");
+    if (fl[0] & 16) INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tiles: squared distances outside 1e-30 .. 1e30");
+    if (fl[0] & 1) INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tiles: a tile's neighbours exceed %d", ucap);
+    return INCH_OK;
+  };
+  if (pairs) {   // second call
+    INCH_REQUIRE(ulen && ulist && rec && umax_out && ucap > 0 && ucap <= inch_tile_max_union(tile),
+                 "inch_anm_tiles: bad args of the fill call");
+    INCH_REQUIRE(blocks_out && *blocks_out <= pair_blocks, "inch_anm_tiles: pairs too small");
+    k_tile_coords<<<(unsigned)((slots + bs - 1) / bs), bs, 0, st>>>(slots, tile_atoms, xyz, rec);
+    HIP_TRY(hipGetLastError());
+    if (images)
+      k_tile_fill<true><<<(unsigned)ntile, 256, 0, st>>>(n, tile, lanes, xyz, rowptr, col, images, box_x, box_y,
+                                                         tile_atoms, slot_of, (const int2 *)waves, ucap, ulen, ulist,
+                                                         pairs, (int32_t *)flags.p, umax);
+    else
+      k_tile_fill<false><<<(unsigned)ntile, 256, 0, st>>>(n, tile, lanes, xyz, rowptr, col, images, 0.0, 0.0,
+                                                          tile_atoms, slot_of, (const int2 *)waves, ucap, ulen, ulist,
+                                                          pairs, (int32_t *)flags.p, umax);
+    HIP_TRY(hipGetLastError());
+    const inch_status s = check();
+    if (s != INCH_OK) return s;
+    *umax_out = fl[1];
+    return INCH_OK;
+  }
+  INCH_REQUIRE(blocks_out && order && tile_start, "inch_anm_tiles: bad args of the first call");
+  DevBuf cnt, passes, blocks, ptr;
+  HIP_TRY(hipMalloc(&cnt.p, n * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&passes.p, nw * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&blocks.p, nw * sizeof(int32_t)));
+  HIP_TRY(hipMalloc(&ptr.p, (nw + 1) * sizeof(int32_t)));
+  const unsigned cg = (unsigned)((16 * n + bs - 1) / bs);
+  if (images)
+    k_tile_count<true><<<cg, bs, 0, st>>>(n, xyz, rowptr, col, images, box_x, box_y, (int32_t *)cnt.p, (int32_t *)flags.p);
+  else
+    k_tile_count<false><<<cg, bs, 0, st>>>(n, xyz, rowptr, col, images, 0.0, 0.0, (int32_t *)cnt.p, (int32_t *)flags.p);
+  HIP_TRY(hipGetLastError());
+  k_tile_slots<<<(unsigned)ntile, 64, 0, st>>>(tile, lanes, order, tile_start, (const int32_t *)cnt.p, tile_atoms, slot_of,
+                                               (int32_t *)passes.p, (int32_t *)blocks.p);
+  HIP_TRY(hipGetLastError());
+  SCAN_TRY(nw, (const int32_t *)blocks.p, (int32_t *)ptr.p);
+  k_tile_waves<<<(unsigned)((nw + bs - 1) / bs), bs, 0, st>>>(nw, (const int32_t *)ptr.p, (const int32_t *)passes.p,
+                                                              (int2 *)waves);
+  HIP_TRY(hipGetLastError());
+  int32_t total = 0;
+  HIP_TRY(hipMemcpyAsync(&total, (const int32_t *)ptr.p + nw, sizeof(total), hipMemcpyDeviceToHost, st));
+  const inch_status s = check();   // syncs
+  if (s != INCH_OK) return s;
+  *blocks_out = total;
   return INCH_OK;
 }

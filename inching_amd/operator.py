@@ -14,14 +14,15 @@ filtered matvec of degree m is m launches of the fused SpMV + three-term-recurre
 ``timer``: optional list; when set, every operator launch is bracketed by HIP events on
 the current stream and the event pairs are appended (kernel-time accounting).
 
-With the matrix-free float64 operator on the cluster layout, a filtered application runs
-its recurrence on records (``ops.anm_records``): the input is packed once into cluster order
-next to the coordinates, the degree products read and write records, and the accumulated
-result is unpacked once (``records=False`` or ``INCHING_RECORDS=0`` keeps the vectors in the
-matrix's order).
+With the matrix-free float64 operator, a filtered application runs its recurrence in slot
+order (``BlockHessian.slot_form``: tiles, or records of the cluster layout): the input is
+packed once next to the coordinates, the degree products read and write records, and the
+accumulated result is unpacked once (``records=False`` or ``INCHING_RECORDS=0`` keeps the
+vectors in the matrix's order).
 """
 import os
 
+import numpy as np
 import torch
 
 from . import ops
@@ -47,12 +48,13 @@ class Operator:
         self.Q = Q
         self.shift = float(shift)
         use_rec = RECORDS if records is None else bool(records)
-        rec_ok = (pol is not None and precision == "mf64" and use_rec and getattr(A, "images", None) is None
-                  and (lanes is None or int(lanes) // 1000 & 4) and A.records() is not None)
+        # a launch code for the matrix's order (other than the cluster layout's) asks for that order
+        rec_ok = (pol is not None and precision == "mf64" and use_rec
+                  and (lanes is None or int(lanes) // 1000 & 4) and A.slot_form() is not None)
         if lanes is not None:
             self.lanes = int(lanes)
         elif rec_ok:
-            self.lanes = 6001 if A.clusters() is not None else 161   # plain products only; no tuning needed
+            self.lanes = None     # plain products only: picked when the first one comes
         elif tune:
             from .autotune import best_config
             self.lanes = best_config(A, precision)
@@ -76,8 +78,10 @@ class Operator:
             self.degree = int(pol.AdjustedDegree)
         self.rec = None
         if rec_ok:
-            self.rec = A.records()
-            self._acc_rec = torch.empty(3 * A.clusters()[0].numel(), dtype=torch.float64, device=dev)
+            self.rec = A.slot_form()
+            self._recs = self.rec.buffers(3)
+            self._acc_rec = torch.empty(3 * self.rec.slots, dtype=torch.float64, device=dev)
+            self._mu = np.array(self.mu, dtype=np.float64)
         if Q is not None:
             if Q.dtype != torch.float64 or Q.shape[1] != self.n:
                 raise ValueError("Q must be float64 [m, 3N]")
@@ -92,6 +96,8 @@ class Operator:
             e1 = torch.cuda.Event(enable_timing=True)
             e0.record()
         if self.vals is None:
+            if self.lanes is None:
+                self.lanes = 161 if self.A.images is not None or self.A.clusters() is None else 6001
             self.A.matfree_spmv(x, y, config=self.lanes, **epi)
         else:
             ops.bsr_spmv(self.A.n_atoms, self.A.rowptr, self.A.col, self.vals, x, y, lanes=self.blanes,
@@ -104,35 +110,19 @@ class Operator:
 
     def _filtered_records(self, v64, u64):
         """u = sum_k mu_k T_k((A - cc)/dd) v with the recurrence on records: v packed into
-        cluster order, three record buffers in turn (T_k, T_{k-1} read, T_{k+1} written),
+        slot order, three record buffers in turn (T_k, T_{k-1} read, T_{k+1} written),
         the accumulator in slot order unpacked into u at the end."""
-        pol = self.pol
-        dd, cc = float(pol.dd), float(pol.cc)
-        recs, rent = self.rec
-        atoms, ptr = self.A.clusters()[:2]
-        acc = self._acc_rec
-        plus_i = self.A.plus_i
-        cur, prev = recs[0], None
-        free = [recs[1], recs[2]]
-        ops.rec_pack(atoms, v64, cur, acc, self.mu[0])
+        pol, form, acc = self.pol, self.rec, self._acc_rec
+        ops.rec_pack(form.atoms, v64, self._recs[0], acc, self.mu[0])
         if self.timer is not None:
             e0 = torch.cuda.Event(enable_timing=True)
             e1 = torch.cuda.Event(enable_timing=True)
             e0.record()
-        for k in range(1, self.degree + 1):
-            out = free.pop(0)
-            if k == 1:
-                ops.matfree_rec(cur, None, out, ptr, rent, plus_i, s1=1.0 / dd, c0=cc, acc=acc, mu=self.mu[1])
-            else:
-                ops.matfree_rec(cur, prev, out, ptr, rent, plus_i, s1=2.0 / dd, c0=cc, c2=1.0, acc=acc,
-                                mu=self.mu[k])
-            if prev is not None:
-                free.append(prev)
-            prev, cur = cur, out
+        form.chebyshev(self._recs, self._mu, float(pol.cc), float(pol.dd), self.A.plus_i, acc)
         if self.timer is not None:
             e1.record()
             self.timer.append(("mf64rec", "cheb", e0, e1, self.degree))
-        ops.rec_unpack(atoms, acc, u64)
+        ops.rec_unpack(form.atoms, acc, u64)
         self.n_spmv += self.degree
 
     def filtered(self, v64, u64):

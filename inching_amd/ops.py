@@ -296,6 +296,73 @@ def matfree_rec(rec_in, rec_z, rec_out, cl_ptr, rec_entries, plus_i, s1=1.0, c0=
          float(plus_i), float(s1), float(c0), float(c2), P(acc), float(mu), 1 if xcd else 0, stream_ptr(stream))
 
 
+class Tiles:
+    """Tile form of the matrix-free operator (inch_anm_tiles): the slots' atoms, every tile's
+    union of neighbours and its atoms' lists into it. Holds the arrays and the launch's fixed
+    arguments; the record buffers of a recurrence are the caller's (``buffers``)."""
+
+    def __init__(self, xyz, rowptr, col, side, shape, images=None, box=None, stream=None):
+        require_gpu()
+        _check_dev(xyz, rowptr, col)
+        n, dev = xyz.shape[0], xyz.device
+        if rowptr.numel() != n + 1 or (images is not None and images.numel() != col.numel()):
+            raise ValueError("rowptr / images inconsistent with the coordinates")
+        tile, lanes = shape
+        i32 = dict(dtype=torch.int32, device=dev)
+        order, start = torch.empty(n, **i32), torch.empty(n + 1, **i32)
+        nt = C.c_int64(0)
+        call("inch_anm_tile_order", n, P(xyz), float(side), tile, P(order), P(start), C.byref(nt), stream_ptr(stream))
+        nt = nt.value
+        self.shape, self.ntile, self.slots = (tile, lanes), nt, nt * tile
+        ucap = 65536 // 48 - tile
+        self.atoms = torch.empty(self.slots, **i32)
+        slot_of = torch.empty(n, **i32)
+        self.waves = torch.empty(2 * self.slots * lanes // 64, **i32)
+        bx, by = (0.0, 0.0) if box is None else (float(box[0]), float(box[1]))
+        blocks, umax = C.c_int64(0), C.c_int32(0)
+        head = (n, P(xyz), P(rowptr), P(col), P(images), bx, by, nt, tile, lanes, P(order), P(start), P(self.atoms),
+                P(slot_of), P(self.waves), C.byref(blocks))
+        call("inch_anm_tiles", *head, ucap, None, None, None, 0, None, None, stream_ptr(stream))
+        self.pairs = torch.empty(1024 * max(1, blocks.value), dtype=torch.uint8, device=dev)
+        self.ulen = torch.empty(nt, **i32)
+        self.ulist = torch.empty(nt * ucap, **i32)
+        self.rec = torch.empty(6 * self.slots, dtype=torch.float64, device=dev)
+        call("inch_anm_tiles", *head, ucap, P(self.ulen), P(self.ulist), P(self.pairs), max(1, blocks.value),
+             P(self.rec), C.byref(umax), stream_ptr(stream))
+        self._lists = (P(self.ulen), P(self.ulist), ucap, umax.value, P(self.waves), P(self.pairs), bx, by)
+
+    def buffers(self, count):
+        """``count`` record buffers [6 slots] with the slots' coordinates, the caller's own."""
+        return [self.rec.clone() for _ in range(count)]
+
+    def _records(self, *recs):
+        for r in recs:
+            if r is not None and (r.numel() != 6 * self.slots or r.dtype != torch.float64):
+                raise ValueError("records must be float64 [6 slots]")
+
+    def _vectors(self, *vs):
+        for v in vs:
+            if v is not None and (v.numel() != 3 * self.slots or v.dtype != torch.float64):
+                raise ValueError("acc and y must be float64 [3 slots]")
+
+    def product(self, rec_in, rec_z, rec_out, plus_i, s1=1.0, c0=0.0, c2=0.0, acc=None, mu=0.0, y=None, stream=None):
+        """One Chebyshev step on records (inch_anm_matfree_tile)."""
+        self._records(rec_in, rec_z, rec_out)
+        self._vectors(acc, y)
+        call("inch_anm_matfree_tile", self.ntile, *self.shape, P(rec_in), P(rec_z), P(rec_out), P(y), *self._lists,
+             float(plus_i), float(s1), float(c0), float(c2), P(acc), float(mu), stream_ptr(stream))
+
+    def chebyshev(self, recs, mu, cc, dd, plus_i, acc, stream=None):
+        """acc += sum_k mu[k] T_k((A - cc) / dd) x over k >= 1, x packed in recs[0]
+        (inch_anm_chebyshev_tile); mu: contiguous float64 numpy array."""
+        self._records(*recs)
+        self._vectors(acc)
+        if mu.dtype != np.float64 or not mu.flags.c_contiguous:
+            raise ValueError("mu must be a contiguous float64 array")
+        call("inch_anm_chebyshev_tile", self.ntile, *self.shape, P(recs[0]), P(recs[1]), P(recs[2]), mu.size - 1,
+             mu.ctypes.data, float(cc), float(dd), *self._lists, float(plus_i), P(acc), stream_ptr(stream))
+
+
 def rec_pack(cluster_atoms, v, rec, acc=None, mu0=0.0, stream=None, ncl=None):
     """Vector part of the records from v (matrix order through cluster_atoms, or slot order
     when cluster_atoms is None, then ``ncl`` is required)."""

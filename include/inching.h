@@ -269,6 +269,53 @@ inch_status inch_anm_records(int64_t n, const double *xyz, int64_t ncl, const in
 inch_status inch_anm_matfree_rec(int64_t ncl, const double *rec_in, const double *rec_z, double *rec_out, double *y,
                                  const int64_t *cl_ptr, const uint32_t *rec_entries, double plus_i, double s1,
                                  double c0, double c2, double *acc, double mu, int32_t xcd, void *stream);
+/* Tile form of the matrix-free operator for the same recurrence (no reference counterpart as a
+ * layout; the product is that of Burn/Krylov/T3.py:54-239). inch_anm_tile_order sorts the atoms
+ * along columns of side x side in x and y (order int32 [n]) and cuts every column into equal
+ * tiles of at most `tile` atoms: tile t holds order[tile_start[t]] .. order[tile_start[t + 1] - 1]
+ * (tile_start int32 [n + 1], of which *ntile_out + 1 are written; syncs).
+ * inch_anm_tiles: slot q = tile t + p is place p of tile t (tile_atoms int32 [tile ntile], -1 on
+ * padding slots; slot_of int32 [n] its inverse). Every tile
+ * lists the union of its atoms' neighbours (ulen int32 [ntile] words of ulist uint32
+ * [ntile ucap]: 48 (slot of the neighbour) | image, ascending; image = bit number
+ * (sx + 1) * 3 + (sy + 1) of the periodic image, 4 for open boundaries); every wave of
+ * 64 / lanes atoms has waves int32 [2 tile ntile lanes / 64] = (first block, passes) and blocks
+ * of 64 lanes x 8 passes of uint16 byte offsets into the union's 48-byte records, pairs uint16
+ * [512 pair_blocks]: term q of an atom at pass q / lanes, its lane q % lanes; passes beyond an
+ * atom's terms hold 48 (ulen + the atom's place in its tile). Pairs at zero distance have no
+ * term. (tile, lanes) is one of (64, 8), (32, 16), (16, 32); ucap at most
+ * 65536 / 48 - tile. images NULL: open boundaries; else the masks of
+ * inch_neighbors_celllist_pbc with its box.
+ * Two calls: with pairs NULL it writes tile_atoms, slot_of, waves and *blocks_out; with pairs
+ * (pair_blocks >= *blocks_out) and the arrays of the first call it writes ulen, ulist, pairs,
+ * rec float64 [6 tile ntile] (records as inch_anm_records: coordinates, zero vector part) and
+ * *umax_out, the longest union (order and tile_start are then unused). INCH_ERR_CAPACITY when a
+ * union exceeds ucap, a squared distance lies outside 1e-30 .. 1e30 or the slots exceed the
+ * 32-bit record offsets; syncs. */
+inch_status inch_anm_tile_order(int64_t n, const double *xyz, double side, int32_t tile, int32_t *order,
+                                int32_t *tile_start, int64_t *ntile_out, void *stream);
+inch_status inch_anm_tiles(int64_t n, const double *xyz, const int64_t *rowptr, const int32_t *col,
+                           const uint16_t *images, double box_x, double box_y, int64_t ntile, int32_t tile,
+                           int32_t lanes, const int32_t *order, const int32_t *tile_start, int32_t *tile_atoms,
+                           int32_t *slot_of, int32_t *waves, int64_t *blocks_out, int32_t ucap, int32_t *ulen,
+                           uint32_t *ulist, uint16_t *pairs, int64_t pair_blocks, double *rec, int32_t *umax_out,
+                           void *stream);
+/* One step of the recurrence on the tile form: as inch_anm_matfree_rec, with records, y and acc
+ * of tile ntile slots. box_x > 0: periodic images (the box of the layout). */
+inch_status inch_anm_matfree_tile(int64_t ntile, int32_t tile, int32_t lanes, const double *rec_in,
+                                  const double *rec_z, double *rec_out, double *y, const int32_t *ulen,
+                                  const uint32_t *ulist, int32_t ucap, int32_t umax, const int32_t *waves,
+                                  const uint16_t *pairs, double box_x, double box_y, double plus_i, double s1,
+                                  double c0, double c2, double *acc, double mu, void *stream);
+/* The recurrence of one filtered application (ChebAv, Burn/PolynomialFilters/T2.py:28-92) on the
+ * tile form: T_0 in rec0, T_1 = (A - cc) T_0 / dd, T_k+1 = 2 (A - cc) T_k / dd - T_k-1, and
+ * acc += mu[k] T_k for k = 1 .. degree (mu: host, degree + 1 entries). rec0, rec1, rec2 are
+ * three record buffers with the layout's coordinates; their vector parts are overwritten. */
+inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, double *rec0, double *rec1,
+                                    double *rec2, int32_t degree, const double *mu, double cc, double dd,
+                                    const int32_t *ulen, const uint32_t *ulist, int32_t ucap, int32_t umax,
+                                    const int32_t *waves, const uint16_t *pairs, double box_x, double box_y,
+                                    double plus_i, double *acc, void *stream);
 /* Vector part of rec for slot q = v[3 a .. 3 a + 2] with a = cluster_atoms[q] (0 for padding),
  * or v[3 q .. 3 q + 2] when cluster_atoms is NULL (v in slot order, [12 ncl]); acc (may be
  * NULL) [12 ncl] = mu0 times the same. */
