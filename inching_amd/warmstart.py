@@ -34,7 +34,6 @@ from ._lib import call
 HIDDEN = 64
 LAYERS = 4
 NFEAT = 16
-F16, F32 = 2, 0
 WEIGHTS = os.path.join(os.path.dirname(os.path.abspath(__file__)), "weights", "warmstart_gnn.npz")
 
 P_ = ops.P
@@ -93,50 +92,42 @@ def _dense_bwd(X, W, dY, dX, dW, db):
     call("inch_gnn_dense_bwd", N, Din, Dout, P_(X), P_(W), P_(dY), P_(dX), P_(dW), P_(db), P_(work), SP())
 
 
-def _aggregate(g, X, xdt, Y, ydt, mode):
-    call("inch_gnn_aggregate", g.N, X.shape[1], P_(g.rowptr), P_(g.col), P_(X), xdt, P_(Y), ydt, mode, SP())
-
-
 class GraphLayer(torch.autograd.Function):
     """h_out = relu(h W_s + agg(h) W_n + b). Activations enter the kernels as float16,
     weights as float16, accumulation and gradients are float32."""
 
     @staticmethod
     def forward(ctx, h, Ws, Wn, b, g):
-        N = h.shape[0]
+        N, Din = h.shape
         Dout = Ws.shape[1]
+        dev = h.device
         h16 = h.to(torch.float16).contiguous()
-        Ws16, Wn16 = Ws.to(torch.float16).contiguous(), Wn.to(torch.float16).contiguous()
-        agg = torch.empty_like(h16)
-        _aggregate(g, h16, F16, agg, F16, 0)
-        a = torch.empty((N, Dout), dtype=torch.float32, device=h.device)
-        c = torch.empty_like(a)
-        _dense_fwd(h16, Ws16, b.contiguous(), a)
-        _dense_fwd(agg, Wn16, None, c)
-        pre = a + c
+        Ws32, Wn32 = Ws.to(torch.float32).contiguous(), Wn.to(torch.float32).contiguous()
+        half = dict(dtype=torch.float16, device=dev)
+        agg, Ws16, Wn16 = torch.empty_like(h16), torch.empty((Din, Dout), **half), torch.empty((Din, Dout), **half)
+        pre = torch.empty((N, Dout), dtype=torch.float32, device=dev)
+        out = torch.empty_like(pre)
+        call("inch_gnn_layer_fwd", N, Din, Dout, P_(g.rowptr), P_(g.col), P_(h16), P_(Ws32), P_(Wn32),
+             P_(b.contiguous()), P_(agg), P_(Ws16), P_(Wn16), P_(pre), P_(out), SP())
         ctx.save_for_backward(h16, agg, Ws16, Wn16, pre)
         ctx.g = g
-        return torch.relu(pre)
+        return out
 
     @staticmethod
     def backward(ctx, dout):
         h16, agg, Ws16, Wn16, pre = ctx.saved_tensors
         g = ctx.g
-        dout = dout.to(torch.float32).contiguous()
-        dpre = torch.empty_like(pre)
-        call("inch_gnn_relu_bwd", pre.numel(), P_(pre), P_(dout), P_(dpre), SP())
+        N = h16.shape[0]
         Din, Dout = Ws16.shape
-        dh = torch.empty((h16.shape[0], Din), dtype=torch.float32, device=h16.device)
-        dagg = torch.empty_like(dh)
-        dWs = torch.empty((Din, Dout), dtype=torch.float32, device=h16.device)
-        dWn = torch.empty_like(dWs)
-        db = torch.empty(Dout, dtype=torch.float32, device=h16.device)
-        db2 = torch.empty_like(db)
-        _dense_bwd(h16, Ws16, dpre, dh, dWs, db)
-        _dense_bwd(agg, Wn16, dpre, dagg, dWn, db2)
-        dh2 = torch.empty_like(dh)
-        _aggregate(g, dagg, F32, dh2, F32, 1)
-        return dh + dh2, dWs, dWn, db, None
+        f32 = dict(dtype=torch.float32, device=h16.device)
+        dout = dout.to(torch.float32).contiguous()
+        # the first layer's input has no gradient: its neighbour sum is left out
+        dh = torch.empty((N, Din), **f32) if ctx.needs_input_grad[0] else None
+        dWs, dWn, db = torch.empty((Din, Dout), **f32), torch.empty((Din, Dout), **f32), torch.empty(Dout, **f32)
+        work = torch.empty(int(call("inch_gnn_layer_work_size", N, Din, Dout)), **f32)
+        call("inch_gnn_layer_bwd", N, Din, Dout, P_(g.rowptr), P_(g.col), P_(h16), P_(agg), P_(Ws16), P_(Wn16),
+             P_(pre), P_(dout), P_(dh), P_(dWs), P_(dWn), P_(db), P_(work), SP())
+        return dh, dWs, dWn, db, None
 
 
 class Head(torch.autograd.Function):

@@ -409,6 +409,19 @@ inch_status inch_gnn_dense_bwd(int64_t N, int32_t Din, int32_t Dout, const void 
  * mode 1 its adjoint. dtype codes: 0 float32, 2 float16. */
 inch_status inch_gnn_aggregate(int64_t N, int32_t D, const int64_t *rowptr, const int32_t *col, const void *X,
                                int32_t xdt, void *Y, int32_t ydt, int32_t mode, void *stream);
+/* A graph layer, out = relu(pre), pre = (b + h Ws) + agg Wn, agg = neighbour mean of h (mode 0
+ * above): h float16 [N, Din]; Ws, Wn float32 [Din, Dout], rounded to float16 (written to Ws16,
+ * Wn16); writes agg (float16 [N, Din]), pre and out (float32 [N, Dout]). The backward takes those
+ * and dout, and writes dWs, dWn, db and dh (may be NULL); work: inch_gnn_layer_work_size floats.
+ */
+inch_status inch_gnn_layer_fwd(int64_t N, int32_t Din, int32_t Dout, const int64_t *rowptr, const int32_t *col,
+                               const void *h, const float *Ws, const float *Wn, const float *b, void *agg, void *Ws16,
+                               void *Wn16, float *pre, float *out, void *stream);
+int64_t inch_gnn_layer_work_size(int64_t N, int32_t Din, int32_t Dout);
+inch_status inch_gnn_layer_bwd(int64_t N, int32_t Din, int32_t Dout, const int64_t *rowptr, const int32_t *col,
+                               const void *h, const void *agg, const void *Ws16, const void *Wn16, const float *pre,
+                               const float *dout, float *dh, float *dWs, float *dWn, float *db, float *work,
+                               void *stream);
 /* dPre = dY where pre > 0 else 0. */
 inch_status inch_gnn_relu_bwd(int64_t n, const float *pre, const float *dY, float *dPre, void *stream);
 
