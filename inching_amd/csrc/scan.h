@@ -1,6 +1,6 @@
 // Exclusive prefix sums on the device, shared by the construction and the ordering:
 // out[i] = sum in[0..i-1] for i <= m (out[m] = the total). One block of 1024 threads walks
-// short arrays in chunks; longer ones take three passes: per-tile sums (kScanTile elements
+// short arrays; longer ones take three passes: per-tile sums (kScanTile elements
 // per 256-thread block), the single-block scan of the tile sums, and a rescan of every tile
 // from its offset.
 #pragma once
@@ -10,29 +10,44 @@
 
 namespace {
 
+// One block: 8 elements per thread, wave scans and the waves' sums through LDS (two barriers
+// per 8,192 elements; a scan of 1,024 at a time over LDS took 22 barriers for each).
 template <typename T>
-__global__ void k_scan_one(int64_t m, const T *__restrict__ in, T *__restrict__ out) {
-  __shared__ T buf[1024];
-  __shared__ T carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int64_t base = 0; base < m; base += 1024) {
-    const int64_t i = base + threadIdx.x;
-    const T v = i < m ? in[i] : 0;
-    buf[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const T t = (int)threadIdx.x >= off ? buf[threadIdx.x - off] : 0;
-      __syncthreads();
-      buf[threadIdx.x] += t;
-      __syncthreads();
+__global__ void __launch_bounds__(1024) k_scan_one(int64_t m, const T *__restrict__ in, T *__restrict__ out) {
+  __shared__ T sums[16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  T carry = 0;
+  for (int64_t base = 0; base < m; base += 8192) {
+    T v[8], t = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int64_t i = base + 8 * tid + q;
+      v[q] = i < m ? in[i] : 0;
+      t += v[q];
     }
-    if (i < m) out[i] = carry + buf[threadIdx.x] - v;
+    T inc = t;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const T x = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += x;
+    }
     __syncthreads();
-    if (threadIdx.x == 1023) carry += buf[1023];
+    if (lane == 63) sums[w] = inc;
     __syncthreads();
+    T before = carry + inc - t;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      if (q < w) before += sums[q];
+      carry += sums[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int64_t i = base + 8 * tid + q;
+      if (i < m) out[i] = before;
+      before += v[q];
+    }
   }
-  if (threadIdx.x == 0) out[m] = carry;
+  if (tid == 0) out[m] = carry;
 }
 
 constexpr int kScanPer = 16;                 // elements per thread of a tile
