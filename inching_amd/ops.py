@@ -115,19 +115,23 @@ def batch_head(n, maxleaf):
 
 # ---------------------------------------------------------------- device ----
 
-def neighbours(xyz, rc, stream=None):
-    """Cell-list neighbour CSR of device float64 coordinates [n,3] -> (indptr, indices)."""
+def neighbours(xyz, rc, stream=None, ascending=True):
+    """Cell-list neighbour CSR of device float64 coordinates [n,3] -> (indptr, indices).
+    ``ascending=False`` leaves each row's columns in an unspecified order."""
     require_gpu()
     _check_dev(xyz)
     if xyz.dtype != torch.float64 or xyz.dim() != 2 or xyz.shape[1] != 3:
         raise ValueError("xyz must be float64 [n,3]")
-    n = xyz.shape[0]
-    indptr = torch.empty(n + 1, dtype=torch.int64, device=xyz.device)
-    nnz = C.c_int64(0)
-    call("inch_neighbors_celllist", n, P(xyz), float(rc), P(indptr), None, 0, C.byref(nnz), stream_ptr(stream))
-    indices = torch.empty(max(1, nnz.value), dtype=torch.int32, device=xyz.device)
-    call("inch_neighbors_celllist", n, P(xyz), float(rc), P(indptr), P(indices), nnz.value, C.byref(nnz),
-         stream_ptr(stream))
+    n, dev, sp = xyz.shape[0], xyz.device, stream_ptr(stream)
+    rc = float(rc)
+    indptr = torch.empty(n + 1, dtype=torch.int64, device=dev)
+    plan, size, nnz = (C.c_double * 7)(), C.c_int64(0), C.c_int64(0)
+    scratch = torch.empty(256 * 6, dtype=torch.float64, device=dev)
+    call("inch_cells_plan", n, P(xyz), rc, plan, C.byref(size), P(scratch), sp)
+    work = torch.empty(size.value, dtype=torch.uint8, device=dev)
+    call("inch_cells_count", n, P(xyz), rc, plan, P(work), size.value, P(indptr), C.byref(nnz), sp)
+    indices = torch.empty(max(1, nnz.value), dtype=torch.int32, device=dev)
+    call("inch_cells_fill", n, rc, plan, P(work), size.value, P(indptr), P(indices), 1 if ascending else 0, sp)
     return indptr, indices[:nnz.value]
 
 

@@ -109,6 +109,18 @@ inch_status inch_batch_head(int64_t n, int64_t maxleaf, int64_t *head, int64_t c
 inch_status inch_neighbors_celllist(int64_t n, const double *xyz, double rc, int64_t *indptr,
                                     int32_t *indices, int64_t capacity, int64_t *nnz_out,
                                     void *stream);
+/* The same search in steps that share one grid and a caller's scratch (no reference counterpart
+ * as calls): inch_cells_plan finds the cells (plan: host double[7]; scratch: device float64[1536];
+ * *work_bytes: the scratch of the other two) and syncs; inch_cells_count writes indptr and
+ * *nnz_out and syncs (INCH_ERR_CAPACITY for rows over 2048 entries); inch_cells_fill writes the
+ * rows (indices int32 [nnz]) from the lists that inch_cells_count left in work, ascending when
+ * sorted != 0, else in an unspecified order, without a sync. */
+inch_status inch_cells_plan(int64_t n, const double *xyz, double rc, double *plan, int64_t *work_bytes,
+                            double *scratch, void *stream);
+inch_status inch_cells_count(int64_t n, const double *xyz, double rc, const double *plan, void *work,
+                             int64_t work_bytes, int64_t *indptr, int64_t *nnz_out, void *stream);
+inch_status inch_cells_fill(int64_t n, double rc, const double *plan, void *work, int64_t work_bytes,
+                            const int64_t *indptr, int32_t *indices, int32_t sorted, void *stream);
 /* The neighbour CSR renumbered by a permutation (no reference counterpart as one call: the
  * reference searches the reordered coordinates again, Fuel/Coordinate/T1.py:331-481 after
  * :171-323). order[i] = old index of new atom i (int32), undo[old] = new index (int64);

@@ -1,0 +1,78 @@
+"""Neighbour search where its workgroups can go wrong: runs of 32 atoms at their edges and across
+columns of cells, more candidates than one LDS stage, the unordered rows, and row sorting at the
+edges of its 64- and 256-entry forms and with equal entries."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import small_globule
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(ip, ix):
+    ip, ix = ip.cpu().numpy(), ix.cpu().numpy()
+    return [ix[ip[i]:ip[i + 1]] for i in range(len(ip) - 1)]
+
+
+def _brute(X, rc):
+    d = X[None, :, :] - X[:, None, :]
+    return ((d[..., 0] * d[..., 0] + d[..., 1] * d[..., 1]) + d[..., 2] * d[..., 2]) <= rc * rc
+
+
+CASES = {
+    "one": lambda r: r.uniform(0, 5, (1, 3)),
+    "run_edge_31": lambda r: r.uniform(0, 20, (31, 3)),
+    "run_edge_33": lambda r: r.uniform(0, 20, (33, 3)),
+    "many_columns": lambda r: r.uniform(0, 1, (700, 3)) * [300, 300, 4],
+    "one_column": lambda r: r.uniform(0, 1, (700, 3)) * [4, 4, 900],
+    "one_cell_two_stages": lambda r: r.uniform(0, 7, (1500, 3)),
+    "coincident": lambda r: np.repeat(r.uniform(0, 12, (60, 3)), 3, axis=0),
+    "globule": lambda r: small_globule(1500, seed=11) - 40.0,
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_neighbours_equal_brute_force(cuda, case):
+    from inching_amd import ops
+    print("case: neighbours %s" % case, flush=True)
+    X = CASES[case](np.random.default_rng(8))
+    want = _brute(X, 8.0)
+    xyz = torch.as_tensor(X, device="cuda")
+    ip, ix = ops.neighbours(xyz, 8.0)
+    for i, row in enumerate(_rows(ip, ix)):
+        assert np.array_equal(row, np.nonzero(want[i])[0]), i
+    ip2, ix2 = ops.neighbours(xyz, 8.0, ascending=False)
+    assert torch.equal(ip, ip2)
+    for a, b in zip(_rows(ip, ix), _rows(ip2, ix2)):
+        assert np.array_equal(a, np.sort(b))
+
+
+def test_neighbours_reject_rows_over_the_limit(cuda):
+    from inching_amd import ops
+    print("case: 2,049 neighbours", flush=True)
+    X = np.random.default_rng(8).uniform(0, 2, (2049, 3))
+    for ascending in (True, False):
+        with pytest.raises(ops.InchingError) as e:
+            ops.neighbours(torch.as_tensor(X, device="cuda"), 8.0, ascending=ascending)
+        assert e.value.status == -3
+
+
+@pytest.mark.parametrize("equal", [False, True])
+def test_row_sort_at_its_edges(cuda, equal):
+    """Rows of 0 to 2048 entries through the renumbering, also with repeated columns."""
+    from inching_amd import ops
+    print("case: row sort, equal entries %s" % equal, flush=True)
+    r = np.random.default_rng(3)
+    lens = [0, 1, 3, 4, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 700, 2048]
+    n = 4096
+    lens = lens + [1] * (n - len(lens))
+    rows = [r.choice(n, k, replace=False) if not equal else r.integers(0, max(1, k // 2), k) for k in lens]
+    ip = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    order = r.permutation(n).astype(np.int32)
+    undo = np.empty(n, np.int64)
+    undo[order] = np.arange(n)
+    dev = lambda a: torch.as_tensor(a, device="cuda")    # noqa: E731
+    op, oi = ops.csr_permute(dev(ip), dev(np.concatenate(rows).astype(np.int32)), dev(order), dev(undo))
+    for i, row in enumerate(_rows(op, oi)):
+        assert np.array_equal(row, np.sort(undo[rows[order[i]]])), i
