@@ -971,15 +971,36 @@ __global__ void k_tile_waves(int64_t nw, const int32_t *__restrict__ ptr, const 
   if (w < nw) waves[w] = make_int2(ptr[w], passes[w]);
 }
 
+// Place (pass, lane of the atom's G) of the rho-th term whose union place has residue r mod 16, for
+// the atom at place a of its tile. The product's 16-byte LDS reads serve a half wave in two groups
+// of 16 lanes, lanes {0-3, 12-15, 20-23, 24-27} and the others (measured: these are the only sets
+// of 16 that conflict among themselves), and a record's three reads meet banks by its place mod 16
+// (48 bytes are three groups of four of the 64 banks). So the 16 lanes of a group take 16
+// different residues in every pass: with G = 8 a group holds 4 lanes of 4 atoms, which take the
+// residues by quarters, another quarter each pass; with G = 16 8 lanes of 2 atoms, by halves;
+// with G = 32 the 16 lanes of one atom. Terms beyond a residue's places fill the gaps of others.
+__device__ __forceinline__ int2 tile_place(int G, int r, int rho, int a) {
+  const int half = rho & 1, c = rho >> 1;
+  if (G == 8) return make_int2(4 * c + (((r >> 2) - a) & 3), (r & 3) + 4 * half);
+  if (G == 16) {
+    const int q = r & 7;
+    return make_int2(2 * c + (((r >> 3) ^ a) & 1), half ? 4 + q : (q < 4 ? q : q + 8));
+  }
+  // lanes of the two groups in order: r-th lane of group `half`
+  const int g4 = r >> 2;
+  const int base = half ? (g4 == 0 ? 4 : g4 == 1 ? 8 : g4 == 2 ? 16 : 28) : (g4 == 0 ? 0 : g4 == 1 ? 12 : g4 == 2 ? 20 : 24);
+  return make_int2(c, base + (r & 3));
+}
+
 constexpr int kTileHash = 4096;   // slots of the union's hash table: at least 3 x the largest union
 
 // One block per tile. The (neighbour slot, image) words of its rows go into an LDS hash
 // table; the distinct ones, sorted, are the tile's union (written as 48 slot | image: the
 // byte offset of the neighbour's record, the image in its low 4 bits). Then a wave per row
-// writes its terms as 16-bit byte offsets 48 p of their places p in the union, term number q
-// of an atom at pass q / G, lane q % G of its G lanes, 8 passes to a block of 64 lanes x 16
-// bytes. Passes that a row does not fill name the atom's own dummy record 48 (union + atom),
-// whose term is zero. flags bit 0: the union exceeds ucap.
+// writes its terms as 16-bit byte offsets 48 p of their places p in the union, each to its pass
+// and lane (tile_place), 8 passes to a block of 64 lanes x 16 bytes. Places that a row does not
+// fill name the atom's own dummy record 48 (union + atom), whose term is zero. flags bit 0: the
+// union exceeds ucap.
 template <bool PBC>
 __global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, const double *__restrict__ xyz,
                                                    const int64_t *__restrict__ rowptr,
@@ -993,6 +1014,8 @@ __global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, con
   __shared__ uint32_t hkey[kTileHash];
   __shared__ uint16_t hpos[kTileHash];
   __shared__ uint32_t list[2048];
+  __shared__ uint32_t taken[4][64];      // a wave's places in use: at most ucap + G < 2,048
+  __shared__ uint16_t spills[4][1408];   // at most ucap
   __shared__ int s_n;
   const int64_t t = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -1071,16 +1094,20 @@ __global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, con
   }
   __syncthreads();
   const int AW = 64 / G, NW = TA / AW;
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
   for (int a = w; a < TA; a += 4) {
     const int32_t i = tile_atoms[t * TA + a];
     const int2 wv = waves[t * NW + a / AW];
+    const int passes = wv.y, slots = passes * G;
     uint16_t *out = pairs + 512 * (int64_t)wv.x;
-    const int l0 = (a % AW) * G, room = 8 * G * ((wv.y + 7) / 8);
-    auto put = [&](int q, uint32_t p) {   // term q of the atom
-      const int pass = q / G;
-      out[((pass >> 3) * 64 + l0 + q % G) * 8 + (pass & 7)] = (uint16_t)(48u * p);
+    const int l0 = (a % AW) * G;
+    auto put = [&](int pass, int l, uint32_t p) {
+      out[((pass >> 3) * 64 + l0 + l) * 8 + (pass & 7)] = (uint16_t)(48u * p);
     };
-    int done = 0;
+    taken[w][lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    int seen = 0, spilled = 0;   // lane r < 16: terms of residue r so far; terms without a place of their own
     if (i >= 0) {
       const int64_t e1 = rowptr[i + 1];
       for (int64_t e0 = rowptr[i]; e0 < e1; e0 += 64) {
@@ -1092,26 +1119,54 @@ __global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, con
           m = tile_images<PBC>(xyz, i, j, images, e, bx, by, far);
           s = (uint32_t)slot_of[j];
         }
-        int c = __popc(m), inc = c;
+        while (true) {   // one image per lane at a time
+          const uint64_t has = __ballot(m != 0);
+          if (!has) break;
+          uint32_t p = 0;
+          if (m) {
+            const uint32_t k = (s << 4) | (uint32_t)(__ffs(m) - 1);
+            uint32_t h = place(k);
+            while (hkey[h] != k) h = (h + 1) & (kTileHash - 1);
+            p = hpos[h];
+          }
+          const uint32_t r = p & 15u;
+          uint64_t same = has, mine = has;   // lanes of this lane's residue; of residue `lane`
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const int v = __shfl_up(inc, off, 64);
-          if (lane >= off) inc += v;
-        }
-        int q = done + inc - c;
-        while (m) {
-          const int bit = __ffs(m) - 1;
+          for (int q = 0; q < 4; ++q) {
+            const uint64_t bal = __ballot((r >> q) & 1u);
+            same &= (r >> q) & 1u ? bal : ~bal;
+            mine &= (lane >> q) & 1 ? bal : ~bal;
+          }
+          const int rho = __shfl(seen, (int)r, 64) + __popcll(same & below);
+          seen += __popcll(mine);
+          const int2 at = tile_place(G, (int)r, rho, a);
+          const bool spill = m && at.x >= passes;
+          if (m && !spill) {
+            put(at.x, at.y, p);
+            const int q = at.x * G + at.y;
+            atomicOr(&taken[w][q >> 5], 1u << (q & 31));
+          }
+          const uint64_t sp = __ballot(spill);
+          if (spill) spills[w][spilled + __popcll(sp & below)] = (uint16_t)p;
+          spilled += __popcll(sp);
           m &= m - 1;
-          const uint32_t k = (s << 4) | (uint32_t)bit;
-          uint32_t h = place(k);
-          while (hkey[h] != k) h = (h + 1) & (kTileHash - 1);
-          if (q < room) put(q, hpos[h]);   // always, by the count that sized the blocks
-          ++q;
         }
-        done += __shfl(inc, 63, 64);
       }
     }
-    for (int q = done + lane; q < room; q += 64) put(q, (uint32_t)(ul + a));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    int free_before = 0;
+    for (int q0 = 0; q0 < 8 * G * ((passes + 7) / 8); q0 += 64) {
+      const int q = q0 + lane;
+      const bool open = q < slots && !((taken[w][q >> 5] >> (q & 31)) & 1u);
+      const uint64_t bal = __ballot(open);
+      const int k = free_before + __popcll(bal & below);
+      free_before += __popcll(bal);
+      if (open || (q >= slots && q < 8 * G * ((passes + 7) / 8)))
+        put(q / G, q % G, open && k < spilled ? (uint32_t)spills[w][k] : (uint32_t)(ul + a));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
