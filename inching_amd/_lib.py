@@ -61,6 +61,9 @@ SIGNATURES = {
                                         _dbl, _dbl, _dbl, _dbl, _dbl, _vp, _dbl, _vp]),
     "inch_anm_chebyshev_tile": (_STATUS, [_i64, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _dbl, _dbl, _vp, _vp, _i32, _i32,
                                           _vp, _vp, _dbl, _dbl, _dbl, _vp, _vp]),
+    "inch_anm_tile_apply_work_size": (_i64, [_i64, _i32, _i32]),
+    "inch_anm_matfree_tile_apply": (_STATUS, [_i64, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp, _dbl, _dbl, _dbl,
+                                              _vp, _vp, _i32, _vp, _vp]),
     "inch_rec_pack": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _dbl, _vp]),
     "inch_rec_unpack": (_STATUS, [_i64, _vp, _vp, _vp, _vp]),
     "inch_anm_matfree_cl": (_STATUS, [_i64, _vp, _i64, _vp, _vp, _vp, _vp, _dbl, _i32, _vp, _vp, _dbl, _dbl, _vp,

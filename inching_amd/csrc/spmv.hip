@@ -655,11 +655,13 @@ k_matfree_rec(int64_t ncl, const double *__restrict__ rin, const double *__restr
 // entry for all 4) no lane idles on a pair outside the cutoff (0.61 of them are inside) or in a
 // list's last chunk, nothing is masked or branched on, and a neighbour's record is gathered 9
 // instead of 45 times per atom. Measured per product, record form -> tile form: 2.4M-atom
-// assembly 676 -> 432 us, 300,000-atom globule 73 -> 60 us, 1,200 atoms 3.7 -> 3.4 us; a periodic
-// slab of 60,000 atoms (per-row kernel before) 92 -> 14 us. FP64 issue bounds it: 19 FP64
+// assembly 676 -> 419 us, 300,000-atom globule 73 -> 55 us, 1,200 atoms 3.7 -> 3.3 us; a periodic
+// slab of 60,000 atoms (per-row kernel before) 92 -> 12.5 us. FP64 issue bounds it: 19 FP64
 // operations per pair at the measured rate of three-register FMAs (2.5 ns per wave and SIMD) are
 // 0.21 ms on the assembly; the same kernel without its LDS reads or without staging takes 0.92 of
-// its time.
+// its time. The order of an atom's terms (inch_anm_tiles) keeps the LDS reads of a half wave on
+// different banks: in list order 57% of the LDS cycles were conflicts and the products took 60 us
+// at 300,000 atoms (now 55), 14.2 in the periodic slab (now 12.5) and 432 on the assembly (now 419).
 // Periodic images: a union entry names its image in its low 4 bits, and the shift is added as
 // the record is staged, so the inner loop is the same.
 // The reciprocal: a float32 seed (about 22 bits; the layout keeps r2 inside float32's normal
@@ -795,6 +797,161 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
   if (rout) rout[6 * slot + 3 + l] = out;
   if (yout) yout[3 * slot + l] = out;
   if (acc) acc[3 * slot + l] = av + mu * out;
+}
+
+// Several right-hand sides on the tile form: Y = (H + plus_i I) X, X and Y row-major [3n, nrhs] in
+// the matrix's order. X is first packed per group of kBlockCols columns into 96-byte records in
+// slot order (k_block_pack), so that a neighbour's entries of a group are one piece of memory and
+// a group's records (10 MB for 100,000 atoms) stay in the caches while all tiles use them: gathering
+// the 32-byte pieces of row-major rows fetched a 128-byte line for each and ran at the memory's
+// rate (1.2 ms for 100,003 atoms and 64 columns). A workgroup takes a tile and a column group: it
+// stages the union's coordinates and entries in LDS, and G lanes per atom walk the atom's list,
+// each forming a pair's geometry (12 FP64 operations and the reciprocal's seed) once for the 9 per
+// column. The halves of a component's four entries change places with bit 3 of 3 x the record's
+// number, so that the reads of 16 lanes spread over all banks. FP64 issue bounds it (VALU busy 82%
+// of the time). 100,003 atoms, 64 columns: the kernel on the cluster layout (one column per lane, a
+// third of its pairs outside the cutoff, 44 gathers per atom) took 1.83 ms; this takes 0.63, of
+// which the packing 0.05.
+constexpr int kBlockCols = 4;
+constexpr size_t kTileBlockLds = 160 * 1024;
+
+// P[(group * slots + q) * 12 + 4 k + c] = X[3 a + k, 4 group + c], a the atom of slot q; zeros on
+// padding slots and past the last column. 16 slots per workgroup, 64 columns at a time through LDS.
+__global__ void __launch_bounds__(192) k_block_pack(int64_t slots, const int32_t *__restrict__ atoms,
+                                                    const double *__restrict__ X, int nrhs, double *__restrict__ P) {
+  __shared__ double tile[16][3][65];
+  const int64_t q0 = 16 * (int64_t)blockIdx.x;
+  const int c0 = 64 * (int)blockIdx.y, nc = nrhs - c0 < 64 ? nrhs - c0 : 64;
+  const int t = threadIdx.x, col = t & 63, comp = t >> 6;
+  double x[16];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {   // 16 rows in flight
+    const int32_t at = q0 + s < slots ? atoms[q0 + s] : -1;
+    x[s] = at >= 0 && col < nc ? X[(3 * (int64_t)at + comp) * nrhs + c0 + col] : 0.0;
+  }
+#pragma unroll
+  for (int s = 0; s < 16; ++s) tile[s][comp][col] = x[s];
+  __syncthreads();
+  const int s = t / 12, u = t % 12, k = u >> 2, c = u & 3;
+  if (q0 + s >= slots) return;
+  const int groups = (nc + kBlockCols - 1) / kBlockCols;
+  double *out = P + ((int64_t)(c0 / kBlockCols) * slots + q0 + s) * 12 + u;
+#pragma unroll 4
+  for (int g = 0; g < groups; ++g) out[12 * slots * (int64_t)g] = tile[s][k][kBlockCols * g + c];
+}
+
+template <int TA, int G, bool PBC>
+__global__ void __launch_bounds__(TA *G)
+k_matfree_tile_block(int64_t slots, const double *__restrict__ rec, const int32_t *__restrict__ atoms,
+                     const int32_t *__restrict__ ulen, const uint32_t *__restrict__ ulist, int ucap, int umax,
+                     const int2 *__restrict__ waves, const u32x4 *__restrict__ pairs, double bx, double by,
+                     double plus_i, const double *__restrict__ P, double *__restrict__ Y, int nrhs) {
+  extern __shared__ double lds[];   // the union's entries (3 x C each), then its coordinates
+  constexpr int NW = TA * G / 64, C = kBlockCols, NT = TA * G;
+  double2 *sx = (double2 *)lds;
+  double *sp = lds + 3 * C * umax;
+  const int64_t t = xcd_block(true);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c0 = C * (int)blockIdx.y;
+  const int ul = ulen[t];
+  const int2 wv = waves[t * NW + w];
+  const int passes = wv.y;
+  const u32x4 *pl = pairs + 64 * (int64_t)wv.x + lane;
+  u32x4 ix = {0, 0, 0, 0};
+  if (passes > 0) ix = pl[0];
+  const int a = tid / G, l = lane & (G - 1);
+  const int32_t at = atoms[TA * t + a];
+  const double *me = rec + 6 * (TA * t + a);
+  const double p0 = me[0], p1 = me[1], p2 = me[2];
+  const double2 *pg = (const double2 *)(P + 12 * slots * (int64_t)blockIdx.y);
+  double v[3][C], s[3][C];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double2 x = pg[6 * (TA * t + a) + 2 * k], y = pg[6 * (TA * t + a) + 2 * k + 1];
+    v[k][0] = x.x;
+    v[k][1] = x.y;
+    v[k][2] = y.x;
+    v[k][3] = y.y;
+#pragma unroll
+    for (int c = 0; c < C; ++c) s[k][c] = 0.0;
+  }
+  const uint32_t lim = 48u * (uint32_t)ul;   // offsets from here on are empty passes
+  for (int e = tid; e < ul; e += NT) {
+    const uint32_t w32 = ulist[t * ucap + e], slot = w32 / 48u;
+    const double *q = rec + 6 * (int64_t)slot;
+    const double2 *x = pg + 6 * (int64_t)slot;
+    double q0 = q[0], q1 = q[1];
+    if constexpr (PBC) {
+      const int bit = (int)(w32 & 15u);
+      q0 += (double)(bit / 3 - 1) * bx;
+      q1 += (double)(bit % 3 - 1) * by;
+    }
+    sp[3 * e] = q0;
+    sp[3 * e + 1] = q1;
+    sp[3 * e + 2] = q[2];
+    const int f = (3 * e >> 3) & 1;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      sx[6 * e + 2 * k + f] = x[2 * k];
+      sx[6 * e + 2 * k + (f ^ 1)] = x[2 * k + 1];
+    }
+  }
+  __syncthreads();
+  auto term = [&](uint32_t off) {   // off = 48 x the record's number
+    const double *q = (const double *)((const char *)sp + (off >> 1));
+    const uint32_t f = (off >> 3) & 16u;
+    const char *ra = (const char *)sx + (2 * off + f), *rb = (const char *)sx + (2 * off + (f ^ 16u));
+    double2 x[3][2];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      x[k][0] = *(const double2 *)(ra + 32 * k);
+      x[k][1] = *(const double2 *)(rb + 32 * k);
+    }
+    const double d0 = q[0] - p0, d1 = q[1] - p1, d2 = q[2] - p2;
+    const double r2 = __builtin_fma(d2, d2, __builtin_fma(d1, d1, d0 * d0));
+    double inv = (double)__builtin_amdgcn_rcpf((float)r2);
+    const double e = __builtin_fma(-r2, inv, 1.0);
+    inv = __builtin_fma(inv, __builtin_fma(e, e, e), inv);
+    const double g0 = d0 * inv, g1 = d1 * inv, g2 = d2 * inv;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const double x0 = c & 1 ? x[0][c >> 1].y : x[0][c >> 1].x, x1 = c & 1 ? x[1][c >> 1].y : x[1][c >> 1].x,
+                   x2 = c & 1 ? x[2][c >> 1].y : x[2][c >> 1].x;
+      const double w0 = v[0][c] - x0, w1 = v[1][c] - x1, w2 = v[2][c] - x2;
+      const double dw = __builtin_fma(d2, w2, __builtin_fma(d1, w1, d0 * w0));
+      s[0][c] = __builtin_fma(g0, dw, s[0][c]);
+      s[1][c] = __builtin_fma(g1, dw, s[1][c]);
+      s[2][c] = __builtin_fma(g2, dw, s[2][c]);
+    }
+  };
+  for (int k = 0; k < passes; k += 8) {
+    u32x4 nx = ix;
+    if (k + 8 < passes) nx = pl[8 * (k + 8)];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t o0 = ix[q] & 0xffffu, o1 = ix[q] >> 16;
+      if (k + 2 * q < passes && o0 < lim) term(o0);
+      if (k + 2 * q + 1 < passes && o1 < lim) term(o1);
+    }
+    ix = nx;
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int c = 0; c < C; ++c) s[k][c] = group_sum<G>(s[k][c]);
+  if (at >= 0 && l < C && c0 + l < nrhs) {   // lane l of the atom's writes column c0 + l
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      double y = s[k][0], x = v[k][0];
+#pragma unroll
+      for (int c = 1; c < C; ++c)
+        if (l == c) {
+          y = s[k][c];
+          x = v[k][c];
+        }
+      Y[(3 * (int64_t)at + k) * nrhs + c0 + l] = y + plus_i * x;
+    }
+  }
 }
 
 // Records from a vector in the matrix's order: rec's vector part of slot q = v of atom
@@ -1721,6 +1878,54 @@ inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, 
     cur = out;
     out = old;
   }
+  return INCH_OK;
+}
+
+int64_t inch_anm_tile_apply_work_size(int64_t ntile, int32_t tile, int32_t nrhs) {
+  return 12 * ntile * tile * ((nrhs + kBlockCols - 1) / kBlockCols);
+}
+
+inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lanes, const double *rec,
+                                        const int32_t *tile_atoms, const int32_t *ulen, const uint32_t *ulist,
+                                        int32_t ucap, int32_t umax, const int32_t *waves, const uint16_t *pairs,
+                                        double box_x, double box_y, double plus_i, const double *x, double *y,
+                                        int32_t nrhs, double *work, void *stream) {
+  INCH_REQUIRE(ntile > 0 && rec && tile_atoms && ulen && ulist && waves && pairs && x && y && x != y && nrhs > 0 && work,
+               "inch_anm_matfree_tile_apply: bad args");
+  INCH_REQUIRE(inch_tile_shape_ok(tile, lanes), "inch_anm_matfree_tile_apply: no tile shape of %d atoms x %d lanes",
+               tile, lanes);
+  INCH_REQUIRE(umax >= 0 && umax <= ucap && ucap <= inch_tile_max_union(tile), "inch_anm_matfree_tile_apply: bad union");
+  INCH_REQUIRE(nrhs <= kBlockCols * 65535, "inch_anm_matfree_tile_apply: nrhs too large");
+  const size_t lds = (size_t)umax * (24 * kBlockCols + 24);
+  if (lds > kTileBlockLds)
+    INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_matfree_tile_apply: a tile's %d neighbours exceed the LDS", umax);
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t slots = ntile * tile;
+  k_block_pack<<<dim3((unsigned)((slots + 15) / 16), (unsigned)((nrhs + 63) / 64)), 192, 0, st>>>(slots, tile_atoms, x,
+                                                                                                 nrhs, work);
+  HIP_TRY(hipGetLastError());
+  const dim3 grid((unsigned)ntile, (unsigned)((nrhs + kBlockCols - 1) / kBlockCols));
+#define INCH_TB(TA, GG, PB)                                                                                         \
+  do {                                                                                                              \
+    HIP_TRY(hipFuncSetAttribute((const void *)k_matfree_tile_block<TA, GG, PB>,                                     \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                             \
+    k_matfree_tile_block<TA, GG, PB><<<grid, TA * GG, lds, st>>>(slots, rec, tile_atoms, ulen, ulist, ucap, umax,   \
+                                                                 (const int2 *)waves, (const u32x4 *)pairs, box_x,  \
+                                                                 box_y, plus_i, work, y, nrhs);                     \
+  } while (0)
+#define INCH_TILE_BLOCK(TA, GG)        \
+  if (tile == TA && lanes == GG) {     \
+    if (box_x > 0.0)                   \
+      INCH_TB(TA, GG, true);           \
+    else                               \
+      INCH_TB(TA, GG, false);          \
+  }
+  INCH_TILE_BLOCK(64, 8)
+  INCH_TILE_BLOCK(32, 16)
+  INCH_TILE_BLOCK(16, 32)
+#undef INCH_TILE_BLOCK
+#undef INCH_TB
+  HIP_TRY(hipGetLastError());
   return INCH_OK;
 }
 

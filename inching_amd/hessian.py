@@ -27,8 +27,8 @@ def tile_shapes(n):
     """(atoms, lanes per atom) of the tiles for n atoms, the preferred shape first, then the
     smaller ones, whose unions are smaller. Few atoms need many lanes each to fill the chip, many
     atoms large tiles, which share their neighbours' records: per product (64, 8) / (32, 16) /
-    (16, 32) took 4.5 / 3.7 / 3.4 us at 1,200 atoms, 5.0 / 3.9 / 4.5 at 6,000, 7.7 / 6.9 / 7.9
-    at 20,000 and 60 / 63 / 84 at 300,000."""
+    (16, 32) took 4.4 / 3.6 / 3.3 us at 1,200 atoms, 4.7 / 3.8 / 4.3 at 6,000, 7.1 / 6.3 / 7.7
+    at 20,000 and 55 / 61 / 82 at 300,000."""
     shapes = ((64, 8), (32, 16), (16, 32))
     return shapes[2 if n < 4000 else (1 if n < 40000 else 0):]
 
@@ -227,7 +227,9 @@ class BlockHessian:
     def matfree(self, X):
         """FP64 (H + PlusI I) X recomputed from coordinates (X [3n] or [3n, r])."""
         Y = torch.empty_like(X)
-        if self.images is not None:
+        if self.tiles() is not None and X.numel() and X.dtype == torch.float64 and Y.is_contiguous():
+            self.tiles().apply(X.contiguous(), Y, self.plus_i)
+        elif self.images is not None:
             ops.matfree_pbc(self.xyz, self.rowptr, self.col, self.images, self.box, self.plus_i, X.contiguous(), Y)
         elif self.clusters() is not None:
             ops.matfree_cl_apply(self.xyz, self.clusters(), self.plus_i, X.contiguous(), Y)

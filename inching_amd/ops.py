@@ -317,7 +317,7 @@ class Tiles:
         nt = C.c_int64(0)
         call("inch_anm_tile_order", n, P(xyz), float(side), tile, P(order), P(start), C.byref(nt), stream_ptr(stream))
         nt = nt.value
-        self.shape, self.ntile, self.slots = (tile, lanes), nt, nt * tile
+        self.shape, self.ntile, self.slots, self.nd = (tile, lanes), nt, nt * tile, 3 * n
         ucap = 65536 // 48 - tile
         self.atoms = torch.empty(self.slots, **i32)
         slot_of = torch.empty(n, **i32)
@@ -355,6 +355,18 @@ class Tiles:
         self._vectors(acc, y)
         call("inch_anm_matfree_tile", self.ntile, *self.shape, P(rec_in), P(rec_z), P(rec_out), P(y), *self._lists,
              float(plus_i), float(s1), float(c0), float(c2), P(acc), float(mu), stream_ptr(stream))
+
+    def apply(self, X, Y, plus_i, stream=None):
+        """Y = (H + plus_i I) X in the matrix's order, float64 [3n] or [3n, r] (inch_anm_matfree_tile_apply)."""
+        if X.shape != Y.shape or X.shape[0] != self.nd or X.dim() > 2:
+            raise ValueError("X and Y must be [3n] or [3n, r]")
+        if X.dtype != torch.float64 or Y.dtype != torch.float64 or not X.is_contiguous() or not Y.is_contiguous():
+            raise ValueError("X and Y must be contiguous float64 [3n, r]")
+        r = 1 if X.dim() == 1 else X.shape[1]
+        size = int(call("inch_anm_tile_apply_work_size", self.ntile, self.shape[0], r))
+        work = torch.empty(size, dtype=torch.float64, device=X.device)
+        call("inch_anm_matfree_tile_apply", self.ntile, *self.shape, P(self.rec), P(self.atoms), *self._lists,
+             float(plus_i), P(X), P(Y), r, P(work), stream_ptr(stream))
 
     def chebyshev(self, recs, mu, cc, dd, plus_i, acc, stream=None):
         """acc += sum_k mu[k] T_k((A - cc) / dd) x over k >= 1, x packed in recs[0]

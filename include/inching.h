@@ -293,8 +293,8 @@ inch_status inch_anm_matfree_rec(int64_t ncl, const double *rec_in, const double
  * (sx + 1) * 3 + (sy + 1) of the periodic image, 4 for open boundaries); every wave of
  * 64 / lanes atoms has waves int32 [2 tile ntile lanes / 64] = (first block, passes) and blocks
  * of 64 lanes x 8 passes of uint16 byte offsets into the union's 48-byte records, pairs uint16
- * [512 pair_blocks]: term q of an atom at pass q / lanes, its lane q % lanes; passes beyond an
- * atom's terms hold 48 (ulen + the atom's place in its tile). Pairs at zero distance have no
+ * [512 pair_blocks]: an atom's terms in some order (one that spreads the LDS banks) over its
+ * lanes' passes, whose other places hold 48 (ulen + the atom's place in its tile). Pairs at zero distance have no
  * term. (tile, lanes) is one of (64, 8), (32, 16), (16, 32); ucap at most
  * 65536 / 48 - tile. images NULL: open boundaries; else the masks of
  * inch_neighbors_celllist_pbc with its box.
@@ -328,6 +328,16 @@ inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, 
                                     const int32_t *ulen, const uint32_t *ulist, int32_t ucap, int32_t umax,
                                     const int32_t *waves, const uint16_t *pairs, double box_x, double box_y,
                                     double plus_i, double *acc, void *stream);
+/* inch_anm_matfree_apply on the tile form: Y = (H + plus_i I) X for nrhs row-major right-hand
+ * sides (X, Y float64 [3n, nrhs]) in the matrix's order; rec: records with the layout's
+ * coordinates (their vector parts are not read); work: inch_anm_tile_apply_work_size doubles.
+ * INCH_ERR_CAPACITY when the longest union does not fit the LDS with four columns (over 1,365). */
+int64_t inch_anm_tile_apply_work_size(int64_t ntile, int32_t tile, int32_t nrhs);
+inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lanes, const double *rec,
+                                        const int32_t *tile_atoms, const int32_t *ulen, const uint32_t *ulist,
+                                        int32_t ucap, int32_t umax, const int32_t *waves, const uint16_t *pairs,
+                                        double box_x, double box_y, double plus_i, const double *x, double *y,
+                                        int32_t nrhs, double *work, void *stream);
 /* Vector part of rec for slot q = v[3 a .. 3 a + 2] with a = cluster_atoms[q] (0 for padding),
  * or v[3 q .. 3 q + 2] when cluster_atoms is NULL (v in slot order, [12 ncl]); acc (may be
  * NULL) [12 ncl] = mu0 times the same. */

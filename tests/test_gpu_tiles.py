@@ -121,6 +121,29 @@ def test_tile_layout_and_product(cuda, case, shape):
     assert np.abs(back.cpu().numpy() - ref).max() <= 1e-12 * max(np.abs(v).max() for v in t)
 
 
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("case", CASES)
+def test_tile_block_product(cuda, case, shape):
+    """Several right-hand sides: column counts around the groups of 4 and the 64 of the packing."""
+    from inching_amd import ops
+    print("case: tile block %s %s" % (case, shape), flush=True)
+    X, box, xyz, ip, ix, im, D = _matrix(case)
+    T = ops.Tiles(xyz, ip, ix, 8.0 * (shape[0] / 117.0) ** (1 / 3) * 1.6, shape, images=im, box=box)
+    rng = np.random.default_rng(7)
+    for r in (1, 2, 3, 4, 5, 63, 64, 67):
+        V = rng.standard_normal((3 * len(X), r))
+        Y = torch.full(V.shape, float("nan"), dtype=torch.float64, device="cuda")
+        T.apply(torch.as_tensor(V, device="cuda"), Y, 1.0)
+        ref = D @ V
+        assert np.abs(Y.cpu().numpy() - ref).max() <= 1e-12 * np.abs(ref).max(), r
+    v = torch.as_tensor(V[:, 0].copy(), device="cuda")
+    y = torch.empty_like(v)
+    T.apply(v, y, 1.0)
+    assert np.abs(y.cpu().numpy() - ref[:, 0]).max() <= 1e-12 * np.abs(ref).max()
+    with pytest.raises(ValueError):
+        T.apply(Y.T, Y.T, 1.0)
+
+
 def test_periodic_filter_in_slot_order_matches_matrix_order(cuda):
     from inching_amd import chebyshev as CH
     from inching_amd.hessian import build_hessian
