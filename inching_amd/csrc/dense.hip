@@ -22,50 +22,72 @@ constexpr int kChunk = 32;   // columns of n staged in LDS per step
 constexpr int kGramBlocks = 256;   // fixed grid of the residual-norm reduction
 constexpr int kGramGrid = 1024;    // most column blocks of a Gram product (at least 1,024 columns each)
 
-// One workgroup = 4 waves; wave w owns output rows [16w, 16w+16) of the tile and the 4
-// column blocks of 16. Operands are staged through LDS with coalesced row loads; the
-// contraction dimension is the column index i of X and Y.
+// One workgroup = 4 waves; wave w owns output rows [16w, 16w+16) of the tile and its NT column
+// blocks of 16 (as many as Y has rows left: 6 rows of Y need one, not four). Operands are staged
+// through LDS with coalesced row loads, the next chunk's in flight while the current one is used;
+// when X and Y are the same rows (SAME) they are staged once. The contraction dimension is the
+// column index i of X and Y. Memory bounds it: 64 x 64 over 900,000 columns took 289 us with both
+// operands staged and a wait on memory per chunk, now 164 (0.46 GB read, the matrix cores busy for
+// three quarters of it); 64 x 6 with its sum took 247, now 94.
 // v_mfma_f64_16x16x4f64 operand layout: A (16x4): lane l holds A[l%16][l/16];
 // B (4x16): lane l holds B[l/16][l%16]; D (16x16): lane l, element r holds
 // D[(l/16) + 4*r][l%16] (checked on gfx950 with one-hot operands).
+template <int NT, bool SAME>
 __global__ void __launch_bounds__(256) k_gram_mfma(int64_t len, int k1, const double *__restrict__ X, int64_t ldx,
                                                     int k2, const double *__restrict__ Y, int64_t ldy,
                                                     double *__restrict__ part) {
+  constexpr int PX = kTile * kChunk / 256, PY = SAME ? 0 : 16 * NT * kChunk / 256;   // elements staged per thread
   __shared__ double xs[kTile][kChunk + 1];
-  __shared__ double ys[kTile][kChunk + 1];
+  __shared__ double ys_own[SAME ? 1 : 16 * NT][kChunk + 1];
+  auto &ys = *reinterpret_cast<double(*)[SAME ? kTile : 16 * NT][kChunk + 1]>(SAME ? &xs[0][0] : &ys_own[0][0]);
   const int a0 = blockIdx.y * kTile, b0 = blockIdx.z * kTile;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  double4_t acc[4];
+  double4_t acc[NT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < NT; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
   const int64_t per = (len + gridDim.x - 1) / gridDim.x;
   const int64_t i_beg = blockIdx.x * per;
   const int64_t i_end = (i_beg + per < len) ? i_beg + per : len;
+  // thread t stages column t % 32 of rows t / 32 + 8 s
+  const int c = tid % kChunk, r0 = tid / kChunk;
+  double xr[PX], yr[PY > 0 ? PY : 1];
+  auto fetch = [&](int64_t i0) {
+    const int64_t i = i0 + c;
+    const bool in = i < i_end;
+#pragma unroll
+    for (int s = 0; s < PX; ++s) {
+      const int r = a0 + r0 + 8 * s;
+      xr[s] = (in && r < k1) ? X[(int64_t)r * ldx + i] : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < PY; ++s) {
+      const int r = b0 + r0 + 8 * s;
+      yr[s] = (in && r < k2) ? Y[(int64_t)r * ldy + i] : 0.0;
+    }
+  };
+  if (i_beg < i_end) fetch(i_beg);
   for (int64_t i0 = i_beg; i0 < i_end; i0 += kChunk) {
     __syncthreads();
-    // stage: 64 rows x 32 columns of each operand; thread t loads column t%32 of rows t/32 + 8s
-    for (int s = 0; s < kTile * kChunk / 256; ++s) {
-      const int r = tid / kChunk + s * (256 / kChunk);
-      const int c = tid % kChunk;
-      const int64_t i = i0 + c;
-      xs[r][c] = (a0 + r < k1 && i < i_end) ? X[(int64_t)(a0 + r) * ldx + i] : 0.0;
-      ys[r][c] = (b0 + r < k2 && i < i_end) ? Y[(int64_t)(b0 + r) * ldy + i] : 0.0;
-    }
+#pragma unroll
+    for (int s = 0; s < PX; ++s) xs[r0 + 8 * s][c] = xr[s];
+#pragma unroll
+    for (int s = 0; s < PY; ++s) ys_own[r0 + 8 * s][c] = yr[s];
     __syncthreads();
+    if (i0 + kChunk < i_end) fetch(i0 + kChunk);
 #pragma unroll
     for (int kk = 0; kk < kChunk; kk += 4) {
       const double av = xs[16 * w + (lane & 15)][kk + (lane >> 4)];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < NT; ++t) {
         const double bv = ys[16 * t + (lane & 15)][kk + (lane >> 4)];
         acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
       }
     }
   }
-  // write the 64x64 partial tile of this block
+  // write the 64 x (16 NT) partial tile of this block
   double *dst = part + (int64_t)blockIdx.x * k1 * k2;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
+  for (int t = 0; t < NT; ++t) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int a = a0 + 16 * w + (lane >> 4) + 4 * r;
@@ -75,15 +97,26 @@ __global__ void __launch_bounds__(256) k_gram_mfma(int64_t len, int k1, const do
   }
 }
 
-// Sum of nparts partials per output: thread per output when there are many outputs,
-// workgroup per output (fixed tree) when there are few. Both orders are fixed.
-__global__ void k_sum_parts(int nparts, int64_t m, const double *__restrict__ part, double *__restrict__ out,
-                            int do_sqrt) {
-  const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (j >= m) return;
+// Sum of nparts partials per output. Many outputs: 32 per workgroup, 8 threads each over every 8th
+// partial, their sums added in order (one thread per output waited for all nparts loads: 254 us
+// for 879 partials of 4,096 outputs, now 9). Few: a workgroup per output (fixed tree). All
+// orders are fixed.
+__global__ void __launch_bounds__(256) k_sum_parts(int nparts, int64_t m, const double *__restrict__ part,
+                                                   double *__restrict__ out) {
+  __shared__ double red[8][32];
+  const int c = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int64_t j = blockIdx.x * (int64_t)32 + c;
   double s = 0.0;
-  for (int p = 0; p < nparts; ++p) s += part[(int64_t)p * m + j];
-  out[j] = do_sqrt ? sqrt(s) : s;
+  if (j < m) {
+#pragma unroll 8
+    for (int p = g; p < nparts; p += 8) s += part[(int64_t)p * m + j];
+  }
+  red[g][c] = s;
+  __syncthreads();
+  if (g || j >= m) return;
+#pragma unroll
+  for (int q = 1; q < 8; ++q) s += red[q][c];
+  out[j] = s;
 }
 
 __global__ void __launch_bounds__(256) k_sum_parts_wg(int nparts, int64_t m, const double *__restrict__ part,
@@ -139,11 +172,26 @@ inch_status inch_gram(int64_t len, int32_t k1, const double *X, int64_t ldx, int
   if (gx > kGramGrid) gx = kGramGrid;
   if (gx < 1) gx = 1;
   dim3 grid((unsigned)gx, (k1 + kTile - 1) / kTile, (k2 + kTile - 1) / kTile);
-  k_gram_mfma<<<grid, 256, 0, st>>>(len, k1, X, ldx, k2, Y, ldy, work);
+  // one block of rows with itself is staged once; beyond 64 rows the tiles off the diagonal need both
+  const bool same = X == Y && ldx == ldy && k1 == k2 && k1 <= kTile;
+#define INCH_GRAM(NT)                                                                        \
+  do {                                                                                       \
+    if (same)                                                                                \
+      k_gram_mfma<NT, true><<<grid, 256, 0, st>>>(len, k1, X, ldx, k2, Y, ldy, work);        \
+    else                                                                                     \
+      k_gram_mfma<NT, false><<<grid, 256, 0, st>>>(len, k1, X, ldx, k2, Y, ldy, work);       \
+  } while (0)
+  if (k2 <= 16)
+    INCH_GRAM(1);
+  else if (k2 <= 32)
+    INCH_GRAM(2);
+  else
+    INCH_GRAM(4);
+#undef INCH_GRAM
   HIP_TRY(hipGetLastError());
   const int64_t m = (int64_t)k1 * k2;
   if (m >= 1024)
-    k_sum_parts<<<(unsigned)((m + 255) / 256), 256, 0, st>>>((int)gx, m, work, G, 0);
+    k_sum_parts<<<(unsigned)((m + 31) / 32), 256, 0, st>>>((int)gx, m, work, G);
   else
     k_sum_parts_wg<<<(unsigned)m, 256, 0, st>>>((int)gx, m, work, G, 0);
   HIP_TRY(hipGetLastError());

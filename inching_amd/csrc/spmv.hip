@@ -1244,34 +1244,53 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 // A[l % 16][l / 16]; B (4 x 16): lane l holds B[l / 16][l % 16]; D (16 x 16): lane l, element
 // e holds D[l / 16 + 4 e][l % 16]. Here A[q][r] = W[r][q] and B[r][i] = V[r][i]: each lane
 // loads one element of V per slice and 4 rows (16 consecutive columns of 4 rows per wave).
-template <int NS, int NT>
+// The next 4 rows of V are loaded while the products of the current 4 run: 900,000 columns took
+// 277 us at m = k = 64, now 235 to 263, and 604 at m = 192, now 539 (0.92 and 1.84 GB moved). Loads two
+// steps ahead, two slices instead of four and workgroups that walk column blocks gained nothing.
+// SUB: out[q, i] -= the sum instead, in one pass over out.
+template <int NS, int NT, bool SUB>
 __global__ void __launch_bounds__(256) k_rr_combine_mfma(int64_t len, int m, int k, const double *__restrict__ V,
                                                           int64_t ld, const double *__restrict__ W,
                                                           double *__restrict__ out, int64_t ld_out) {
-  __shared__ double ws[64][65];
+  __shared__ double ws[64][16 * NT + 1];
   const int q0 = blockIdx.y * 16 * NT;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  int64_t col[NS];
+  // columns of the wave's slices: c0 + 64 s
+  const int64_t c0 = (int64_t)blockIdx.x * (64 * NS) + 16 * w + (lane & 15);
+  auto fetch = [&](int r, double (&v)[NS]) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) col[s] = (int64_t)blockIdx.x * (64 * NS) + 64 * s + 16 * w + (lane & 15);
+    for (int s = 0; s < NS; ++s) v[s] = (c0 + 64 * s < len && r < m) ? V[(int64_t)r * ld + c0 + 64 * s] : 0.0;
+  };
+  double next[NS];
+  fetch(lane >> 4, next);
   double4_t acc[NS][NT];
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[s][t] = (double4_t){0.0, 0.0, 0.0, 0.0};
+    for (int t = 0; t < NT; ++t) {
+      acc[s][t] = (double4_t){0.0, 0.0, 0.0, 0.0};
+      if constexpr (SUB) {   // the sums start from out, all of its loads in flight
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int q = q0 + 16 * t + (lane >> 4) + 4 * e;
+          if (q < k && c0 + 64 * s < len) acc[s][t][e] = out[(int64_t)q * ld_out + c0 + 64 * s];
+        }
+      }
+    }
   for (int rc = 0; rc < m; rc += 64) {
     const int nr = (m - rc) < 64 ? (m - rc) : 64;
-    __syncthreads();
+    if (rc) __syncthreads();
     for (int t = tid; t < 64 * 16 * NT; t += 256) {
       const int r = t / (16 * NT), q = t % (16 * NT);
-      ws[r][q] = (r < nr && q0 + q < k) ? W[(int64_t)(rc + r) * k + q0 + q] : 0.0;
+      const double v = (r < nr && q0 + q < k) ? W[(int64_t)(rc + r) * k + q0 + q] : 0.0;
+      ws[r][q] = SUB ? -v : v;
     }
     __syncthreads();
     for (int r0 = 0; r0 < nr; r0 += 4) {
-      const int r = r0 + (lane >> 4);
       double bv[NS];
 #pragma unroll
-      for (int s = 0; s < NS; ++s) bv[s] = (col[s] < len && r < nr) ? V[(int64_t)(rc + r) * ld + col[s]] : 0.0;
+      for (int s = 0; s < NS; ++s) bv[s] = next[s];
+      fetch(rc + r0 + 4 + (lane >> 4), next);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const double av = ws[r0 + (lane >> 4)][16 * t + (lane & 15)];
@@ -1282,14 +1301,42 @@ __global__ void __launch_bounds__(256) k_rr_combine_mfma(int64_t len, int m, int
   }
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    if (col[s] >= len) continue;
+    if (c0 + 64 * s >= len) continue;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int q = q0 + 16 * t + (lane >> 4) + 4 * e;
-        if (q < k) out[(int64_t)q * ld_out + col[s]] = acc[s][t][e];
+        if (q < k) out[(int64_t)q * ld_out + c0 + 64 * s] = acc[s][t][e];
       }
+  }
+}
+
+// out[q, i] -= sum_r W[r, q] V[r, i] for m <= 8 rows V (rigid-body rows): a thread takes one column
+// and 16 rows of out, whose loads are all in flight with those of V; the weights are wave-uniform.
+// Memory bounds it (out read and written): 64 rows of 900,000 off 6 in 162 us; the matrix-core
+// form takes 229, a combination and an axpby 430.
+template <int M>
+__global__ void __launch_bounds__(256) k_project_few(int64_t len, int m, int k, const double *__restrict__ V, int64_t ld,
+                                                     const double *__restrict__ W, double *__restrict__ out,
+                                                     int64_t ld_out) {
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (i >= len) return;
+  const int q0 = 16 * blockIdx.y;
+  double v[M], x[16];
+#pragma unroll
+  for (int r = 0; r < M; ++r) v[r] = r < m ? V[(int64_t)r * ld + i] : 0.0;
+#pragma unroll
+  for (int q = 0; q < 16; ++q)
+    if (q0 + q < k) x[q] = out[(int64_t)(q0 + q) * ld_out + i];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    if (q0 + q >= k) break;
+    double s = 0.0;
+#pragma unroll
+    for (int r = 0; r < M; ++r)
+      if (r < m) s = __builtin_fma(W[(int64_t)r * k + q0 + q], v[r], s);
+    out[(int64_t)(q0 + q) * ld_out + i] = x[q] - s;
   }
 }
 
@@ -1970,6 +2017,25 @@ namespace {
 // per-block partial dots, the reduced dots, the coefficients, the norm partials). Every word
 // of `work` that a kernel reads was written earlier in the same step, so the scratch needs no
 // clearing between steps.
+template <bool SUB>
+inch_status launch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld, const double *W,
+                              double *out, int64_t ld_out, hipStream_t st) {
+  // 4 output tiles with 4 slices (256 columns) per workgroup, fewer tiles with 8 slices (measured
+  // best: 8 slices with 4 tiles took 0.74 against 0.68 ms for m = 192, k = 64, 900k columns)
+  if (k > 32) {
+    dim3 grid((unsigned)((len + 255) / 256), (unsigned)((k + 63) / 64));
+    k_rr_combine_mfma<4, 4, SUB><<<grid, 256, 0, st>>>(len, m, k, V, ld, W, out, ld_out);
+  } else if (k > 16) {
+    dim3 grid((unsigned)((len + 511) / 512), 1);
+    k_rr_combine_mfma<8, 2, SUB><<<grid, 256, 0, st>>>(len, m, k, V, ld, W, out, ld_out);
+  } else {
+    dim3 grid((unsigned)((len + 511) / 512), 1);
+    k_rr_combine_mfma<8, 1, SUB><<<grid, 256, 0, st>>>(len, m, k, V, ld, W, out, ld_out);
+  }
+  HIP_TRY(hipGetLastError());
+  return INCH_OK;
+}
+
 inch_status dcgs2_launch(int64_t len, int32_t J, double *V, int64_t ld, double *u, double *alpha,
                          const double *beta, double *beta_out, double *vnext, double *work, hipStream_t st) {
   constexpr int JT = 8;
@@ -2171,20 +2237,17 @@ inch_status inch_vec_axpby(int64_t len, double a, const void *x, int32_t xdt, do
 inch_status inch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld, const double *W,
                             double *out, int64_t ld_out, void *stream) {
   INCH_REQUIRE(len > 0 && m > 0 && k > 0 && V && W && out && ld >= len && ld_out >= len, "inch_rr_combine: bad args");
-  hipStream_t st = (hipStream_t)stream;
-  // 4 output tiles with 4 slices (256 columns) per workgroup, fewer tiles with 8 slices (measured
-  // best: 8 slices with 4 tiles took 0.74 against 0.68 ms for m = 192, k = 64, 900k columns)
   INCH_REQUIRE(len < ((int64_t)1 << 38) && k <= 64 * 65535, "inch_rr_combine: len or k too large");
-  if (k > 32) {
-    dim3 grid((unsigned)((len + 255) / 256), (unsigned)((k + 63) / 64));
-    k_rr_combine_mfma<4, 4><<<grid, 256, 0, st>>>(len, m, k, V, ld, W, out, ld_out);
-  } else if (k > 16) {
-    dim3 grid((unsigned)((len + 511) / 512), 1);
-    k_rr_combine_mfma<8, 2><<<grid, 256, 0, st>>>(len, m, k, V, ld, W, out, ld_out);
-  } else {
-    dim3 grid((unsigned)((len + 511) / 512), 1);
-    k_rr_combine_mfma<8, 1><<<grid, 256, 0, st>>>(len, m, k, V, ld, W, out, ld_out);
-  }
+  return launch_rr_combine<false>(len, m, k, V, ld, W, out, ld_out, (hipStream_t)stream);
+}
+
+inch_status inch_rr_project(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld, const double *W,
+                            double *out, int64_t ld_out, void *stream) {
+  INCH_REQUIRE(len > 0 && m > 0 && k > 0 && V && W && out && ld >= len && ld_out >= len, "inch_rr_project: bad args");
+  INCH_REQUIRE(len < ((int64_t)1 << 38) && k <= 64 * 65535, "inch_rr_project: len or k too large");
+  if (m > 8) return launch_rr_combine<true>(len, m, k, V, ld, W, out, ld_out, (hipStream_t)stream);
+  k_project_few<8><<<dim3((unsigned)((len + 255) / 256), (unsigned)((k + 15) / 16)), 256, 0, (hipStream_t)stream>>>(
+      len, m, k, V, ld, W, out, ld_out);
   HIP_TRY(hipGetLastError());
   return INCH_OK;
 }

@@ -585,6 +585,19 @@ def rr_combine(V, m, W, out, stream=None):
          out.stride(0), stream_ptr(stream))
 
 
+def rr_project(V, m, W, out, stream=None):
+    """out[:k] -= W^T V[:m]   (W float64 [m, k] on device, out [k, len])."""
+    k = W.shape[1]
+    if W.shape[0] != m or V.shape[0] < m or out.shape[0] != k or out.shape[1] != V.shape[1]:
+        raise ValueError("shape mismatch in rr_project")
+    if out.data_ptr() == V.data_ptr():
+        raise ValueError("rr_project output must not alias V")
+    if not out.is_contiguous() or V.stride(1) != 1:
+        raise RuntimeError("rr_project: out must be contiguous, and the rows of V")
+    call("inch_rr_project", V.shape[1], int(m), int(k), P(V), V.stride(0), P(W.contiguous()), P(out),
+         out.stride(0), stream_ptr(stream))
+
+
 class GramWorkspace:
     def __init__(self, k1, k2, device):
         from ._lib import lib

@@ -34,9 +34,7 @@ def orthonormalise(X, Q=None, passes=2):
     if Q is not None:
         for _ in range(2):
             C = ops.gram(X, Q, ws=ws)                     # [k, m]
-            P = torch.empty_like(X)
-            ops.rr_combine(Q, m, C.T.contiguous(), P)     # P[q] = sum_r C[q, r] Q[r]
-            ops.axpby(-1.0, P.view(-1), 1.0, X.view(-1))
+            ops.rr_project(Q, m, C.T.contiguous(), X)     # X[q] -= sum_r C[q, r] Q[r]
     for _ in range(passes):
         G = _gram(X, X, ws)
         G = 0.5 * (G + G.T)

@@ -416,6 +416,10 @@ inch_status inch_dcgs2_step_noalloc(int64_t len, int32_t J, double *V, int64_t l
  * (W float64 [m, k] row-major on device; out must not alias V). FP64 MFMA 16x16x4. */
 inch_status inch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld,
                             const double *W, double *out, int64_t ld_out, void *stream);
+/* out[q*ld_out + i] -= sum_r W[r*k + q] * V[r*ld + i] (arguments as inch_rr_combine; with W = V out^T it
+ * projects the rows of out off those of V, Burn/Orthogonalization/T2.py:64-137). */
+inch_status inch_rr_project(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld, const double *W,
+                            double *out, int64_t ld_out, void *stream);
 
 /* ------------------------------------- learned warm start (graph network) ---- */
 /* No counterpart in the reference (its solvers start from random vectors). Layer widths
