@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "dcgs2.h"
 
 #define HIP_TRY(expr)                                                                      \
   do {                                                                                     \
@@ -17,13 +18,7 @@ namespace {
 
 constexpr int kSegMaxJ = 512;
 
-__device__ __forceinline__ double block_sum(double v, double *red) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
+using dcgs2::block_sum;
 
 // part[c*J + j] = sum_{i in chunk c} V[j*ld + i] * u[i]; blockIdx.y picks the tile of 8 rows
 __global__ void __launch_bounds__(256) k_seg_dot_part(const int64_t *__restrict__ cbeg, const int64_t *__restrict__ cend,
@@ -35,11 +30,17 @@ __global__ void __launch_bounds__(256) k_seg_dot_part(const int64_t *__restrict_
   {
     const int j0 = 8 * (int)blockIdx.y;
     double a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    // rows past the last repeat it and are dropped (no test between the loads)
+    const double *row[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) row[t] = V + (int64_t)(j0 + t < J ? j0 + t : J - 1) * ld;
     for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
       const double ui = u[i];
+      double v[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
-        if (j0 + t < J) a[t] += V[(int64_t)(j0 + t) * ld + i] * ui;
+      for (int t = 0; t < 8; ++t) v[t] = row[t][i];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) a[t] += v[t] * ui;
     }
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -222,127 +223,38 @@ __global__ void __launch_bounds__(256) k_seg_cgs_b(const int64_t *__restrict__ c
 // Delayed CGS2 step, per segment (the segmented form of inch_dcgs2_step): i = J - 1, V[i] is
 // the provisional vector, u = Op V[i].
 
-// Two neighbouring doubles in one load; V, u and a segment's first dof are 8-byte aligned only.
-struct __attribute__((packed, aligned(8))) Pair {
-  double x, y;
-};
-
 // part[c*2J + j] = V_j . u and part[c*2J + J + j] = V_j . w over chunk c (w = V[J-1]), 8 rows per
-// workgroup. Reading V bounds it. The row tiles of a chunk follow each other on one XCD (workgroups go
-// round the 8 XCDs), so u and w come from its L2 after the first tile:
-// 49 rows of 7.2 million dofs in 510 us (2.9 GB, 5.7 TB/s), 654 when the tiles ran one after the other over
-// all chunks, read u and w again from memory and took one double per load.
+// workgroup. Reading V bounds it: 49 rows of 7.2 million dofs in 510 us (2.9 GB, 5.7 TB/s), 654 when the tiles
+// ran one after the other over all chunks, read u and w again from memory and took one double per load.
 __global__ void __launch_bounds__(256) k_seg_dual_dot_part(int nchunk, const int64_t *__restrict__ cbeg,
                                                             const int64_t *__restrict__ cend, int J,
                                                             const double *__restrict__ V, int64_t ld,
                                                             const double *__restrict__ u,
                                                             const double *__restrict__ w, double *__restrict__ part) {
-  __shared__ double red[4][16];
-  const unsigned tiles = (unsigned)(J + 7) / 8, k = blockIdx.x >> 3;
-  const int c = (int)(k / tiles * 8 + (blockIdx.x & 7)), j0 = 8 * (int)(k % tiles);
-  if (c >= nchunk) return;
-  const int64_t b = cbeg[c], e = cend[c];
-  double a[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // V_j . u, then V_j . w
-  const double *Vt = V + (int64_t)j0 * ld;
-  for (int64_t i = b + 2 * (int)threadIdx.x; i < e; i += 512) {
-    if (i + 1 < e) {
-      const Pair ui = *(const Pair *)(u + i), wi = *(const Pair *)(w + i);
-      Pair v[8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t)
-        if (j0 + t < J) v[t] = *(const Pair *)(Vt + t * ld + i);
-#pragma unroll
-      for (int t = 0; t < 8; ++t)
-        if (j0 + t < J) {
-          a[t] += v[t].x * ui.x;
-          a[t] += v[t].y * ui.y;
-          a[8 + t] += v[t].x * wi.x;
-          a[8 + t] += v[t].y * wi.y;
-        }
-    } else {
-      const double ui = u[i], wi = w[i];
-#pragma unroll
-      for (int t = 0; t < 8; ++t)
-        if (j0 + t < J) {
-          const double v = Vt[t * ld + i];
-          a[t] += v * ui;
-          a[8 + t] += v * wi;
-        }
-    }
-  }
-  // 16 sums over the wave: each step gives half of the values to half of the lanes
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int h = 8, m = 32; h > 0; h >>= 1, m >>= 1)
-#pragma unroll
-    for (int t = 0; t < h; ++t) {
-      const double keep = (lane & m) ? a[t + h] : a[t], give = (lane & m) ? a[t] : a[t + h];
-      a[t] = keep + __shfl_xor(give, m, 64);
-    }
-  a[0] += __shfl_xor(a[0], 2, 64);
-  a[0] += __shfl_xor(a[0], 1, 64);
-  if ((lane & 3) == 0) red[threadIdx.x >> 6][lane >> 2] = a[0];
-  __syncthreads();
-  const int q = threadIdx.x;
-  if (q < 16 && j0 + (q & 7) < J)
-    part[(int64_t)c * 2 * J + (q >> 3) * J + j0 + (q & 7)] = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
+  int c, tile;
+  dcgs2::chunk_and_tile((unsigned)(J + 7) / 8, c, tile);
+  if (c < nchunk) dcgs2::dual_dot(cbeg[c], cend[c], J, 8 * tile, V, ld, u, w, part + (int64_t)c * 2 * J);
 }
 
-// One workgroup per segment s: (s_0..s_i, g_0..g_{i-1}, -) are the sums of its chunks' partials
-// (thread groups over every ngrp-th chunk, then in order over the groups). With v_i = ~v_i - sum g_l V_l:
-// coef[s, i] = v_i . u = s_i - g . s, coef[s, j] = s_j - coef[s, i] g_j (j < i),
-// coef[s, J + l] = g_l and alpha_i[s] = coef[s, i] - beta_prev[s] g_{i-1} (the one operator
-// term left in a Krylov basis). Latency bounds it: 6 us for 60 segments of 30 chunks (98 sums each); a
-// sum kernel with one thread per sum took 12 before it, and grew with the chunks of a segment.
+// One workgroup per segment s: its coefficients coef[s], from the partials of its chunks. Latency bounds it:
+// 6 us for 60 segments of 30 chunks (98 sums each); a sum kernel with one thread per sum took 12 before
+// it, and grew with the chunks of a segment.
 __global__ void __launch_bounds__(1024) k_seg_dcgs2_coef(int J, const int64_t *__restrict__ sptr,
                                                           const double *__restrict__ part,
                                                           const double *__restrict__ beta_prev,
                                                           double *__restrict__ coef, double *__restrict__ alpha_i) {
-  __shared__ double red[1024];
-  const int s = blockIdx.x, tid = threadIdx.x;
-  const int i = J - 1;
-  const int width = (2 * J + 63) & ~63, ngrp = 1024 / width;   // width <= 512
-  const int o = tid % width, grp = tid / width;
-  double sum = 0.0;
-  if (o < 2 * J && grp < ngrp) {
-    const int64_t ce = sptr[s + 1];
-#pragma unroll 4
-    for (int64_t c = sptr[s] + grp; c < ce; c += ngrp) sum += part[c * 2 * J + o];
-  }
-  red[tid] = sum;
-  __syncthreads();
-  if (tid < width)
-    for (int q = 1; q < ngrp; ++q) sum += red[q * width + tid];
-  __syncthreads();
-  if (tid < width) red[tid] = sum;
-  __syncthreads();
-  if (tid >= 64) return;
-  const int lane = tid;
-  const double *sv = red, *g = red + J;
-  double *cf = coef + (int64_t)s * 2 * J;
-  double p = 0.0;
-  for (int l = lane; l < i; l += 64) p += g[l] * sv[l];
-  for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off, 64);
-  const double ci = sv[i] - p;
-  for (int j = lane; j < i; j += 64) {
-    cf[j] = sv[j] - ci * g[j];
-    cf[J + j] = g[j];
-  }
-  if (lane == 0) {
-    cf[i] = ci;
-    alpha_i[s] = i > 0 ? ci - beta_prev[s] * g[i - 1] : ci;
-  }
+  const int s = blockIdx.x;
+  dcgs2::coefficients(J, sptr[s], sptr[s + 1], part, beta_prev + s, coef + (int64_t)s * 2 * J, alpha_i + s);
 }
 
 constexpr int kSegSub = 4;   // workgroups per chunk of the update
 
 // u -= sum_{j<=i} coef[s, j] V_j and V[i] -= sum_{l<i} coef[s, J + l] V_l over quarter q of chunk c of
-// segment s, in one read of V[0..i]; part[kSegSub c + q] = |u'|^2 over it. A thread takes 4 dofs at a
-// time (two pairs), the loads of 4 rows in flight. Chunks go last to first: the memory-side cache
-// (256 MB) still holds what the dot products read last (the step over 900,000 dofs and 49 rows, 353 MB,
-// takes 157 us, first to last 170). 49 rows of 7.2 million dofs: 555 us (3.0 GB, 5.5 TB/s), 637 with a
-// workgroup per chunk and one load of V in flight after the other; two workgroups per chunk 569, 8 rows in
-// flight the same.
+// segment s, in one read of V[0..i]; part[kSegSub c + q] = |u'|^2 over it. Chunks go last to first: the
+// memory-side cache (256 MB) still holds what the dot products read last (the step over 900,000 dofs and 49
+// rows, 353 MB, takes 153 us, first to last about 12 more). 49 rows of 7.2 million dofs: 555 us (3.0 GB, 5.5 TB/s), 637
+// with a workgroup per chunk and one load of V in flight after the other; two workgroups per chunk 569, 8 rows
+// in flight the same.
 __global__ void __launch_bounds__(256) k_seg_dcgs2_update(int nchunk, const int64_t *__restrict__ cbeg,
                                                            const int64_t *__restrict__ cend,
                                                            const int32_t *__restrict__ cseg, int J,
@@ -351,50 +263,10 @@ __global__ void __launch_bounds__(256) k_seg_dcgs2_update(int nchunk, const int6
                                                            double *__restrict__ part) {
   __shared__ double red[4];
   const int c = nchunk - 1 - (int)(blockIdx.x / kSegSub), q = (int)(blockIdx.x % kSegSub);
-  const int i = J - 1;
-  const double *ca = coef + (int64_t)cseg[c] * 2 * J, *cg = ca + J;
-  const int64_t b = cbeg[c], per = (cend[c] - b + kSegSub - 1) / kSegSub;
-  const int64_t x0 = b + q * per, x1 = x0 + per < cend[c] ? x0 + per : cend[c];
-  double ss = 0.0;
-  int64_t xb = x0;
-  for (; xb + 1024 <= x1; xb += 1024) {
-    const int64_t x = xb + 2 * (int)threadIdx.x;
-    double su[4] = {0, 0, 0, 0}, sv[4] = {0, 0, 0, 0};
-    const double *Vx = V + x;
-#pragma unroll 4
-    for (int j = 0; j < i; ++j) {
-      const Pair v0 = *(const Pair *)(Vx + (int64_t)j * ld), v1 = *(const Pair *)(Vx + (int64_t)j * ld + 512);
-      const double a = ca[j], g = cg[j];
-      su[0] += a * v0.x, su[1] += a * v0.y, su[2] += a * v1.x, su[3] += a * v1.y;
-      sv[0] += g * v0.x, sv[1] += g * v0.y, sv[2] += g * v1.x, sv[3] += g * v1.y;
-    }
-    const double ai = ca[i];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      Pair *vp = (Pair *)(V + (int64_t)i * ld + x + 512 * h), *up = (Pair *)(u + x + 512 * h);
-      const Pair vi = *vp, uo = *up;
-      const Pair un = {uo.x - (su[2 * h] + ai * vi.x), uo.y - (su[2 * h + 1] + ai * vi.y)};
-      *up = un;
-      *vp = {vi.x - sv[2 * h], vi.y - sv[2 * h + 1]};
-      ss += un.x * un.x;
-      ss += un.y * un.y;
-    }
-  }
-  for (int64_t x = xb + threadIdx.x; x < x1; x += 256) {   // fewer than 1,024 left
-    double su = 0.0, sv = 0.0;
-#pragma unroll 8
-    for (int j = 0; j < i; ++j) {
-      const double v = V[(int64_t)j * ld + x];
-      su += ca[j] * v;
-      sv += cg[j] * v;
-    }
-    const double vi = V[(int64_t)i * ld + x];
-    const double un = u[x] - (su + ca[i] * vi);
-    u[x] = un;
-    V[(int64_t)i * ld + x] = vi - sv;
-    ss += un * un;
-  }
-  const double tot = block_sum(ss, red);
+  const double *ca = coef + (int64_t)cseg[c] * 2 * J;
+  const int64_t b = cbeg[c], e = cend[c], per = (e - b + kSegSub - 1) / kSegSub;
+  const int64_t x0 = b + q * per;
+  const double tot = block_sum(dcgs2::update(x0, x0 + per < e ? x0 + per : e, J, V, ld, ca, ca + J, u), red);
   if (threadIdx.x == 0) part[(int64_t)kSegSub * c + q] = tot;
 }
 
@@ -606,9 +478,8 @@ inch_status inch_seg_dcgs2_step(int32_t nchunk, int32_t S, const int64_t *cbeg, 
   double *part = work;
   double *coef = part + (int64_t)nchunk * 2 * J;
   double *npart = coef + (int64_t)S * 2 * J;
-  const unsigned tiles = (unsigned)(J + 7) / 8;
-  k_seg_dual_dot_part<<<((unsigned)nchunk + 7) / 8 * 8 * tiles, 256, 0, st>>>(nchunk, cbeg, cend, J, V, ld, u,
-                                                                              V + (int64_t)(J - 1) * ld, part);
+  k_seg_dual_dot_part<<<dcgs2::chunk_tile_grid(nchunk, (J + 7) / 8), 256, 0, st>>>(
+      nchunk, cbeg, cend, J, V, ld, u, V + (int64_t)(J - 1) * ld, part);
   HIP_TRY(hipGetLastError());
   k_seg_dcgs2_coef<<<S, 1024, 0, st>>>(J, sptr, part, beta_prev, coef, alpha_i);
   HIP_TRY(hipGetLastError());

@@ -11,9 +11,11 @@
 // group apply the epilogue to the row's 3 dofs.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
+#include "dcgs2.h"
 #include "tile.h"
 
 #define HIP_TRY(expr)                                                                      \
@@ -1146,13 +1148,20 @@ __global__ void __launch_bounds__(256) k_multidot_part(int64_t len, int J, const
   // part[blockIdx.x * J + j] for j in this block's tile [blockIdx.y*JT, +JT)
   const int j0 = blockIdx.y * JT;
   double a[JT];
+  // rows past the last repeat it and are dropped: a test between the loads would make each wait for the one before
+  const double *row[JT];
 #pragma unroll
-  for (int t = 0; t < JT; ++t) a[t] = 0.0;
+  for (int t = 0; t < JT; ++t) {
+    a[t] = 0.0;
+    row[t] = V + (int64_t)(j0 + t < J ? j0 + t : J - 1) * ld;
+  }
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x) {
     const double ui = u[i];
+    double v[JT];
 #pragma unroll
-    for (int t = 0; t < JT; ++t)
-      if (j0 + t < J) a[t] += V[(int64_t)(j0 + t) * ld + i] * ui;
+    for (int t = 0; t < JT; ++t) v[t] = row[t][i];
+#pragma unroll
+    for (int t = 0; t < JT; ++t) a[t] += v[t] * ui;
   }
   __shared__ double red[JT][4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1382,55 +1391,25 @@ __global__ void k_axpby(int64_t len, double a, const X *__restrict__ x, double b
 // Bielich, Langou, Thomas, Swirydowicz, Yamazaki, Boman 2022). The operator correction uses
 // the projected matrix T: Op V[0..i-1] = V[0..i] T[0..i, 0..i-1].
 constexpr int kDcgsMaxJ = 256;
+constexpr int kDcgsChunks = 512;     // most chunks of the dot products
+constexpr int kDcgsChunk = 1024;     // fewest dofs of one: two pairs per thread
+constexpr int kDcgsUpdates = 1024;   // most workgroups of the update
+constexpr int64_t dcgs2_words(int64_t J) { return kDcgsChunks * 2 * J + 4 * J + kDcgsUpdates; }
+constexpr int64_t kDcgsNarrow = 524288;
 
-// part[p*2J + j] = V_j . u (j < J), part[p*2J + J + j] = V_j . w (j < J), w = V[J-1]
-template <int JT>
-__global__ void __launch_bounds__(256) k_dual_dot_part(int64_t len, int J, const double *__restrict__ V, int64_t ld,
+// part[c*2J + j] = V_j . u (j < J), part[c*2J + J + j] = V_j . w (j < J), w = V[J-1], over dofs
+// [c per, (c + 1) per), 8 rows per workgroup. Memory or, for short
+// vectors, the latency of one round of loads bounds it: 64 rows of 18,021 / 150,000 / 900,000 dofs take 5.7 / 16.7 /
+// 88 us (900,000: 5.3 TB/s); 11.9 / 43.6 / 104 with a row test between the loads and the tiles of a chunk apart.
+__global__ void __launch_bounds__(256) k_dual_dot_part(int64_t len, int64_t per, int nchunk, int J,
+                                                        const double *__restrict__ V, int64_t ld,
                                                         const double *__restrict__ u, const double *__restrict__ w,
                                                         double *__restrict__ part) {
-  const int j0 = blockIdx.y * JT;
-  double a[JT], b[JT];
-#pragma unroll
-  for (int t = 0; t < JT; ++t) a[t] = b[t] = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x) {
-    const double ui = u[i], wi = w[i];
-#pragma unroll
-    for (int t = 0; t < JT; ++t)
-      if (j0 + t < J) {
-        const double v = V[(int64_t)(j0 + t) * ld + i];
-        a[t] += v * ui;
-        b[t] += v * wi;
-      }
-  }
-  __shared__ double red[2 * JT][4];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int t = 0; t < JT; ++t) {
-    double x = a[t], y = b[t];
-    for (int off = 32; off > 0; off >>= 1) {
-      x += __shfl_xor(x, off, 64);
-      y += __shfl_xor(y, off, 64);
-    }
-    if (lane == 0) {
-      red[t][wv] = x;
-      red[JT + t][wv] = y;
-    }
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < 2 * JT) {
-    const int t = threadIdx.x % JT, which = threadIdx.x / JT;
-    if (j0 + t < J)
-      part[(int64_t)blockIdx.x * 2 * J + which * J + j0 + t] =
-          ((red[threadIdx.x][0] + red[threadIdx.x][1]) + (red[threadIdx.x][2] + red[threadIdx.x][3]));
-  }
-}
-
-__device__ __forceinline__ double block_sum256(double v, double *red) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
+  int c, tile;
+  dcgs2::chunk_and_tile((unsigned)(J + 7) / 8, c, tile);
+  if (c >= nchunk) return;
+  const int64_t b = c * per;
+  dcgs2::dual_dot(b, b + per < len ? b + per : len, J, 8 * tile, V, ld, u, w, part + (int64_t)c * 2 * J);
 }
 
 // One workgroup. sg = (s, g): s_j = V_j . u (j <= i), g_l = V_l . ~v_i (l < i), i = J - 1,
@@ -1450,7 +1429,7 @@ __global__ void __launch_bounds__(256) k_dcgs2_coef(int J, const double *__restr
   const int tid = threadIdx.x;
   double p = 0.0;
   for (int l = tid; l < i; l += blockDim.x) p += g[l] * s[l];
-  const double ci = s[i] - block_sum256(p, red);
+  const double ci = s[i] - dcgs2::block_sum(p, red);
   for (int j = tid; j < i; j += blockDim.x) {
     coef[j] = s[j] - ci * g[j];
     coef[J + j] = g[j];
@@ -1461,40 +1440,52 @@ __global__ void __launch_bounds__(256) k_dcgs2_coef(int J, const double *__restr
   }
 }
 
-// u -= sum_{j<=i} coef[j] V_j and V[i] -= sum_{l<i} coef[J+l] V_l in one read of V[0..i];
-// part[block] = the block's sum of u'^2. LDS: coefficients staged in LDS (J <= 256);
-// otherwise read from global memory (wave-uniform loads).
-template <bool LDS>
-__global__ void __launch_bounds__(256) k_dcgs2_update(int64_t len, int J, double *__restrict__ V, int64_t ld,
-                                                       const double *__restrict__ coef, double *__restrict__ u,
-                                                       double *__restrict__ part) {
-  __shared__ double cs[LDS ? 2 * kDcgsMaxJ : 1];
+// The sums and the coefficients in one workgroup (J <= kDcgsMaxJ; beyond, k_reduce_parts and k_dcgs2_coef).
+__global__ void __launch_bounds__(1024) k_dcgs2_sum_coef(int J, int nchunk, const double *__restrict__ part,
+                                                          const double *__restrict__ beta_prev,
+                                                          double *__restrict__ coef, double *__restrict__ alpha_i) {
+  dcgs2::coefficients(J, 0, nchunk, part, beta_prev, coef, alpha_i);
+}
+
+// u -= sum_{j<=i} coef[j] V_j and V[i] -= sum_{l<i} coef[J+l] V_l in one read of V[0..i]; part[block] = the
+// block's sum of u'^2. Blocks go from the last dofs to the first (what the dot products read last may still be in
+// the memory-side cache). NARROW: 64 dofs at a time with the rows dealt to the waves.
+// 64 rows of 18,021 / 150,000 / 900,000 dofs: 4.8 (narrow) / 14.9 / 81 us (900,000: 5.9 TB/s), with one
+// load in flight after the other 7.0 / 20 / 98.
+template <bool NARROW>
+__global__ void __launch_bounds__(256) k_dcgs2_update(int64_t len, int64_t per, int J, double *__restrict__ V,
+                                                       int64_t ld, const double *__restrict__ coef,
+                                                       double *__restrict__ u, double *__restrict__ part) {
   __shared__ double red[4];
-  const int i = J - 1;
-  const double *ca = coef, *cg = coef + J;
-  if constexpr (LDS) {
-    for (int t = threadIdx.x; t <= i; t += blockDim.x) cs[t] = coef[t];
-    for (int t = threadIdx.x; t < i; t += blockDim.x) cs[kDcgsMaxJ + t] = coef[J + t];
-    __syncthreads();
-    ca = cs;
-    cg = cs + kDcgsMaxJ;
-  }
+  const int64_t x0 = (gridDim.x - 1 - blockIdx.x) * per, x1 = x0 + per < len ? x0 + per : len;
   double ss = 0.0;
-  for (int64_t d = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; d < len; d += (int64_t)gridDim.x * blockDim.x) {
-    double su = 0.0, sv = 0.0;
-    for (int j = 0; j < i; ++j) {
-      const double v = V[(int64_t)j * ld + d];
-      su += ca[j] * v;
-      sv += cg[j] * v;
-    }
-    const double vi = V[(int64_t)i * ld + d];
-    const double un = u[d] - (su + ca[i] * vi);
-    u[d] = un;
-    V[(int64_t)i * ld + d] = vi - sv;
-    ss += un * un;
-  }
-  const double tot = block_sum256(ss, red);
+  if constexpr (NARROW)
+    for (int64_t x = x0; x < x1; x += 64) ss += dcgs2::update_narrow(x, x1, J, V, ld, coef, coef + J, u);
+  else
+    ss = dcgs2::update(x0, x1, J, V, ld, coef, coef + J, u);
+  const double tot = dcgs2::block_sum(ss, red);
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
+}
+
+// *norm = sqrt of the sum of part[0 .. nparts), which every block forms alike, and (given vnext)
+// vnext = u / *norm, 1,024 dofs a block. Latency bounds it: 3.3 us for 18,021 dofs, a sum and a scaling kernel
+// took 4.9 and the gap between them.
+__global__ void __launch_bounds__(256) k_norm_scale(int64_t len, int nparts, const double *__restrict__ part,
+                                                    const double *__restrict__ u, double *__restrict__ norm,
+                                                    double *__restrict__ vnext) {
+  __shared__ double red[4];
+  const int64_t i0 = blockIdx.x * (int64_t)1024 + threadIdx.x;
+  double x[4], s = 0.0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) x[t] = vnext && i0 + 256 * t < len ? u[i0 + 256 * t] : 0.0;
+  for (int p = threadIdx.x; p < nparts; p += 256) s += part[p];
+  const double nrm = sqrt(dcgs2::block_sum(s, red));
+  if (blockIdx.x == 0 && threadIdx.x == 0) *norm = nrm;
+  if (!vnext) return;
+  const double inv = 1.0 / nrm;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (i0 + 256 * t < len) vnext[i0 + 256 * t] = x[t] * inv;
 }
 
 int grid_for(int64_t len, int bs, int cap) {
@@ -2007,7 +1998,7 @@ inch_status inch_anm_matfree_cl_apply(int64_t n, const double *xyz, int64_t ncl,
   return INCH_OK;
 }
 
-int64_t inch_dcgs2_work_size(int32_t J) { return (int64_t)kRedBlocks * (2 * (int64_t)J + 1) + 4 * (int64_t)J; }
+int64_t inch_dcgs2_work_size(int32_t J) { return dcgs2_words(J); }
 
 }  // extern "C"
 
@@ -2038,30 +2029,42 @@ inch_status launch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V
 
 inch_status dcgs2_launch(int64_t len, int32_t J, double *V, int64_t ld, double *u, double *alpha,
                          const double *beta, double *beta_out, double *vnext, double *work, hipStream_t st) {
-  constexpr int JT = 8;
-  const int gx = grid_for(len, 256, kRedBlocks);
+  const int tiles = (J + 7) / 8;
+  // about 1,024 workgroups for the dot products, few enough partials for the one that sums them (whole step, 100
+  // rows of 60,000 dofs: 37 us with at most 64 or 128 chunks, 43 with 256; 8 rows of 900,000: 43 with 256, 59 with 64)
+  const int64_t most = std::min(kDcgsChunks, std::max(64, 1024 / tiles));
+  const int64_t per = std::max<int64_t>(kDcgsChunk, (len + 2 * most - 1) / (2 * most) * 2);
+  const int gx = (int)((len + per - 1) / per);   // <= most
+  // inch_dcgs2_work_size words: 512 * 2J partials, 4J sums and coefficients, 1,024 squares
   double *part = work;
-  double *sg = part + (int64_t)gx * 2 * J;
-  double *coef = sg + 2 * J;
-  double *npart = coef + 2 * J;
-  dim3 grid(gx, (J + JT - 1) / JT);
-  k_dual_dot_part<JT><<<grid, 256, 0, st>>>(len, J, V, ld, u, V + (int64_t)(J - 1) * ld, part);
+  double *coef = part + (int64_t)gx * 2 * J;
+  double *sg = coef + 2 * J;
+  double *npart = sg + 2 * J;
+  k_dual_dot_part<<<dcgs2::chunk_tile_grid(gx, tiles), 256, 0, st>>>(len, per, gx, J, V, ld, u,
+                                                                         V + (int64_t)(J - 1) * ld, part);
   HIP_TRY(hipGetLastError());
-  k_reduce_parts<<<2 * J, 256, 0, st>>>(gx, 2 * J, part, sg, 0);
-  HIP_TRY(hipGetLastError());
-  k_dcgs2_coef<<<1, 256, 0, st>>>(J, sg, beta, coef, alpha + (J - 1));
-  HIP_TRY(hipGetLastError());
-  if (J <= kDcgsMaxJ)
-    k_dcgs2_update<true><<<gx, 256, 0, st>>>(len, J, V, ld, coef, u, npart);
-  else
-    k_dcgs2_update<false><<<gx, 256, 0, st>>>(len, J, V, ld, coef, u, npart);
-  HIP_TRY(hipGetLastError());
-  k_reduce_parts<<<1, 256, 0, st>>>(gx, 1, npart, beta_out, 1);
-  HIP_TRY(hipGetLastError());
-  if (vnext) {
-    k_scale_div<<<grid_for(len, 256, 4096), 256, 0, st>>>(len, u, beta_out, vnext, nullptr);
+  if (J <= kDcgsMaxJ) {
+    k_dcgs2_sum_coef<<<1, 1024, 0, st>>>(J, gx, part, J > 1 ? beta + (J - 2) : nullptr, coef, alpha + (J - 1));
+  } else {
+    k_reduce_parts<<<2 * J, 256, 0, st>>>(gx, 2 * J, part, sg, 0);
     HIP_TRY(hipGetLastError());
+    k_dcgs2_coef<<<1, 256, 0, st>>>(J, sg, beta, coef, alpha + (J - 1));
   }
+  HIP_TRY(hipGetLastError());
+  // The wide form takes 1,024 dofs a workgroup, so it leaves most CUs idle up to 131,072 dofs (whole step, 64 rows
+  // of 60,000: 39 us wide, 32 narrow; 150,000: 44 wide, 47 narrow) and its second round of workgroups nearly
+  // empty between 262,144 and three times that (300,000: 72 wide, 66 narrow; 900,000: 181 wide, 193 narrow).
+  const bool narrow = len <= 131072 || (len > 262144 && len <= 786432);
+  const int64_t step = narrow ? 64 : 1024;
+  const int64_t uper = ((len + step - 1) / step + kDcgsUpdates - 1) / kDcgsUpdates * step;
+  const int ux = (int)((len + uper - 1) / uper);   // <= kDcgsUpdates
+  if (narrow)
+    k_dcgs2_update<true><<<ux, 256, 0, st>>>(len, uper, J, V, ld, coef, u, npart);
+  else
+    k_dcgs2_update<false><<<ux, 256, 0, st>>>(len, uper, J, V, ld, coef, u, npart);
+  HIP_TRY(hipGetLastError());
+  k_norm_scale<<<vnext ? (unsigned)((len + 1023) / 1024) : 1u, 256, 0, st>>>(len, ux, npart, u, beta_out, vnext);
+  HIP_TRY(hipGetLastError());
   return INCH_OK;
 }
 
@@ -2070,7 +2073,7 @@ inch_status dcgs2_launch(int64_t len, int32_t J, double *V, int64_t ld, double *
 // array's name to a kernel: its device address comes from hipGetSymbolAddress, once per
 // device (with that device current), and is kept per device.
 constexpr int32_t kNoAllocMaxJ = 256;
-constexpr int64_t kNoAllocWords = (int64_t)kRedBlocks * (2 * kNoAllocMaxJ + 1) + 4 * kNoAllocMaxJ;
+constexpr int64_t kNoAllocWords = dcgs2_words(kNoAllocMaxJ);
 static __device__ __align__(256) double scratch[kNoAllocWords];
 
 constexpr int kMaxDevices = 64;
@@ -2132,10 +2135,13 @@ inch_status inch_multidot(int64_t len, int32_t J, const double *V, int64_t ld, c
                           double *work, void *stream) {
   INCH_REQUIRE(len > 0 && J > 0 && V && u && h && work && ld >= len, "inch_multidot: bad args");
   hipStream_t st = (hipStream_t)stream;
-  constexpr int JT = 8;
   const int gx = grid_for(len, 256, kRedBlocks);
-  dim3 grid(gx, (J + JT - 1) / JT);
-  k_multidot_part<JT><<<grid, 256, 0, st>>>(len, J, V, ld, u, work);
+  if (J > 4)
+    k_multidot_part<8><<<dim3(gx, (J + 7) / 8), 256, 0, st>>>(len, J, V, ld, u, work);
+  else if (J > 1)
+    k_multidot_part<4><<<gx, 256, 0, st>>>(len, J, V, ld, u, work);
+  else
+    k_multidot_part<1><<<gx, 256, 0, st>>>(len, J, V, ld, u, work);
   HIP_TRY(hipGetLastError());
   k_reduce_parts<<<J, 256, 0, st>>>(gx, J, work, h, 0);
   HIP_TRY(hipGetLastError());
