@@ -556,7 +556,7 @@ KERNEL_DESC = {"f32": "block SpMV, fp32 values, Chebyshev epilogue",
 
 def kernel_key(kind, A):
     """Template name of the operator kernel the autotuner picked for this matrix."""
-    from inching_amd.autotune import best_config
+    from inching_amd.autotune import BSR_TILE, best_config
     if kind == "mf64rec":
         T = A.tiles()
         return "k_matfree_rec<true>" if T is None else "k_matfree_tile<%d,%d,false>" % T.shape
@@ -570,6 +570,8 @@ def kernel_key(kind, A):
         return "k_matfree_epi<double,%d,%d,%s,%s>" % (c // 10, c % 10, "unsigned short" if f & 1 else "int",
                                                        "true" if f & 2 else "false")
     t = "float" if kind == "f32" else "double"
+    if cfg == BSR_TILE:
+        return "k_bsr_spmv_tile<%s,%s,%d>" % (t, t, cfg - 3000)
     if cfg >= 1200:
         return "k_bsr_spmv<%s,%s,%d,unsigned short,true>" % (t, t, cfg - 1200)
     if cfg >= 200:

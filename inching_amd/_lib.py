@@ -44,6 +44,9 @@ SIGNATURES = {
                                        _vp, _dbl, _vp, _dbl, _vp, _vp, _i32, _vp]),
     "inch_anm_matfree_spmv16": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _dbl, _i32, _vp, _vp, _dbl, _dbl, _vp, _dbl, _vp,
                                           _dbl, _vp, _vp, _i32, _i32, _vp]),
+    "inch_bsr_tiles": (_STATUS, [_i64, _vp, _vp, _i64, _vp, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "inch_bsr_spmv_tile": (_STATUS, [_i64, _i64, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp, _dbl, _dbl,
+                                     _vp, _dbl, _vp, _dbl, _vp, _vp, _i32, _i32, _vp]),
     "inch_bsr_spmv16": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp, _dbl, _dbl, _vp, _dbl, _vp, _dbl,
                                   _vp, _vp, _i32, _i32, _vp]),
     "inch_bsr_col16": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _vp]),

@@ -17,6 +17,10 @@ import torch
 from . import ops
 
 BSR_LANES = (4, 8, 16, 32, 64)
+# Tiles of rows (BlockHessian.bsr_tiles): 153 us against 192 for the best other shape at 150,000
+# atoms in float32 and 96 against 123 at 50,000 in float64; level with it at 700 atoms (6.6 us),
+# where the tie goes to the shapes that need no lists.
+BSR_TILE = 3000 + ops.BsrTiles.LANES
 # Times within NOISE of the fastest count as ties, resolved by a fixed preference order
 # (candidates listed first win), so that the choice does not flip between runs on timing
 # noise: block SpMV shapes with 16-bit columns and XCD-contiguous rows first (the lowest
@@ -115,7 +119,7 @@ def best_config(A, precision, reps=5):
                                reps)
         order = CLUSTER_PREFERENCE + tuple(c for c in codes if c < 4000)
     else:
-        order = BSR_PREFERENCE
+        order = BSR_PREFERENCE + (BSR_TILE,)
         # int32 columns: code = lanes; 16-bit column offsets: code = 200 + lanes
         vals = A.vals(precision)
         for lanes in BSR_LANES:
@@ -128,6 +132,10 @@ def best_config(A, precision, reps=5):
                     times[base + lanes] = _time(lambda: ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, vals, x, y, s1=0.1,
                                                                      c0=1.0, z=z, c2=1.0, acc=acc, mu=0.1, lanes=arg,
                                                                      col16=c16), reps)
+        tiles = A.bsr_tiles()
+        if tiles is not None:
+            times[BSR_TILE] = _time(lambda: ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, vals, x, y, s1=0.1, c0=1.0, z=z,
+                                                         c2=1.0, acc=acc, mu=0.1, lanes=tiles.LANES, col16=tiles), reps)
     best = _pick(times, order)
     _cache[k] = {"best": int(best), "ms": {str(c): round(t, 5) for c, t in times.items()}}
     _save()
@@ -144,9 +152,14 @@ def _pick(times, order):
 
 
 def bsr_launch(A, code):
-    """(lanes argument, col16 or None) of a block-SpMV config code: lanes (int32 columns),
-    200 + lanes (16-bit columns), 1200 + lanes (16-bit columns, XCD-contiguous rows)."""
+    """(lanes argument, col16 argument) of a block-SpMV config code: lanes (int32 columns),
+    200 + lanes (16-bit columns), 1200 + lanes (16-bit columns, XCD-contiguous rows), BSR_TILE
+    (tiles of rows; a matrix of the same class without them takes 1200 + 32, or 32)."""
     code = int(code)
+    if code == BSR_TILE:
+        if A.bsr_tiles() is not None:
+            return A.bsr_tiles().LANES, A.bsr_tiles()
+        return (1032, A.col16()) if A.col16() is not None else (32, None)
     if code >= 1200:
         return code - 1200 + 1000, A.col16()
     if code >= 200:

@@ -41,6 +41,39 @@ __device__ __forceinline__ int64_t xcd_block(bool remap) {
   return xcd * q + (xcd < r ? xcd : r) + idx;   // a bijection of [0, nb)
 }
 
+// y = s1 (w - c0 x) - c2 z (+ the Hotelling term) and acc += mu y at one dof: what it reads, and the rest.
+template <typename MT>
+struct RowTerms {
+  MT x, z, acc;
+  double q;
+  template <typename VT>
+  __device__ __forceinline__ void finish(MT w, int64_t dof, VT *__restrict__ y, MT s1, MT c0, const VT *has_z, MT c2,
+                                         VT *__restrict__ acc_out, MT mu, const double *has_q) const {
+    MT out = w;
+    if (c0 != (MT)0) out -= c0 * x;
+    out *= s1;
+    if (has_z) out -= c2 * z;
+    if (has_q) out += (MT)q;
+    y[dof] = (VT)out;
+    if (acc_out) acc_out[dof] = (VT)(acc + mu * out);
+  }
+};
+
+template <typename MT, typename VT>
+__device__ __forceinline__ RowTerms<MT> row_terms(bool in, int64_t n, int64_t dof, const VT *__restrict__ x, MT c0,
+                                                  const VT *__restrict__ z, const VT *__restrict__ acc,
+                                                  const double *__restrict__ Q, const double *__restrict__ qcoef,
+                                                  int mq) {
+  RowTerms<MT> t{0, 0, 0, 0.0};
+  if (!in) return t;
+  if (c0 != (MT)0) t.x = (MT)x[dof];
+  if (z) t.z = (MT)z[dof];
+  if (acc) t.acc = (MT)acc[dof];
+  if (qcoef)
+    for (int m = 0; m < mq; ++m) t.q += qcoef[m] * Q[m * 3 * n + dof];
+  return t;
+}
+
 template <typename MT, typename VT, int G, typename CT, bool XCD = false>
 __global__ void __launch_bounds__(256) k_bsr_spmv(int64_t n, const int64_t *__restrict__ rowptr,
                                                    const CT *__restrict__ col, const int32_t *__restrict__ rowbase,
@@ -85,20 +118,92 @@ __global__ void __launch_bounds__(256) k_bsr_spmv(int64_t n, const int64_t *__re
   }
   if (lane < 3) {
     const int64_t dof = 3 * row + lane;
-    const MT w = lane == 0 ? a0 : (lane == 1 ? a1 : a2);
-    MT out = w;
-    if (c0 != (MT)0) out -= c0 * (MT)x[dof];
-    out *= s1;
-    if (z) out -= c2 * (MT)z[dof];
-    if (qcoef) {
-      double q = 0.0;
-      const int64_t nd = 3 * n;
-      for (int m = 0; m < mq; ++m) q += qcoef[m] * Q[m * nd + dof];
-      out += (MT)q;
-    }
-    y[dof] = (VT)out;
-    if (acc) acc[dof] = (VT)((MT)acc[dof] + mu * out);
+    row_terms<MT>(true, n, dof, x, c0, z, acc, Q, qcoef, mq)
+        .finish(lane == 0 ? a0 : (lane == 1 ? a1 : a2), dof, y, s1, c0, z, c2, acc, mu, qcoef);
   }
+}
+
+// The product on tiles of rows (inch_bsr_tiles): a workgroup takes a tile of neighbouring atoms, gathers the x
+// entries that its rows meet once into LDS, and the rows read them from there by 16-bit places (as much index
+// traffic as 16-bit columns). What bounded k_bsr_spmv was the gather through L1: 0.8 lines from L2 per block, while
+// the blocks stream through the same L1 (192 us in float32 at 150,000 atoms, 108 with every x entry at the row's
+// own place). A tile of 16 rows meets 300 different entries in 1,870 references. Now 153 us (0.67 GB, 4.4 TB/s),
+// and 96 against 123 in float64 at 50,000 atoms (0.42 GB). What is left above the stream: rows of a tile lie
+// apart in memory (rows one after the other took 131 and 79), and the gather (10 and 3). Tiles of 8, 32 and 64
+// rows took 158, 155 and 163; tiles of consecutive rows share few entries (1,745 per 16 rows) and took 179.
+// G lanes per row; U blocks per lane at a time, all of their loads in flight, the first ones while x is gathered
+// (U = 4 takes 162 and 108: fewer waves).
+template <typename MT, typename VT, int G>
+__global__ void __launch_bounds__(512) k_bsr_spmv_tile(int64_t n, const int4 *__restrict__ slots, int ustride,
+                                                        const int32_t *__restrict__ ulen,
+                                                        const int32_t *__restrict__ ulist,
+                                                        const uint16_t *__restrict__ uidx,
+                                                        const MT *__restrict__ vals, const VT *__restrict__ x,
+                                                        VT *__restrict__ y, MT s1, MT c0, const VT *__restrict__ z,
+                                                        MT c2, VT *__restrict__ acc, MT mu,
+                                                        const double *__restrict__ Q,
+                                                        const double *__restrict__ qcoef, int mq) {
+  constexpr int U = 2;
+  extern __shared__ __align__(16) char tile_x[];
+  MT *xs = (MT *)tile_x;
+  const int64_t t = xcd_block(true);
+  const int lane = threadIdx.x & (G - 1), tile = blockDim.x / G;
+  const int4 slot = slots[t * tile + threadIdx.x / G];
+  const int len = ulen[t];
+  const int32_t *ul = ulist + t * ustride;
+  const int64_t b0 = (int64_t)(((uint64_t)(uint32_t)slot.w << 32) | (uint32_t)slot.z);
+  const int nb = slot.y;                                     // blocks of the row
+  // places past the row's end repeat its last block and are dropped
+  uint16_t c[U];
+  MT h[U][9];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int q = k0 + k * G < nb ? k0 + k * G : nb - 1;
+      const int64_t b = b0 + (q > 0 ? q : 0);
+      c[k] = uidx[b];
+#pragma unroll
+      for (int f = 0; f < 9; ++f) h[k][f] = vals[9 * b + f];
+    }
+  };
+  load(lane);
+  const int64_t dof = 3 * (int64_t)slot.x + lane;
+  const bool mine = slot.x >= 0 && lane < 3;
+  const RowTerms<MT> terms = row_terms<MT>(mine, n, dof, x, c0, z, acc, Q, qcoef, mq);
+  for (int i = threadIdx.x; i < ustride; i += blockDim.x) {
+    const int64_t j = ul[i];
+    if (i < len) {
+      const VT *xj = x + 3 * j;
+      xs[3 * i] = (MT)xj[0];
+      xs[3 * i + 1] = (MT)xj[1];
+      xs[3 * i + 2] = (MT)xj[2];
+    }
+  }
+  __syncthreads();
+  MT a0 = 0, a1 = 0, a2 = 0;
+  for (int k0 = lane;;) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const MT x0 = xs[3 * c[k]], x1 = xs[3 * c[k] + 1], x2 = xs[3 * c[k] + 2];
+      const MT w0 = a0 + (h[k][0] * x0 + h[k][1] * x1 + h[k][2] * x2);
+      const MT w1 = a1 + (h[k][3] * x0 + h[k][4] * x1 + h[k][5] * x2);
+      const MT w2 = a2 + (h[k][6] * x0 + h[k][7] * x1 + h[k][8] * x2);
+      const bool in = k0 + k * G < nb;
+      a0 = in ? w0 : a0;
+      a1 = in ? w1 : a1;
+      a2 = in ? w2 : a2;
+    }
+    k0 += U * G;
+    if (k0 - lane >= nb) break;
+    load(k0);
+  }
+#pragma unroll
+  for (int off = G / 2; off > 0; off >>= 1) {
+    a0 += __shfl_xor(a0, off, G);
+    a1 += __shfl_xor(a1, off, G);
+    a2 += __shfl_xor(a2, off, G);
+  }
+  if (mine) terms.finish(lane == 0 ? a0 : (lane == 1 ? a1 : a2), dof, y, s1, c0, z, c2, acc, mu, qcoef);
 }
 
 template <typename MT, typename VT, int G, int R>
@@ -1667,6 +1772,48 @@ inch_status inch_bsr_spmv(int64_t n, const int64_t *rowptr, const int32_t *col, 
   if (mdt == INCH_F64 && vdt == INCH_F64)
     return launch_spmv<double, double>(n, rowptr, col, nb, vals, x, y, s1, c0, z, c2, acc, mu, Q, qcoef, m_q, G, st);
   INCH_FAIL(INCH_ERR_INVALID, "inch_bsr_spmv: unsupported dtype pair (%d,%d)", mdt, vdt);
+}
+
+inch_status inch_bsr_spmv_tile(int64_t n, int64_t ntile, int32_t tile, const int32_t *slots, int32_t ustride,
+                               const int32_t *ulen, const int32_t *ulist, const uint16_t *uidx, const void *vals,
+                               int32_t mdt, int32_t vdt, const void *x, void *y, double s1, double c0, const void *z,
+                               double c2, void *acc, double mu, const double *Q, const double *qcoef, int32_t m_q,
+                               int32_t lanes, void *stream) {
+  INCH_REQUIRE(n > 0 && ntile > 0 && ntile <= n && slots && ulen && ulist && uidx && vals && x && y,
+               "inch_bsr_spmv_tile: bad args");
+  INCH_REQUIRE(!qcoef || (Q && m_q > 0), "inch_bsr_spmv_tile: qcoef needs Q and m_q > 0");
+  INCH_REQUIRE(x != y, "inch_bsr_spmv_tile: x and y must not alias");
+  INCH_REQUIRE(tile > 0 && lanes > 0 && tile <= 512 / lanes && tile * lanes % 64 == 0 && ustride > 0,
+               "inch_bsr_spmv_tile: bad tile");
+  const size_t lds = 3 * (size_t)ustride * (mdt == INCH_F64 ? 8 : 4);
+  INCH_REQUIRE(lds <= 65536, "inch_bsr_spmv_tile: the union exceeds the LDS");
+  hipStream_t st = (hipStream_t)stream;
+#define INCH_TILE_CASE(MT, VT, G)                                                                                      \
+  case G:                                                                                                              \
+    k_bsr_spmv_tile<MT, VT, G><<<(unsigned)ntile, tile * G, lds, st>>>(                                                \
+        n, (const int4 *)slots, ustride, ulen, ulist, uidx, (const MT *)vals, (const VT *)x, (VT *)y, (MT)s1, (MT)c0,  \
+        (const VT *)z, (MT)c2, (VT *)acc, (MT)mu, Q, qcoef, m_q);                                                      \
+    break;
+#define INCH_TILE_TYPES(MT, VT)                                                                                        \
+  switch (lanes) {                                                                                                     \
+    INCH_TILE_CASE(MT, VT, 8)                                                                                          \
+    INCH_TILE_CASE(MT, VT, 16)                                                                                         \
+    INCH_TILE_CASE(MT, VT, 32)                                                                                         \
+    default: INCH_FAIL(INCH_ERR_INVALID, "inch_bsr_spmv_tile: lanes must be 8, 16 or 32 (got %d)", lanes);             \
+  }
+  if (mdt == INCH_F32 && vdt == INCH_F32) {
+    INCH_TILE_TYPES(float, float)
+  } else if (mdt == INCH_F32 && vdt == INCH_F64) {
+    INCH_TILE_TYPES(float, double)
+  } else if (mdt == INCH_F64 && vdt == INCH_F64) {
+    INCH_TILE_TYPES(double, double)
+  } else {
+    INCH_FAIL(INCH_ERR_INVALID, "inch_bsr_spmv_tile: unsupported dtype pair (%d,%d)", mdt, vdt);
+  }
+#undef INCH_TILE_TYPES
+#undef INCH_TILE_CASE
+  HIP_TRY(hipGetLastError());
+  return INCH_OK;
 }
 
 inch_status inch_bsr_spmv16(int64_t n, const int64_t *rowptr, const int32_t *rowbase, const uint16_t *col16,

@@ -164,6 +164,17 @@ class BlockHessian:
                         break
         return self._tiles
 
+    def bsr_tiles(self):
+        """Tiles of rows for the stored-block product (ops.BsrTiles; built once, immutable), or None
+        when a tile's columns are too many or too far apart."""
+        if "_bsr_tiles" not in self.__dict__:
+            side = self.rc * (ops.BsrTiles.TILE * 4.0 * np.pi / 3.0 / max(1.0, self.nnzb / self.n_atoms)) ** (1.0 / 3.0)
+            try:
+                self._bsr_tiles = ops.BsrTiles(self.xyz, self.rowptr, self.col, side)
+            except (ops.InchingError, torch.OutOfMemoryError):
+                self._bsr_tiles = None
+        return self._bsr_tiles
+
     def slot_form(self):
         """The form of the matrix-free operator that keeps a recurrence's vectors in slot order
         next to the coordinates: the tile form, or where that does not fit the record form, or

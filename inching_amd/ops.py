@@ -435,10 +435,43 @@ def matfree_cl(xyz, clusters, plus_i, x, y, s1=1.0, c0=0.0, z=None, c2=0.0, acc=
          float(s1), float(c0), P(z), float(c2), P(acc), float(mu), P(Q), P(qcoef), mq, int(config), stream_ptr(stream))
 
 
+class BsrTiles:
+    """Tiles of rows for the stored-block product (inch_bsr_tiles): neighbouring atoms' rows share
+    the x entries that they meet. ``side``: the cube of a tile's atoms. Raises InchingError
+    (INCH_ERR_CAPACITY) when a tile's columns are too many or too far apart."""
+
+    TILE, LANES = 16, 32    # rows per tile, lanes per row
+
+    def __init__(self, xyz, rowptr, col, side, stream=None):
+        require_gpu()
+        _check_dev(xyz, rowptr, col)
+        n, dev, tile = xyz.shape[0], xyz.device, self.TILE
+        if rowptr.numel() != n + 1:
+            raise ValueError("rowptr inconsistent with the coordinates")
+        i32 = dict(dtype=torch.int32, device=dev)
+        self.n, self.nnz = n, col.numel()
+        order, start = torch.empty(n, **i32), torch.empty(n + 1, **i32)
+        nt, umax = C.c_int64(0), C.c_int32(0)
+        call("inch_anm_tile_order", n, P(xyz), float(side), tile, P(order), P(start), C.byref(nt), stream_ptr(stream))
+        self.ntile = nt.value
+        self.ulen = torch.empty(self.ntile, **i32)
+        head = (n, P(rowptr), P(col), self.ntile, P(order), P(start), tile)
+        call("inch_bsr_tiles", *head, 0, None, P(self.ulen), None, None, C.byref(umax), stream_ptr(stream))
+        self.stride = max(1, umax.value)
+        if 24 * self.stride > 65536:
+            raise InchingError("inch_bsr_tiles", -3, "a tile's x entries exceed the LDS")
+        self.slots = torch.empty(4 * self.ntile * tile, **i32)
+        self.ulist = torch.empty(self.ntile * self.stride, **i32)
+        self.uidx = torch.empty(max(1, self.nnz), dtype=torch.int16, device=dev)
+        call("inch_bsr_tiles", *head, self.stride, P(self.slots), P(self.ulen), P(self.ulist), P(self.uidx), None,
+             stream_ptr(stream))
+
+
 def bsr_spmv(n_atoms, rowptr, col, vals, x, y, s1=1.0, c0=0.0, z=None, c2=0.0, acc=None, mu=0.0, Q=None,
              qcoef=None, lanes=16, stream=None, col16=None):
     """y = s1 (A x - c0 x) - c2 z (+ sum_m qcoef[m] Q[m]); acc += mu y (all terms optional).
-    ``col16`` = (rowbase, col16) selects the 16-bit column-offset kernel (col is then unused)."""
+    ``col16`` = (rowbase, col16) selects the 16-bit column-offset kernel (col is then unused), a
+    BsrTiles the product on tiles of rows."""
     nd = 3 * n_atoms
     for t in (x, y, z, acc):
         if t is not None and t.numel() != nd:
@@ -456,6 +489,14 @@ def bsr_spmv(n_atoms, rowptr, col, vals, x, y, s1=1.0, c0=0.0, z=None, c2=0.0, a
         mq = Q.shape[0]
         if qcoef.numel() < mq:
             raise ValueError("qcoef too short")
+    if isinstance(col16, BsrTiles):
+        t = col16
+        if t.n != n_atoms or t.nnz != col.numel():
+            raise ValueError("tiles of another matrix")
+        call("inch_bsr_spmv_tile", n_atoms, t.ntile, t.TILE, P(t.slots), t.stride, P(t.ulen), P(t.ulist), P(t.uidx),
+             P(vals), dt(vals), vd, P(x), P(y), float(s1), float(c0), P(z), float(c2), P(acc), float(mu), P(Q),
+             P(qcoef), mq, int(lanes), stream_ptr(stream))
+        return
     if col16 is not None:
         call("inch_bsr_spmv16", n_atoms, P(rowptr), P(col16[0]), P(col16[1]), P(vals), dt(vals), vd, P(x), P(y),
              float(s1), float(c0), P(z), float(c2), P(acc), float(mu), P(Q), P(qcoef), mq, int(lanes),

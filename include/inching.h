@@ -213,6 +213,22 @@ inch_status inch_bsr_spmv16(int64_t n, const int64_t *rowptr, const int32_t *row
                             const void *vals, int32_t mdt, int32_t vdt, const void *x, void *y, double s1, double c0,
                             const void *z, double c2, void *acc, double mu, const double *Q, const double *qcoef,
                             int32_t m_q, int32_t lanes_per_row, void *stream);
+/* The same product on tiles of rows (no reference counterpart as a layout): order and tile_start as
+ * inch_anm_tile_order writes them (at most `tile` rows each). inch_bsr_tiles lists the columns of every tile's
+ * rows, each once and ascending: with ulist NULL it writes ulen [ntile] and *umax_out, the longest list (syncs;
+ * INCH_ERR_CAPACITY when a tile's columns span more than 262,144 or a list exceeds 65,536); with ulist
+ * [ntile * ustride], ustride >= *umax_out, it writes the lists, uidx [nnz], the place of col[b] in its tile's list,
+ * and slots [4 * ntile * tile] (16-byte aligned): per place of a tile its row (-1: none), the row's length and first
+ * block. inch_bsr_spmv_tile: other arguments as inch_bsr_spmv; lanes 8, 16 or 32 per row, tile * lanes a multiple
+ * of 64 up to 512; three values per list entry must fit 64 KiB (ustride of them). */
+inch_status inch_bsr_tiles(int64_t n, const int64_t *rowptr, const int32_t *col, int64_t ntile, const int32_t *order,
+                           const int32_t *tile_start, int32_t tile, int32_t ustride, int32_t *slots, int32_t *ulen,
+                           int32_t *ulist, uint16_t *uidx, int32_t *umax_out, void *stream);
+inch_status inch_bsr_spmv_tile(int64_t n, int64_t ntile, int32_t tile, const int32_t *slots, int32_t ustride,
+                               const int32_t *ulen, const int32_t *ulist, const uint16_t *uidx, const void *vals,
+                               int32_t mdt, int32_t vdt, const void *x, void *y, double s1, double c0, const void *z,
+                               double c2, void *acc, double mu, const double *Q, const double *qcoef, int32_t m_q,
+                               int32_t lanes, void *stream);
 inch_status inch_bsr_col16(int64_t n, const int64_t *rowptr, const int32_t *col, int32_t *rowbase,
                            uint16_t *col16, void *stream);
 
