@@ -107,6 +107,10 @@ SIGNATURES = {
                                      _vp]),
     "inch_gnn_aggregate": (_STATUS, [_i64, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp]),
     "inch_gnn_relu_bwd": (_STATUS, [_i64, _vp, _vp, _vp, _vp]),
+    "inch_shift_apply": (_STATUS, [_i64, _i32, _vp, _i64, _vp, _dbl, _i64, _vp, _vp, _vp, _vp, _vp]),
+    "inch_lanczos3_work_size": (_i64, []),
+    "inch_lanczos3_scale": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "inch_lanczos3_update": (_STATUS, [_i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "inch_rr_combine": (_STATUS, [_i64, _i32, _i32, _vp, _i64, _vp, _vp, _i64, _vp]),
     "inch_rr_project": (_STATUS, [_i64, _i32, _i32, _vp, _i64, _vp, _vp, _i64, _vp]),
     "inch_sqfluct": (_STATUS, [_i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),

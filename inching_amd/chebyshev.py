@@ -510,9 +510,8 @@ def spectrum_bound(A, n_tridiag=300, seed=0, precision="f64", stop_rel=None, inf
     v0 = torch.empty_like(v)
     alpha = torch.zeros(n_tridiag + 1, dtype=torch.float64, device=dev)
     beta = torch.zeros(n_tridiag, dtype=torch.float64, device=dev)
-    ws = ops.Workspace(1, dev)
+    step = ops.Lanczos3(dev)
     vals = A.vals(precision) if precision != "mf64" else None
-    row = v.view(1, -1)
 
     from .autotune import best_config, bsr_launch
     cfg = best_config(A, precision) if rec is None else 0
@@ -520,27 +519,25 @@ def spectrum_bound(A, n_tridiag=300, seed=0, precision="f64", stop_rel=None, inf
 
     def av(x, y):
         if rec is not None:
-            ops.rec_pack(None, x, buf, ncl=rec.slots // ops.CLUSTER_ATOMS)
-            rec.product(buf, None, None, A.plus_i, y=y)
+            rec.product(buf, None, None, A.plus_i, y=y)      # buf holds x
         elif vals is None:
             A.matfree_spmv(x, y, config=cfg)
         else:
             ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, vals, x, y, lanes=blanes, col16=c16)
 
+    if rec is not None:
+        ops.rec_pack(None, v, buf, ncl=rec.slots // ops.CLUSTER_ATOMS)
+    else:
+        buf = None
     av(v, f)
-    ops.multidot(row, 1, f, alpha[0:1], ws)
-    ops.axpy_dev(alpha[0:1], -1.0, v, f)
+    step.update(v, f, alpha[0:1])
     m = n_tridiag + 1            # size of the tridiagonal matrix built
     prev = None
     for i in range(n_tridiag):
-        ops.gemv_update(row, 0, None, f, 0.0, nrm2_out=beta[i:i + 1], ws=ws)   # beta_i = ||f||
         v0, v = v, v0            # the previous vector is kept by swapping buffers
-        ops.scale_div(f, beta[i:i + 1], v)
-        row = v.view(1, -1)
+        step.scale(f, beta[i:i + 1], v, rec=buf)             # beta_i = ||f||
         av(v, f)
-        ops.axpy_dev(beta[i:i + 1], -1.0, v0, f)
-        ops.multidot(row, 1, f, alpha[i + 1:i + 2], ws)
-        ops.axpy_dev(alpha[i + 1:i + 2], -1.0, v, f)
+        step.update(v, f, alpha[i + 1:i + 2], v_prev=v0, beta=beta[i:i + 1])
         if stop_rel is not None and (i + 1) % BOUND_CHECK_EVERY == 0 and i + 1 < n_tridiag:
             mm = i + 2
             top = float(np.linalg.eigvalsh(_tridiag(alpha[:mm].cpu().numpy(), beta[:mm - 1].cpu().numpy()))[-1])

@@ -1572,12 +1572,95 @@ __global__ void __launch_bounds__(256) k_dcgs2_update(int64_t len, int64_t per, 
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 
+// Sum of part[p J + j] over p < nparts in all threads' hs[j] (j < J <= 16, times scale): 16 threads per j over
+// every 16th partial, then in order. red[256], hs[16].
+__device__ __forceinline__ void sum_few(int nparts, int J, const double *__restrict__ part, double scale, double *red,
+                                        double *hs) {
+  const int tid = threadIdx.x, o = tid & 15;
+  double s = 0.0;
+  if (o < J)
+#pragma unroll 4
+    for (int p = tid >> 4; p < nparts; p += 16) s += part[(int64_t)p * J + o];
+  red[tid] = s;
+  __syncthreads();
+  if (tid < J) {
+    for (int q = 1; q < 16; ++q) s += red[16 * q + tid];
+    hs[tid] = s * scale;
+  }
+  __syncthreads();
+}
+
+// u -= scale V^T h for the J <= 16 sums h of `part`, in the launch that forms these sums (every block alike) and, with
+// `atoms`, unpacks acc (slot order) into u first. The operator's Hotelling term: with 6 rows of 18,021 dofs a sum of
+// partials, an update and an unpacking took 8.3 us and the gaps between them, now 4.5 (latency).
+__global__ void __launch_bounds__(256) k_shift(int64_t count, int J, int nparts, const double *__restrict__ part,
+                                               double scale, const double *__restrict__ V, int64_t ld,
+                                               const int32_t *__restrict__ atoms, const double *__restrict__ acc,
+                                               double *__restrict__ u) {
+  __shared__ double red[256], hs[16];
+  sum_few(nparts, J, part, scale, red, hs);
+  for (int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x; t < count; t += (int64_t)gridDim.x * 256) {
+    int64_t i = t;
+    if (atoms) {
+      const int32_t at = atoms[t / 3];
+      if (at < 0) continue;
+      i = 3 * (int64_t)at + t % 3;
+    }
+    const double x = atoms ? acc[t] : u[i];
+    double s = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < J; ++j) s += V[(int64_t)j * ld + i] * hs[j];
+    u[i] = x - s;
+  }
+}
+
+// Three-term Lanczos step without re-orthogonalisation, f = Op v: f -= beta v_prev (v_prev may be null) and
+// part[block] = v . f; then *alpha = v . f, f -= alpha v and part_sq[block] = |f|^2. With k_norm_scale before the
+// product (beta = |f|, v = f / beta, and v into the records) a step is three launches and the product, where it was
+// eight: 61 steps over 18,021 dofs with
+// their products took 3.5 ms, now 2.1.
+__global__ void __launch_bounds__(256) k_lanczos3_dot(int64_t len, const double *__restrict__ beta,
+                                                      const double *__restrict__ v_prev, const double *__restrict__ v,
+                                                      double *__restrict__ f, double *__restrict__ part) {
+  __shared__ double red[4];
+  const double b = v_prev ? beta[0] : 0.0;
+  double s = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < len; i += (int64_t)gridDim.x * 256) {
+    double x = f[i];
+    if (v_prev) {
+      x -= b * v_prev[i];
+      f[i] = x;
+    }
+    s += v[i] * x;
+  }
+  const double tot = dcgs2::block_sum(s, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = tot;
+}
+
+__global__ void __launch_bounds__(256) k_lanczos3_update(int64_t len, const double *__restrict__ part,
+                                                         const double *__restrict__ v, double *__restrict__ f,
+                                                         double *__restrict__ alpha, double *__restrict__ part_sq) {
+  __shared__ double red[4];
+  double s = 0.0;
+  for (int p = threadIdx.x; p < (int)gridDim.x; p += 256) s += part[p];
+  const double a = dcgs2::block_sum(s, red);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *alpha = a;
+  double ss = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < len; i += (int64_t)gridDim.x * 256) {
+    const double x = f[i] - a * v[i];
+    f[i] = x;
+    ss += x * x;
+  }
+  const double tot = dcgs2::block_sum(ss, red);
+  if (threadIdx.x == 0) part_sq[blockIdx.x] = tot;
+}
+
 // *norm = sqrt of the sum of part[0 .. nparts), which every block forms alike, and (given vnext)
-// vnext = u / *norm, 1,024 dofs a block. Latency bounds it: 3.3 us for 18,021 dofs, a sum and a scaling kernel
+// vnext = u / *norm, 1,024 dofs a block, also as the vector part of the records rec (slot order) when given. Latency bounds it: 3.3 us for 18,021 dofs, a sum and a scaling kernel
 // took 4.9 and the gap between them.
 __global__ void __launch_bounds__(256) k_norm_scale(int64_t len, int nparts, const double *__restrict__ part,
                                                     const double *__restrict__ u, double *__restrict__ norm,
-                                                    double *__restrict__ vnext) {
+                                                    double *__restrict__ vnext, double *__restrict__ rec) {
   __shared__ double red[4];
   const int64_t i0 = blockIdx.x * (int64_t)1024 + threadIdx.x;
   double x[4], s = 0.0;
@@ -1590,7 +1673,11 @@ __global__ void __launch_bounds__(256) k_norm_scale(int64_t len, int nparts, con
   const double inv = 1.0 / nrm;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
-    if (i0 + 256 * t < len) vnext[i0 + 256 * t] = x[t] * inv;
+    if (i0 + 256 * t < len) {
+      const int64_t i = i0 + 256 * t;
+      vnext[i] = x[t] * inv;
+      if (rec) rec[6 * (i / 3) + 3 + i % 3] = x[t] * inv;
+    }
 }
 
 int grid_for(int64_t len, int bs, int cap) {
@@ -2210,7 +2297,8 @@ inch_status dcgs2_launch(int64_t len, int32_t J, double *V, int64_t ld, double *
   else
     k_dcgs2_update<false><<<ux, 256, 0, st>>>(len, uper, J, V, ld, coef, u, npart);
   HIP_TRY(hipGetLastError());
-  k_norm_scale<<<vnext ? (unsigned)((len + 1023) / 1024) : 1u, 256, 0, st>>>(len, ux, npart, u, beta_out, vnext);
+  k_norm_scale<<<vnext ? (unsigned)((len + 1023) / 1024) : 1u, 256, 0, st>>>(len, ux, npart, u, beta_out, vnext,
+                                                                             nullptr);
   HIP_TRY(hipGetLastError());
   return INCH_OK;
 }
@@ -2291,6 +2379,48 @@ inch_status inch_multidot(int64_t len, int32_t J, const double *V, int64_t ld, c
     k_multidot_part<1><<<gx, 256, 0, st>>>(len, J, V, ld, u, work);
   HIP_TRY(hipGetLastError());
   k_reduce_parts<<<J, 256, 0, st>>>(gx, J, work, h, 0);
+  HIP_TRY(hipGetLastError());
+  return INCH_OK;
+}
+
+inch_status inch_shift_apply(int64_t len, int32_t m, const double *Q, int64_t ld, const double *v, double scale,
+                             int64_t slots, const int32_t *atoms, const double *acc, double *u, double *work,
+                             void *stream) {
+  INCH_REQUIRE(len > 0 && m > 0 && m <= 16 && Q && v && u && u != v && work && ld >= len, "inch_shift_apply: bad args (0 < m <= 16)");
+  INCH_REQUIRE(!atoms || (acc && slots > 0), "inch_shift_apply: atoms need acc and slots");
+  hipStream_t st = (hipStream_t)stream;
+  const int gx = grid_for(len, 256, kRedBlocks);
+  if (m > 4)
+    k_multidot_part<8><<<dim3(gx, (m + 7) / 8), 256, 0, st>>>(len, m, Q, ld, v, work);
+  else
+    k_multidot_part<4><<<gx, 256, 0, st>>>(len, m, Q, ld, v, work);
+  HIP_TRY(hipGetLastError());
+  const int64_t count = atoms ? 3 * slots : len;
+  k_shift<<<grid_for(count, 256, 2048), 256, 0, st>>>(count, m, gx, work, scale, Q, ld, atoms, acc, u);
+  HIP_TRY(hipGetLastError());
+  return INCH_OK;
+}
+
+int64_t inch_lanczos3_work_size(void) { return 2 * kRedBlocks; }
+
+inch_status inch_lanczos3_scale(int64_t len, const double *f, double *beta, double *v, double *rec, const double *work,
+                                void *stream) {
+  INCH_REQUIRE(len > 0 && f && beta && v && work && (!rec || len % 3 == 0), "inch_lanczos3_scale: bad args");
+  const int gx = grid_for(len, 256, kRedBlocks);
+  k_norm_scale<<<(unsigned)((len + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(len, gx, work + kRedBlocks, f, beta, v,
+                                                                               rec);
+  HIP_TRY(hipGetLastError());
+  return INCH_OK;
+}
+
+inch_status inch_lanczos3_update(int64_t len, const double *beta, const double *v_prev, const double *v, double *f,
+                                 double *alpha, double *work, void *stream) {
+  INCH_REQUIRE(len > 0 && v && f && alpha && work && (!v_prev || beta), "inch_lanczos3_update: bad args");
+  hipStream_t st = (hipStream_t)stream;
+  const int gx = grid_for(len, 256, kRedBlocks);
+  k_lanczos3_dot<<<gx, 256, 0, st>>>(len, beta, v_prev, v, f, work);
+  HIP_TRY(hipGetLastError());
+  k_lanczos3_update<<<gx, 256, 0, st>>>(len, work, v, f, alpha, work + kRedBlocks);
   HIP_TRY(hipGetLastError());
   return INCH_OK;
 }

@@ -108,10 +108,11 @@ class Operator:
             self.timer.append((self.precision, epi, e0, e1, 1))
         self.n_spmv += 1
 
-    def _filtered_records(self, v64, u64):
+    def _filtered_records(self, v64, u64, shift=False):
         """u = sum_k mu_k T_k((A - cc)/dd) v with the recurrence on records: v packed into
         slot order, three record buffers in turn (T_k, T_{k-1} read, T_{k+1} written),
-        the accumulator in slot order unpacked into u at the end."""
+        the accumulator in slot order unpacked into u at the end (``shift``: with the Hotelling
+        term added in the same launch)."""
         pol, form, acc = self.pol, self.rec, self._acc_rec
         ops.rec_pack(form.atoms, v64, self._recs[0], acc, self.mu[0])
         if self.timer is not None:
@@ -122,8 +123,15 @@ class Operator:
         if self.timer is not None:
             e1.record()
             self.timer.append(("mf64rec", "cheb", e0, e1, self.degree))
-        ops.rec_unpack(form.atoms, acc, u64)
+        if shift:
+            ops.shift_apply(self.Q, v64, -self.shift, u64, self._ws, atoms=form.atoms, acc=acc)
+        else:
+            ops.rec_unpack(form.atoms, acc, u64)
         self.n_spmv += self.degree
+
+    def _on_records(self, v64, u64):
+        return (self.rec is not None and v64.dtype == torch.float64 and u64.dtype == torch.float64
+                and v64.is_contiguous() and u64.is_contiguous())
 
     def filtered(self, v64, u64):
         """u = sum_k mu_k T_k((A - cc)/dd) v.
@@ -131,8 +139,7 @@ class Operator:
         With a float64 operator the recurrence starts from v itself (it is only read) and,
         when u does not share v's memory, accumulates straight into u; otherwise v is
         converted into a scratch vector and the accumulator is converted into u at the end."""
-        if (self.rec is not None and v64.dtype == torch.float64 and u64.dtype == torch.float64
-                and v64.is_contiguous() and u64.is_contiguous()):
+        if self._on_records(v64, u64):
             self._filtered_records(v64, u64)
             return
         pol = self.pol
@@ -172,11 +179,20 @@ class Operator:
 
     def apply(self, v64, u64):
         self.n_apply += 1
+        # a few rows Q (the six rigid motions) and a result of its own: the Hotelling term in two launches
+        few = (self.Q is not None and self.shift != 0.0 and self.Q.shape[0] <= ops.SHIFT_MAX_M
+               and v64.dtype == torch.float64 and u64.dtype == torch.float64 and v64.is_contiguous()
+               and u64.is_contiguous() and v64.data_ptr() != u64.data_ptr())
+        if few and self.pol is not None and self._on_records(v64, u64):
+            self._filtered_records(v64, u64, shift=True)
+            return u64
         if self.pol is None:
             self.spmv(v64, u64)
         else:
             self.filtered(v64, u64)
-        if self.Q is not None and self.shift != 0.0:
+        if few:
+            ops.shift_apply(self.Q, v64, -self.shift, u64, self._ws)
+        elif self.Q is not None and self.shift != 0.0:
             m = self.Q.shape[0]
             ops.multidot(self.Q, m, v64, self._h, self._ws)
             ops.gemv_update(self.Q, m, self._h, u64, scale=-self.shift)

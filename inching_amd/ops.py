@@ -586,6 +586,41 @@ def multidot(V, J, u, h, ws, stream=None):
     call("inch_multidot", u.numel(), int(J), P(V), V.stride(0), P(u), P(h), P(ws.buf), stream_ptr(stream))
 
 
+# Most rows of inch_shift_apply: every workgroup sums all partials itself (16 x 512 at most); locked blocks of
+# vectors take a sum kernel and an update instead.
+SHIFT_MAX_M = 16
+
+
+def shift_apply(Q, v, scale, u, ws, atoms=None, acc=None, stream=None):
+    """u -= scale Q^T (Q v) for at most SHIFT_MAX_M rows Q; with ``atoms``, u is first unpacked
+    from acc (slot order)."""
+    if Q.shape[0] > ws.J or Q.shape[0] > SHIFT_MAX_M:
+        raise ValueError("shift_apply: too many rows for the workspace or the kernel")
+    if Q.shape[1] != v.numel() or u.numel() != v.numel():
+        raise ValueError("shape mismatch in shift_apply")
+    slots = 0 if atoms is None else atoms.numel()
+    call("inch_shift_apply", v.numel(), Q.shape[0], P(Q), Q.stride(0), P(v), float(scale), slots, P(atoms), P(acc), P(u),
+         P(ws.buf), stream_ptr(stream))
+
+
+class Lanczos3:
+    """Steps of a Lanczos run without re-orthogonalisation around the caller's products f = Op v
+    (inch_lanczos3_update / _scale)."""
+
+    def __init__(self, device):
+        from ._lib import lib
+        self.work = torch.empty(int(lib().inch_lanczos3_work_size()), dtype=torch.float64, device=device)
+
+    def update(self, v, f, alpha, v_prev=None, beta=None, stream=None):
+        """f -= beta v_prev; alpha = v . f; f -= alpha v."""
+        call("inch_lanczos3_update", f.numel(), P(beta), P(v_prev), P(v), P(f), P(alpha), P(self.work),
+             stream_ptr(stream))
+
+    def scale(self, f, beta, v, rec=None, stream=None):
+        """beta = |f| (of the last update), v = f / beta, also into the records' vector part."""
+        call("inch_lanczos3_scale", f.numel(), P(f), P(beta), P(v), P(rec), P(self.work), stream_ptr(stream))
+
+
 def gemv_update(V, J, h, u, scale=1.0, nrm2_out=None, ws=None, stream=None):
     """u -= scale * V[:J]^T h[:J]; optionally nrm2_out[0] = ||u||."""
     if J > 0 and (V.shape[0] < J or V.shape[1] != u.numel() or h.numel() < J):

@@ -428,6 +428,22 @@ inch_status inch_dcgs2_step(int64_t len, int32_t J, double *V, int64_t ld, doubl
 inch_status inch_dcgs2_step_noalloc(int64_t len, int32_t J, double *V, int64_t ld, double *u, double *alpha,
                                     const double *beta, double *beta_out, double *vnext, void *stream);
 
+/* u -= scale Q^T (Q v) for 0 < m <= 16 rows Q (the Hotelling term, Burn/Orthogonalization/T3.py:62-164) in two
+ * launches; with atoms, u = the unpacked acc (slot order, as inch_rec_unpack with `slots` places) first. u must not
+ * be v. work: inch_multidot_work_size(m) doubles. */
+inch_status inch_shift_apply(int64_t len, int32_t m, const double *Q, int64_t ld, const double *v, double scale,
+                             int64_t slots, const int32_t *atoms, const double *acc, double *u, double *work,
+                             void *stream);
+/* Lanczos step without re-orthogonalisation (Burn/HermitianLanczos/T2.py:30-100) around a product f = Op v.
+ * inch_lanczos3_update: f -= *beta v_prev (v_prev NULL: not), *alpha = v . f, f -= *alpha v, and keeps the parts of
+ * |f|^2 in work (inch_lanczos3_work_size doubles). inch_lanczos3_scale: *beta = |f| from these, v = f / *beta, and
+ * with rec the vector part of its len / 3 records (slot order) is v too. */
+int64_t inch_lanczos3_work_size(void);
+inch_status inch_lanczos3_scale(int64_t len, const double *f, double *beta, double *v, double *rec, const double *work,
+                                void *stream);
+inch_status inch_lanczos3_update(int64_t len, const double *beta, const double *v_prev, const double *v, double *f,
+                                 double *alpha, double *work, void *stream);
+
 /* out[q*ld_out + i] = sum_r W[r*k + q] * V[r*ld + i]  for q < k, r < m
  * (W float64 [m, k] row-major on device; out must not alias V). FP64 MFMA 16x16x4. */
 inch_status inch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld,
