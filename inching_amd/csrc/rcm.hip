@@ -11,9 +11,8 @@
 //   claim   : claim[j] = min position of a level-L neighbour           (atomicMin)
 //   count   : cnt[p]   = number of nodes claimed by the node at position p
 //   scan    : off      = exclusive prefix sum of cnt
-//   scatter : children written into their parent's slot range
-//   sort    : each group sorted by (degree, -index) (one wave per parent, rank by key)
-//   place   : pos[node] = its position
+//   scatter : the children's keys (degree, -index) written into their parent's slot range
+//   place   : each child at its key's rank in its group
 // The level's bounds stay on the device: the kernels of kRounds levels are launched at a time,
 // each over a fixed grid that reads the bounds, and the host looks at them once per batch (a
 // level past the last one finds no nodes and does nothing).
@@ -43,12 +42,9 @@ namespace {
 
 constexpr int kG = 32;  // lanes per level node in the neighbour scans
 
-__global__ void k_rcm_init(int64_t n, int32_t *__restrict__ pos, int32_t *__restrict__ claim) {
+__global__ void k_rcm_init(int64_t n, int32_t *__restrict__ claim) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) {
-    pos[i] = -1;
-    claim[i] = INT_MAX;
-  }
+  if (i < n) claim[i] = INT_MAX;
 }
 
 __global__ void k_rcm_zero(int32_t L, int32_t *__restrict__ a) {
@@ -56,18 +52,21 @@ __global__ void k_rcm_zero(int32_t L, int32_t *__restrict__ a) {
   if (i < L) a[i] = 0;
 }
 
-// The state of the level loop on the device: the current level holds the positions [s, e), its
-// children will be [e, e + next).
+// The state of the level loop on the device, a ring of one per round: the level holds the positions
+// [s, e), its children will be [e, e + next).
 struct Level {
   int32_t s, e, next, bad;
 };
 
+// claim[j]: the position of j's parent (the first of its neighbours), -1 for a seed, INT_MAX while not reached. A
+// node of an earlier or of this level holds a smaller position than the level's own, so it is never claimed again
+// and never counted, without a look at its own position (a level of about 5,000 nodes takes 33 us in 5 launches; 37
+// in 7 with that second gather per edge and with the sort and the advance in kernels of their own).
 // Claims of the level's nodes, and the nodes' final positions (their component's start plus its
 // nodes of earlier levels plus the place in this level's segment).
 __global__ void __launch_bounds__(256) k_rcm_claim(const Level *__restrict__ lv, const int32_t *__restrict__ ord,
                                                    const int64_t *__restrict__ indptr,
-                                                   const int32_t *__restrict__ indices,
-                                                   const int32_t *__restrict__ pos, int32_t *__restrict__ claim,
+                                                   const int32_t *__restrict__ indices, int32_t *__restrict__ claim,
                                                    const int32_t *__restrict__ cv, const int32_t *__restrict__ cstart,
                                                    const int32_t *__restrict__ done,
                                                    const int32_t *__restrict__ first, int32_t *__restrict__ fin) {
@@ -81,9 +80,10 @@ __global__ void __launch_bounds__(256) k_rcm_claim(const Level *__restrict__ lv,
     }
     for (int64_t b = indptr[i] + lane; b < indptr[i + 1]; b += kG) {
       const int32_t j = indices[b];
-      // a load past the L1 sees other groups' claims: most nodes are claimed by the first few
-      // positions, and the rest need no atomic
-      if (pos[j] < 0 && __hip_atomic_load(&claim[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > (int32_t)p)
+      // a cached load drops earlier levels' nodes; one past the L1 sees other groups' claims: most nodes are
+      // claimed by the first few positions, and the rest need no atomic
+      if (claim[j] > (int32_t)p &&
+          __hip_atomic_load(&claim[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > (int32_t)p)
         atomicMin(&claim[j], (int32_t)p);
     }
   }
@@ -92,7 +92,6 @@ __global__ void __launch_bounds__(256) k_rcm_claim(const Level *__restrict__ lv,
 __global__ void __launch_bounds__(256) k_rcm_count(const Level *__restrict__ lv, const int32_t *__restrict__ ord,
                                                    const int64_t *__restrict__ indptr,
                                                    const int32_t *__restrict__ indices,
-                                                   const int32_t *__restrict__ pos,
                                                    const int32_t *__restrict__ claim, int32_t *__restrict__ cnt) {
   const int32_t s = lv->s, e = lv->e;
   const int lane = (int)(threadIdx.x % kG);
@@ -101,7 +100,7 @@ __global__ void __launch_bounds__(256) k_rcm_count(const Level *__restrict__ lv,
     int32_t c = 0;
     for (int64_t b = indptr[i] + lane; b < indptr[i + 1]; b += kG) {
       const int32_t j = indices[b];
-      if (pos[j] < 0 && claim[j] == (int32_t)p) ++c;
+      if (claim[j] == (int32_t)p) ++c;
     }
 #pragma unroll
     for (int o = kG / 2; o > 0; o >>= 1) c += __shfl_xor(c, o, kG);
@@ -109,9 +108,10 @@ __global__ void __launch_bounds__(256) k_rcm_count(const Level *__restrict__ lv,
   }
 }
 
-// off[q] = nodes claimed by the level's first q nodes; lv->next = all of them. One workgroup.
-__global__ void __launch_bounds__(1024) k_rcm_scan(Level *__restrict__ lv, int64_t n, const int32_t *__restrict__ cnt,
-                                                   int32_t *__restrict__ off) {
+// off[q] = nodes claimed by the level's first q nodes; lv->next = all of them, and `after` the next round's level.
+// One workgroup.
+__global__ void __launch_bounds__(1024) k_rcm_scan(Level *__restrict__ lv, Level *__restrict__ after, int64_t n,
+                                                   const int32_t *__restrict__ cnt, int32_t *__restrict__ off) {
   __shared__ int32_t sums[16];
   const int32_t L = lv->e - lv->s;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -151,20 +151,23 @@ __global__ void __launch_bounds__(1024) k_rcm_scan(Level *__restrict__ lv, int64
   if (tid == 0) {
     off[L] = carry;
     // more children than nodes: an inconsistent graph (an edge without its reverse); none are taken
+    int32_t bad = lv->bad;
     if ((int64_t)lv->e + carry > n) {
-      lv->bad = 1;
+      bad = 1;
       carry = 0;
     }
     lv->next = carry;
+    *after = Level{lv->e, lv->e + carry, 0, bad};
   }
 }
 
-__global__ void __launch_bounds__(256) k_rcm_scatter(const Level *__restrict__ lv, int32_t *__restrict__ ord,
+// The children of the level's nodes, grouped by parent, as keys of the order inside a group: ascending degree,
+// then descending index.
+__global__ void __launch_bounds__(256) k_rcm_scatter(const Level *__restrict__ lv, const int32_t *__restrict__ ord,
                                                      const int64_t *__restrict__ indptr,
                                                      const int32_t *__restrict__ indices,
-                                                     const int32_t *__restrict__ pos,
                                                      const int32_t *__restrict__ claim,
-                                                     const int32_t *__restrict__ off) {
+                                                     const int32_t *__restrict__ off, uint64_t *__restrict__ key) {
   const int32_t s = lv->s, e = lv->e;
   if (lv->next == 0) return;
   const int lane = (int)(threadIdx.x % kG);
@@ -175,101 +178,53 @@ __global__ void __launch_bounds__(256) k_rcm_scatter(const Level *__restrict__ l
     const int64_t p = on ? p0 : s;
     const int32_t i = ord[p];
     const int64_t b1 = indptr[i + 1];
-    int32_t *out = ord + e + off[p - s];
+    uint64_t *out = key + off[p - s];
     // lanes past their own row stay in the loop for the group's ballots
     for (int64_t b = indptr[i]; b < b1; b += kG) {
       bool mine = false;
       int32_t j = 0;
       if (on && b + lane < b1) {
         j = indices[b + lane];
-        mine = pos[j] < 0 && claim[j] == (int32_t)p;
+        mine = claim[j] == (int32_t)p;
       }
       const uint32_t m = (uint32_t)((__ballot(mine) >> sh) & ((1ull << kG) - 1));
-      if (mine) out[__popc(m & ((1u << lane) - 1))] = j;
+      if (mine)
+        out[__popc(m & ((1u << lane) - 1))] =
+            ((uint64_t)(indptr[j + 1] - indptr[j]) << 32) | (uint64_t)(0xffffffffu - (uint32_t)j);
       out += __popc(m);
     }
   }
 }
 
-// Children of one parent: ascending degree, then descending index. One wave per parent:
-// each child's key (degree << 32 | ~index) goes to LDS and its rank among the group's keys
-// (all distinct) is its slot, which is the order a stable insertion sort by the same rule
-// gives. Groups above kSortCap children (not produced by the neighbour lists, whose rows
-// hold at most 2048 entries) are sorted by insertion in lane 0.
-constexpr int kSortCap = 2048;
-
-__device__ void rcm_sort_group(uint64_t *key, int32_t *g, int32_t m, const int64_t *__restrict__ indptr) {
-  const int lane = threadIdx.x;
-  if (m > kSortCap) {
-    if (lane == 0) {
-      for (int32_t a = 1; a < m; ++a) {
-        const int32_t v = g[a];
-        const int64_t dv = indptr[v + 1] - indptr[v];
-        int32_t b = a;
-        while (b > 0) {
-          const int32_t u = g[b - 1];
-          const int64_t du = indptr[u + 1] - indptr[u];
-          if (du < dv || (du == dv && u > v)) break;
-          g[b] = u;
-          --b;
-        }
-        g[b] = v;
-      }
-    }
-    return;
-  }
-  for (int32_t a = lane; a < m; a += 64) {
-    const int32_t v = g[a];
-    key[a] = ((uint64_t)(indptr[v + 1] - indptr[v]) << 32) | (uint64_t)(0xffffffffu - (uint32_t)v);
-  }
-  __syncthreads();
-  for (int32_t a0 = 0; a0 < m; a0 += 64) {
-    const int32_t a = a0 + lane;
-    const uint64_t ka = a < m ? key[a] : 0;
-    int32_t r = 0;
-    for (int32_t b = 0; b < m; ++b) r += key[b] < ka;
-    if (a < m) g[r] = (int32_t)(0xffffffffu - (uint32_t)ka);
-  }
-}
-
-__global__ void __launch_bounds__(64) k_rcm_sort_groups(const Level *__restrict__ lv, int32_t *__restrict__ ord,
-                                                        const int64_t *__restrict__ indptr,
-                                                        const int32_t *__restrict__ off) {
-  __shared__ uint64_t key[kSortCap];
-  const int32_t e = lv->e, L = e - lv->s;
-  if (lv->next == 0) return;
-  for (int32_t q = blockIdx.x; q < L; q += gridDim.x) {
-    const int32_t m = off[q + 1] - off[q];
-    if (m > 1) rcm_sort_group(key, ord + e + off[q], m, indptr);
-    __syncthreads();
-  }
-}
-
-// Positions of the new level [e, e + next) and its components' segments: a level's nodes of
-// component c are consecutive (the frontier is grouped by component, in component order, so
+// The new level [e, e + next): a thread per child ranks its key among its parent's children (neighbouring threads
+// read the same keys; a kernel of its own for this took 4 us per level and a launch), and its components' segments:
+// a level's nodes of component c are consecutive (the frontier is grouped by component, in component order, so
 // their children are too), and the segment's bounds come from comparing neighbours: one writer
 // each, no atomics. The first node's thread also closes c's previous segment, whose end the
 // other half of lend holds.
-__global__ void __launch_bounds__(256) k_rcm_place(const Level *__restrict__ lv, const int32_t *__restrict__ ord,
-                                                   int32_t *__restrict__ pos, const int32_t *__restrict__ cv,
+__global__ void __launch_bounds__(256) k_rcm_place(const Level *__restrict__ lv, int32_t *__restrict__ ord,
+                                                   const int32_t *__restrict__ claim, const int32_t *__restrict__ off,
+                                                   const uint64_t *__restrict__ key, const int32_t *__restrict__ cv,
                                                    int32_t *__restrict__ first, const int32_t *__restrict__ lend_old,
                                                    int32_t *__restrict__ lend, int32_t *__restrict__ done) {
-  const int32_t e = lv->e, L1 = lv->next;
+  const int32_t s = lv->s, e = lv->e, L1 = lv->next;
+  auto node = [](uint64_t k) { return (int32_t)(0xffffffffu - (uint32_t)k); };
   for (int32_t t = blockIdx.x * 256 + threadIdx.x; t < L1; t += gridDim.x * 256) {
-    const int32_t q = e + t, v = ord[q], c = cv[v];
-    pos[v] = q;
-    if (t == 0 || cv[ord[q - 1]] != c) {
+    const uint64_t k = key[t];
+    const int32_t v = node(k), c = cv[v], p = claim[v] - s;
+    const int32_t g0 = off[p], g1 = off[p + 1];
+    int32_t r = g0;
+#pragma unroll 8
+    for (int32_t b = g0; b < g1; ++b) r += key[b] < k || (key[b] == k && b < t);
+    ord[e + r] = v;
+    // which of a group's children stands at t does not matter here: they share the component
+    const int32_t q = e + t;
+    if (t == 0 || cv[node(key[t - 1])] != c) {
       done[c] += lend_old[c] - first[c];
       first[c] = q;
     }
-    if (t == L1 - 1 || cv[ord[q + 1]] != c) lend[c] = q + 1;   // one past the segment's end
+    if (t == L1 - 1 || cv[node(key[t + 1])] != c) lend[c] = q + 1;   // one past the segment's end
   }
-}
-
-__global__ void k_rcm_advance(Level *lv) {
-  lv->s = lv->e;
-  lv->e += lv->next;
-  lv->next = 0;
 }
 
 // ---- components: union-find over the edges. A root is only ever hooked (CAS) onto a
@@ -447,13 +402,13 @@ __global__ void __launch_bounds__(256) k_cc_vertex(int64_t n, const int32_t *__r
 
 // round 0: the seeds, one per component, each first in its component
 __global__ void k_rcm_seed_level(int32_t C, const int32_t *__restrict__ S, int32_t *__restrict__ ord,
-                                 int32_t *__restrict__ pos, int32_t *__restrict__ done, int32_t *__restrict__ first,
+                                 int32_t *__restrict__ claim, int32_t *__restrict__ done, int32_t *__restrict__ first,
                                  int32_t *__restrict__ lend, Level *__restrict__ lv) {
   const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c == 0) *lv = Level{0, C, 0, 0};
   if (c >= C) return;
   ord[c] = S[c];
-  pos[S[c]] = c;
+  claim[S[c]] = -1;
   done[c] = 0;
   first[c] = c;
   lend[c] = c + 1;
@@ -508,9 +463,11 @@ unsigned blocks_for(int64_t threads, int bs) { return (unsigned)((threads + bs -
 extern "C" {
 
 constexpr int kRcmArrays = 20;  // int32 arrays of n + 2 entries in the work buffer
+constexpr int kRcmHead = 256;   // bytes before them: the levels' states and a flag
+constexpr int kRounds = 8;      // levels per look at their bounds
 
 int64_t inch_rcm_device_work_size(int64_t n) {
-  return (kRcmArrays * (n + 2) + 2 * (scan_tiles(n + 1) + 2)) * (int64_t)sizeof(int32_t) + 64;
+  return (kRcmArrays * (n + 2) + 2 * (scan_tiles(n + 1) + 2)) * (int64_t)sizeof(int32_t) + kRcmHead;
 }
 
 inch_status inch_rcm_device(int64_t n, const int64_t *indptr, const int32_t *indices, const int64_t *seeds,
@@ -523,12 +480,13 @@ inch_status inch_rcm_device(int64_t n, const int64_t *indptr, const int32_t *ind
                (long long)work_bytes, (long long)inch_rcm_device_work_size(n));
   hipStream_t st = (hipStream_t)stream;
   int32_t *arr[kRcmArrays];
-  for (int q = 0; q < kRcmArrays; ++q) arr[q] = (int32_t *)((char *)work + 64) + q * (n + 2);
-  int32_t *pos = arr[0], *claim = arr[1], *cnt = arr[2], *off = arr[3], *label2 = arr[4], *ord = arr[5];
+  for (int q = 0; q < kRcmArrays; ++q) arr[q] = (int32_t *)((char *)work + kRcmHead) + q * (n + 2);
+  uint64_t *key = (uint64_t *)arr[0];   // two arrays
+  int32_t *cnt = arr[2], *off = arr[3], *label2 = arr[4], *claim = label2, *ord = arr[5];   // claim once label2 is used
   int32_t *label = arr[6], *rank = arr[7], *minr = arr[8], *flag = arr[9], *cidx = arr[10], *croot = arr[11];
   int32_t *cv = arr[12], *csize = arr[13], *cstart = arr[14], *fin = arr[15], *first = arr[16], *lend = arr[17];
   int32_t *done = arr[18], *S = arr[19], *lend2 = flag;   // flag is free once the seeds are known
-  Level *lv = (Level *)((char *)work + 16);
+  Level *lv = (Level *)((char *)work + 16);   // kRounds of them
   int32_t *tsum = arr[kRcmArrays - 1] + (n + 2), *toff = tsum + scan_tiles(n + 1) + 2;
   const int bs = 256;
   int32_t *bad = (int32_t *)((char *)work + 8);
@@ -549,7 +507,6 @@ inch_status inch_rcm_device(int64_t n, const int64_t *indptr, const int32_t *ind
   HIP_TRY(hipMemcpyAsync(&bad_h, bad, sizeof(bad_h), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   INCH_REQUIRE(!bad_h, "inch_rcm_device: seeds is not a permutation");
-  k_rcm_init<<<blocks_for(n, bs), bs, 0, st>>>(n, pos, claim);
   // components, their seeds (first node in the seed order) and sizes, in seed order
   k_cc_init<<<blocks_for(n * kCcLanes, bs), bs, 0, st>>>(n, indptr, indices, label);
   k_cc_flatten<<<blocks_for(n, bs), bs, 0, st>>>(n, label);
@@ -560,6 +517,7 @@ inch_status inch_rcm_device(int64_t n, const int64_t *indptr, const int32_t *ind
   HIP_TRY(hipMemcpyAsync(label2, label, n * sizeof(int32_t), hipMemcpyDeviceToDevice, st));
   k_cc_hook<<<blocks_for(n * kCcLanes, bs), bs, 0, st>>>(n, indptr, indices, label2, label);
   k_cc_flatten<<<blocks_for(n, bs), bs, 0, st>>>(n, label);
+  k_rcm_init<<<blocks_for(n, bs), bs, 0, st>>>(n, claim);
   k_cc_rank<<<blocks_for(n, bs), bs, 0, st>>>(n, seeds, rank, minr);
   k_cc_minrank<<<blocks_for(n, bs), bs, 0, st>>>(n, label, rank, minr);
   k_cc_flag<<<blocks_for(n, bs), bs, 0, st>>>(n, seeds, label, minr, flag);
@@ -572,23 +530,20 @@ inch_status inch_rcm_device(int64_t n, const int64_t *indptr, const int32_t *ind
   HIP_TRY(hipStreamSynchronize(st));
   if (C < 1 || C > n) INCH_FAIL(INCH_ERR_INVALID, "inch_rcm_device: %d components", C);
   HIP_TRY(scan_exclusive_into<int32_t>(C, csize, cstart, tsum, toff, st));
-  k_rcm_seed_level<<<blocks_for(C, bs), bs, 0, st>>>(C, S, ord, pos, done, first, lend, lv);
+  k_rcm_seed_level<<<blocks_for(C, bs), bs, 0, st>>>(C, S, ord, claim, done, first, lend, lv);
   HIP_TRY(hipGetLastError());
   // all components' levels advance together, kRounds levels per look at the bounds
-  constexpr int kRounds = 8;
   const unsigned gg = blocks_for(n * kG, bs) < 2048 ? blocks_for(n * kG, bs) : 2048;
   const unsigned gn = blocks_for(n, bs) < 1024 ? blocks_for(n, bs) : 1024;
-  const unsigned gs = n < 8192 ? (unsigned)n : 8192;
   Level h{0, C, 0, 0};
   while (true) {
     for (int r = 0; r < kRounds; ++r) {
-      k_rcm_claim<<<gg, bs, 0, st>>>(lv, ord, indptr, indices, pos, claim, cv, cstart, done, first, fin);
-      k_rcm_count<<<gg, bs, 0, st>>>(lv, ord, indptr, indices, pos, claim, cnt);
-      k_rcm_scan<<<1, 1024, 0, st>>>(lv, n, cnt, off);
-      k_rcm_scatter<<<gg, bs, 0, st>>>(lv, ord, indptr, indices, pos, claim, off);
-      k_rcm_sort_groups<<<gs, 64, 0, st>>>(lv, ord, indptr, off);
-      k_rcm_place<<<gn, bs, 0, st>>>(lv, ord, pos, cv, first, lend, lend2, done);
-      k_rcm_advance<<<1, 1, 0, st>>>(lv);
+      Level *now = lv + r;
+      k_rcm_claim<<<gg, bs, 0, st>>>(now, ord, indptr, indices, claim, cv, cstart, done, first, fin);
+      k_rcm_count<<<gg, bs, 0, st>>>(now, ord, indptr, indices, claim, cnt);
+      k_rcm_scan<<<1, 1024, 0, st>>>(now, lv + (r + 1) % kRounds, n, cnt, off);
+      k_rcm_scatter<<<gg, bs, 0, st>>>(now, ord, indptr, indices, claim, off, key);
+      k_rcm_place<<<gn, bs, 0, st>>>(now, ord, claim, off, key, cv, first, lend, lend2, done);
       int32_t *swap = lend;
       lend = lend2;
       lend2 = swap;
