@@ -180,3 +180,26 @@ def test_tiles_fall_back(cuda):
     assert tiny.tiles() is None and isinstance(tiny.slot_form(), RecordForm)
     with pytest.raises(ops.InchingError):
         ops.Tiles(A.xyz, A.rowptr, A.col, 5.0, (8, 8))
+
+
+@pytest.mark.parametrize("columns", [1, 5])
+def test_block_product_lays_out_tiles_only_where_they_pay(cuda, columns, monkeypatch):
+    """A fresh matrix: below the line the product leaves the tiles out, at it or with tiles at hand it takes them;
+    both agree to rounding (124 terms a row)."""
+    from inching_amd import hessian
+    print("case: block product rule %d" % columns, flush=True)
+    rng = np.random.default_rng(3)
+    xyz = rng.uniform(0.0, 30.0, (1500, 3))
+    X = torch.as_tensor(rng.standard_normal((4500, columns)), device="cuda")
+    A = hessian.build_hessian(xyz, 8.0, precision=())
+    plain = A.matfree(X)
+    assert "_tiles" not in A.__dict__
+    monkeypatch.setattr(hessian, "TILE_APPLY_TERMS", A.nnzb * columns + 1)
+    A.matfree(X)
+    assert "_tiles" not in A.__dict__
+    monkeypatch.setattr(hessian, "TILE_APPLY_TERMS", A.nnzb * columns)
+    tiled = A.matfree(X)
+    assert A.__dict__["_tiles"] is not None
+    monkeypatch.setattr(hessian, "TILE_APPLY_TERMS", float("inf"))
+    assert torch.equal(A.matfree(X), tiled)
+    assert (plain - tiled).abs().max() <= 1e-11 * plain.abs().max()
