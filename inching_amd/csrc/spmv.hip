@@ -1592,7 +1592,8 @@ __device__ __forceinline__ void sum_few(int nparts, int J, const double *__restr
 
 // u -= scale V^T h for the J <= 16 sums h of `part`, in the launch that forms these sums (every block alike) and, with
 // `atoms`, unpacks acc (slot order) into u first. The operator's Hotelling term: with 6 rows of 18,021 dofs a sum of
-// partials, an update and an unpacking took 8.3 us and the gaps between them, now 4.5 (latency).
+// partials, an update and an unpacking took 8.3 us and the gaps between them, now 4.5 (latency); the caller
+// keeps to vectors short enough for that.
 __global__ void __launch_bounds__(256) k_shift(int64_t count, int J, int nparts, const double *__restrict__ part,
                                                double scale, const double *__restrict__ V, int64_t ld,
                                                const int32_t *__restrict__ atoms, const double *__restrict__ acc,

@@ -179,9 +179,10 @@ class Operator:
 
     def apply(self, v64, u64):
         self.n_apply += 1
-        # a few rows Q (the six rigid motions) and a result of its own: the Hotelling term in two launches
+        # a few rows Q (the six rigid motions) of a short vector and a result of its own: the Hotelling term in two
+        # launches
         few = (self.Q is not None and self.shift != 0.0 and self.Q.shape[0] <= ops.SHIFT_MAX_M
-               and v64.dtype == torch.float64 and u64.dtype == torch.float64 and v64.is_contiguous()
+               and self.n <= ops.SHIFT_MAX_DOF and v64.dtype == torch.float64 and u64.dtype == torch.float64 and v64.is_contiguous()
                and u64.is_contiguous() and v64.data_ptr() != u64.data_ptr())
         if few and self.pol is not None and self._on_records(v64, u64):
             self._filtered_records(v64, u64, shift=True)

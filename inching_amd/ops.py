@@ -589,6 +589,10 @@ def multidot(V, J, u, h, ws, stream=None):
 # Most rows of inch_shift_apply: every workgroup sums all partials itself (16 x 512 at most); locked blocks of
 # vectors take a sum kernel and an update instead.
 SHIFT_MAX_M = 16
+# Most dofs for which it pays (with the unpacking, 6 rows; against an unpacking, a multi-dot and an update): 7.6 and
+# 11.0 us at 18,021 dofs, 9.2 and 11.6 at 60,000, 15.1 and 14.4 at 150,000, where its rows read in slot order cost
+# more than the launches.
+SHIFT_MAX_DOF = 120000
 
 
 def shift_apply(Q, v, scale, u, ws, atoms=None, acc=None, stream=None):

@@ -76,3 +76,22 @@ def test_lanczos3_step(n, records):
     fd.copy_(torch.as_tensor(f0))
     step.update(vd, fd, out[0:1])
     assert abs(out[0].item() - v.astype(L) @ f0) <= tol
+
+
+@pytest.mark.parametrize("pol", [False, True])
+def test_hotelling_term_either_way(pol, monkeypatch):
+    """Operator.apply below and above the line of the two-launch form: the same to rounding."""
+    from inching_amd import chebyshev, hessian
+    from inching_amd.operator import Operator
+    rng = np.random.default_rng(11)
+    A = hessian.build_hessian(rng.uniform(0.0, 30.0, (1500, 3)), 8.0, precision=())
+    Q = torch.linalg.qr(torch.as_tensor(rng.standard_normal((4500, 6)), device="cuda"))[0].T.contiguous()
+    design = chebyshev.design_filter(1.0, 3.0, (1.0, 80.0), 5120, 5, 0.7) if pol else None
+    op = Operator(A, "mf64", pol=design, Q=Q, shift=-40.0)
+    v = torch.as_tensor(rng.standard_normal(4500), device="cuda")
+    a, b = torch.empty_like(v), torch.empty_like(v)
+    op.apply(v, a)
+    monkeypatch.setattr(ops, "SHIFT_MAX_DOF", 4499)
+    op.apply(v, b)
+    h = Q.abs() @ v.abs()
+    assert ((a - b).abs() <= 1e-13 * (a.abs().max() + 40.0 * (Q.abs().T @ h))).all()
