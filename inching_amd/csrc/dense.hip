@@ -27,8 +27,8 @@ constexpr int kGramGrid = 1024;    // most column blocks of a Gram product (at l
 // through LDS with coalesced row loads, the next chunk's in flight while the current one is used;
 // when X and Y are the same rows (SAME) they are staged once. The contraction dimension is the
 // column index i of X and Y. Memory bounds it: 64 x 64 over 900,000 columns took 289 us with both
-// operands staged and a wait on memory per chunk, now 164 (0.46 GB read, the matrix cores busy for
-// three quarters of it); 64 x 6 with its sum took 247, now 94.
+// operands staged and a wait on memory per chunk, 164 with the loads ahead (the matrix cores busy for three
+// quarters of it) and 135 without the tiles that mirror others (0.46 GB, 3.4 TB/s); 64 x 6 with its sum took 247, now 94.
 // v_mfma_f64_16x16x4f64 operand layout: A (16x4): lane l holds A[l%16][l/16];
 // B (4x16): lane l holds B[l/16][l%16]; D (16x16): lane l, element r holds
 // D[(l/16) + 4*r][l%16] (checked on gfx950 with one-hot operands).
@@ -42,9 +42,14 @@ __global__ void __launch_bounds__(256) k_gram_mfma(int64_t len, int k1, const do
   auto &ys = *reinterpret_cast<double(*)[SAME ? kTile : 16 * NT][kChunk + 1]>(SAME ? &xs[0][0] : &ys_own[0][0]);
   const int a0 = blockIdx.y * kTile, b0 = blockIdx.z * kTile;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  double4_t acc[NT];
+  // 64 rows with themselves: of the 4 x 4 tiles wave w forms (w, w), (w, w + 1) and (w, w + 2) round the 4, and
+  // writes the second one's mirror too
+  constexpr bool HALF = SAME && NT == 4;
+  constexpr int TILES = HALF ? 3 : NT;
+  auto tile_of = [&](int t) { return HALF ? (w + t) & 3 : t; };
+  double4_t acc[TILES];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < TILES; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
   const int64_t per = (len + gridDim.x - 1) / gridDim.x;
   const int64_t i_beg = blockIdx.x * per;
   const int64_t i_end = (i_beg + per < len) ? i_beg + per : len;
@@ -78,8 +83,8 @@ __global__ void __launch_bounds__(256) k_gram_mfma(int64_t len, int k1, const do
     for (int kk = 0; kk < kChunk; kk += 4) {
       const double av = xs[16 * w + (lane & 15)][kk + (lane >> 4)];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const double bv = ys[16 * t + (lane & 15)][kk + (lane >> 4)];
+      for (int t = 0; t < TILES; ++t) {
+        const double bv = ys[16 * tile_of(t) + (lane & 15)][kk + (lane >> 4)];
         acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
       }
     }
@@ -87,12 +92,15 @@ __global__ void __launch_bounds__(256) k_gram_mfma(int64_t len, int k1, const do
   // write the 64 x (16 NT) partial tile of this block
   double *dst = part + (int64_t)blockIdx.x * k1 * k2;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
+  for (int t = 0; t < TILES; ++t) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int a = a0 + 16 * w + (lane >> 4) + 4 * r;
-      const int b = b0 + 16 * t + (lane & 15);
-      if (a < k1 && b < k2) dst[(int64_t)a * k2 + b] = acc[t][r];
+      const int b = b0 + 16 * tile_of(t) + (lane & 15);
+      if (a < k1 && b < k2) {
+        dst[(int64_t)a * k2 + b] = acc[t][r];
+        if (HALF && t == 1) dst[(int64_t)b * k2 + a] = acc[t][r];
+      }
     }
   }
 }
