@@ -1864,6 +1864,7 @@ extern "C" inch_status inch_bsr_tiles(int64_t n, const int64_t *rowptr, const in
     k_bsr_tiles<true><<<(unsigned)ntile, 256, 0, st>>>(rowptr, col, order, tile_start, ustride, tile, slots, ulen, ulist,
                                                        uidx, nullptr);
     HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(st));   // the lists may be read on any stream from here on
     return INCH_OK;
   }
   DevBuf um;

@@ -135,3 +135,19 @@ def test_tile_periodic():
     ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, A.vals64, x, y, lanes=T.LANES, col16=T)
     ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, A.vals64, x, y2, lanes=16)
     assert torch.allclose(y, y2, rtol=1e-12, atol=1e-12 * float(y2.abs().max()))
+
+
+def test_tile_lists_on_another_stream():
+    """Lists laid out on one stream are whole for a product on another without a wait in between."""
+    A = _matrix(3000, 4)
+    x = torch.randn(9000, dtype=torch.float64, device="cuda")
+    y, y2 = torch.empty_like(x), torch.empty_like(x)
+    ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, A.vals64, x, y2, lanes=16)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s1):
+        T = A.bsr_tiles()
+    with torch.cuda.stream(s2):
+        ops.bsr_spmv(A.n_atoms, A.rowptr, A.col, A.vals64, x, y, lanes=T.LANES, col16=T)
+    torch.cuda.synchronize()
+    assert torch.allclose(y, y2, rtol=1e-12, atol=1e-12 * float(y2.abs().max()))
