@@ -49,6 +49,12 @@ def _check_dev(*ts):
                 raise ValueError("tensor must be contiguous")
 
 
+def _scratch(k, dtype, device, stream):
+    """Memory for kernels on ``stream`` alone: given back to that stream's pool when it is dropped."""
+    with torch.cuda.stream(stream):
+        return torch.empty(k, dtype=dtype, device=device)
+
+
 # ------------------------------------------------------------------ host ----
 
 def synth_globule(n, radius, dmin, seed, max_attempts=0):
@@ -117,20 +123,29 @@ def batch_head(n, maxleaf):
 
 def neighbours(xyz, rc, stream=None, ascending=True):
     """Cell-list neighbour CSR of device float64 coordinates [n,3] -> (indptr, indices).
-    ``ascending=False`` leaves each row's columns in an unspecified order."""
+    ``ascending=False`` leaves each row's columns in an unspecified order. Both are whole on
+    return, for any stream."""
     require_gpu()
     _check_dev(xyz)
     if xyz.dtype != torch.float64 or xyz.dim() != 2 or xyz.shape[1] != 3:
         raise ValueError("xyz must be float64 [n,3]")
     n, dev, sp = xyz.shape[0], xyz.device, stream_ptr(stream)
     rc = float(rc)
-    indptr = torch.empty(n + 1, dtype=torch.int64, device=dev)
     plan, size, nnz = (C.c_double * 7)(), C.c_int64(0), C.c_int64(0)
-    scratch = torch.empty(256 * 6, dtype=torch.float64, device=dev)
-    call("inch_cells_plan", n, P(xyz), rc, plan, C.byref(size), P(scratch), sp)
-    work = torch.empty(size.value, dtype=torch.uint8, device=dev)
+
+    def result(k, dtype):
+        # the caller's memory, from the current stream: what still runs there on a reused block goes before ``stream``
+        t = torch.empty(k, dtype=dtype, device=dev)
+        if stream is not None:
+            stream.wait_stream(torch.cuda.current_stream(dev))
+        return t
+
+    indptr = result(n + 1, torch.int64)
+    part = _scratch(256 * 6, torch.float64, dev, stream)
+    call("inch_cells_plan", n, P(xyz), rc, plan, C.byref(size), P(part), sp)
+    work = _scratch(size.value, torch.uint8, dev, stream)
     call("inch_cells_count", n, P(xyz), rc, plan, P(work), size.value, P(indptr), C.byref(nnz), sp)
-    indices = torch.empty(max(1, nnz.value), dtype=torch.int32, device=dev)
+    indices = result(max(1, nnz.value), torch.int32)
     call("inch_cells_fill", n, rc, plan, P(work), size.value, P(indptr), P(indices), 1 if ascending else 0, sp)
     return indptr, indices[:nnz.value]
 

@@ -1,0 +1,72 @@
+"""Results that a call hands out are whole on every stream, and its scratch is neither given back while
+kernels still read it nor taken while earlier work still writes it."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import small_globule
+
+pytestmark = pytest.mark.gpu
+
+LONG = 50_000_000     # cycles of a wait that outlasts the launches after it (0.02 s or more)
+
+
+def _cloud(n, seed):
+    return torch.as_tensor(np.random.default_rng(seed).uniform(0.0, (n / 0.05) ** (1.0 / 3.0), (n, 3)), device="cuda")
+
+
+@pytest.mark.parametrize("own", [False, True])
+@pytest.mark.parametrize("ascending", [True, False])
+def test_neighbours_are_whole_on_return(cuda, own, ascending):
+    from inching_amd import ops
+    print("case: neighbours whole on return, stream %s, ascending %s" % (own, ascending), flush=True)
+    xyz = _cloud(60000, 1)
+    s = torch.cuda.Stream() if own else None
+    torch.cuda.synchronize()
+    ip, ix = ops.neighbours(xyz, 8.0, stream=s, ascending=ascending)
+    assert (s or torch.cuda.current_stream()).query()
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):      # no wait between: the list is symmetric, every row names itself
+        total = ip[-1].item()
+        rows = torch.repeat_interleave(torch.arange(60000, device="cuda"), ip.diff(), output_size=total)
+        assert int((rows == ix).sum()) == 60000
+        assert int((rows * 131071 + ix).sum() - (ix.long() * 131071 + rows).sum()) == 0
+    torch.cuda.synchronize()
+
+
+def test_neighbours_wait_for_a_reused_block(cuda):
+    """The result's memory comes from the current stream, where a write to the block's former tensor may still be
+    queued: the search on another stream follows it, and coordinates still being written there too."""
+    from inching_amd import ops
+    print("case: neighbours after a reused block", flush=True)
+    n = 20000
+    xyz = _cloud(n, 2)
+    ip, ix = ops.neighbours(xyz, 8.0)
+    want = ip.clone(), ix.clone()
+    later = torch.full_like(xyz, 1.0)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(LONG)
+    later.copy_(xyz)
+    ip.fill_(0)
+    ix.fill_(0)
+    del ip, ix
+    ip, ix = ops.neighbours(later, 8.0, stream=s)
+    torch.cuda.synchronize()
+    assert torch.equal(ip, want[0]) and torch.equal(ix, want[1])
+
+
+def test_build_without_ordering_on_another_stream(cuda):
+    from inching_amd.hessian import build_hessian
+    print("case: build_hessian on one stream, product on another", flush=True)
+    X = small_globule(3000, seed=4)
+    x = torch.randn(9000, dtype=torch.float64, device="cuda")
+    ref = build_hessian(X, 8.0, reorder=False, precision=()).matfree(x)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s1):
+        A = build_hessian(X, 8.0, reorder=False, precision=())
+    with torch.cuda.stream(s2):
+        y = A.matfree(x)
+    torch.cuda.synchronize()
+    assert torch.equal(y, ref)
