@@ -379,7 +379,7 @@ class Tiles:
             raise ValueError("X and Y must be contiguous float64 [3n, r]")
         r = 1 if X.dim() == 1 else X.shape[1]
         size = int(call("inch_anm_tile_apply_work_size", self.ntile, self.shape[0], r))
-        work = torch.empty(size, dtype=torch.float64, device=X.device)
+        work = _scratch(size, torch.float64, X.device, stream)
         call("inch_anm_matfree_tile_apply", self.ntile, *self.shape, P(self.rec), P(self.atoms), *self._lists,
              float(plus_i), P(X), P(Y), r, P(work), stream_ptr(stream))
 

@@ -70,3 +70,34 @@ def test_build_without_ordering_on_another_stream(cuda):
         y = A.matfree(x)
     torch.cuda.synchronize()
     assert torch.equal(y, ref)
+
+
+def test_block_product_keeps_its_scratch(cuda, monkeypatch):
+    """The packed columns of a block product on another stream are not handed to the current stream while that product
+    has still to run."""
+    from inching_amd import ops
+    from inching_amd.hessian import build_hessian
+    print("case: block product's scratch", flush=True)
+    A = build_hessian(small_globule(3000, seed=5), 8.0, precision=())
+    T = A.tiles()
+    X = torch.randn(9000, 16, dtype=torch.float64, device="cuda")
+    Y, want = torch.empty_like(X), torch.empty_like(X)
+    T.apply(X, want, 1.0)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    work, call = [], ops.call
+
+    def spy(name, *args):
+        if name == "inch_anm_matfree_tile_apply":
+            work.append(args[-2])
+        return call(name, *args)
+
+    monkeypatch.setattr(ops, "call", spy)
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(LONG)
+    T.apply(X, Y, 1.0, stream=s)
+    junk = [torch.empty(12 * T.slots * 4, dtype=torch.float64, device="cuda") for _ in range(4)]
+    assert len(work) == 1 and all(t.data_ptr() != work[0] for t in junk)
+    torch.cuda.synchronize()
+    assert torch.equal(Y, want)
