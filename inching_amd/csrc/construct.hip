@@ -1252,7 +1252,7 @@ struct CellWork {
   }
 };
 
-// grid: lo[3], 1 / cell size, dim[3] of cells of the cutoff over the atoms' bounding box; part:
+// grid: lo[3], 1 / cell size, dim[3] of cells of about the cutoff over the atoms' bounding box; part:
 // device scratch of 256 x 6 doubles. Syncs.
 inch_status cell_grid(int64_t n, const double *xyz, double rc, double *part, Grid &g, int64_t &ncell, const char *who,
                       hipStream_t st) {
@@ -1274,7 +1274,9 @@ inch_status cell_grid(int64_t n, const double *xyz, double rc, double *part, Gri
     }
     if (nan || !std::isfinite(g.lo[a]) || !std::isfinite(hi[a])) INCH_FAIL(INCH_ERR_NAN, "%s: non-finite coordinates", who);
   }
-  g.inv = 1.0 / rc;
+  // cells a millionth wider than the cutoff: (v - lo) inv is off by at most 3 roundings, 4e-7 at 1.1e9 cells, so that
+  // two atoms within the cutoff never lie two cells apart
+  g.inv = (1.0 - 1e-6) / rc;
   ncell = 1;
   for (int a = 0; a < 3; ++a) {
     const double d = std::floor((hi[a] - g.lo[a]) * g.inv) + 1.0;

@@ -76,3 +76,20 @@ def test_row_sort_at_its_edges(cuda, equal):
     op, oi = ops.csr_permute(dev(ip), dev(np.concatenate(rows).astype(np.int32)), dev(order), dev(undo))
     for i, row in enumerate(_rows(op, oi)):
         assert np.array_equal(row, np.sort(undo[rows[order[i]]])), i
+
+
+@pytest.mark.parametrize("rc,lo,step", [(49.0, 0.0, 49.0), (7.3, 0.0, 7.3), (8.0, 5.3, 8.0), (0.8, 0.1, 0.8)])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_pairs_at_the_cutoff_across_rounded_cells(cuda, rc, lo, step, axis):
+    """Atoms one cutoff apart along an axis: (v - lo) / rc rounds to either side of a whole number, so that with cells
+    of the cutoff itself two such atoms could lie two cells apart, and a row held the other while its own did not."""
+    from inching_amd import ops
+    print("case: pairs at the cutoff %g, axis %d" % (rc, axis), flush=True)
+    X = np.zeros((200, 3))
+    X[:, axis] = lo + step * np.arange(200)
+    X[100:, (axis + 1) % 3] = 0.25 * rc
+    X[100:, axis] = X[:100, axis]
+    want = _brute(X, rc)
+    ip, ix = ops.neighbours(torch.as_tensor(X, device="cuda"), rc)
+    for i, row in enumerate(_rows(ip, ix)):
+        assert np.array_equal(row, np.nonzero(want[i])[0]), i
