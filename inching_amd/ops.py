@@ -351,8 +351,11 @@ class Tiles:
         self._lists = (P(self.ulen), P(self.ulist), ucap, umax.value, P(self.waves), P(self.pairs), bx, by)
 
     def buffers(self, count):
-        """``count`` record buffers [6 slots] with the slots' coordinates, the caller's own."""
-        return [self.rec.clone() for _ in range(count)]
+        """``count`` record buffers [6 slots] with the slots' coordinates, the caller's own; whole on return, for any
+        stream."""
+        recs = [self.rec.clone() for _ in range(count)]
+        torch.cuda.current_stream(self.rec.device).synchronize()
+        return recs
 
     def _records(self, *recs):
         for r in recs:

@@ -101,3 +101,26 @@ def test_block_product_keeps_its_scratch(cuda, monkeypatch):
     assert len(work) == 1 and all(t.data_ptr() != work[0] for t in junk)
     torch.cuda.synchronize()
     assert torch.equal(Y, want)
+
+
+def test_filter_on_another_stream_than_its_operator(cuda):
+    """The record buffers of an Operator are whole when it is made: its first application may run elsewhere."""
+    from inching_amd import chebyshev as CH
+    from inching_amd.hessian import build_hessian
+    from inching_amd.operator import Operator
+    print("case: operator made on one stream, applied on another", flush=True)
+    A = build_hessian(small_globule(3000, seed=5), 8.0, precision=())
+    pol = CH.design_filter(1.0, 3.0, (1.0, 80.0), 5120, 5, 0.7)
+    v = torch.randn(9000, dtype=torch.float64, device="cuda")
+    u, want = torch.empty_like(v), torch.empty_like(v)
+    Operator(A, "mf64", pol=pol).apply(v, want)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s1):
+        torch.cuda._sleep(LONG)
+        op = Operator(A, "mf64", pol=pol)
+    assert s1.query()
+    with torch.cuda.stream(s2):
+        op.apply(v, u)
+    torch.cuda.synchronize()
+    assert torch.equal(u, want)
