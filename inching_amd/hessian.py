@@ -60,10 +60,12 @@ class RecordForm:
             prev, cur = cur, out
 
 
-# Pairs times columns from which one block product pays for laying the tiles out first (once they are there, every
-# product takes them). First product on a fresh matrix, with the layout against without: 20,000 atoms x 64 columns
-# (1.4e8) 583 and 358 us, 40,000 x 64 (2.9e8) 742 and 733, 100,000 x 64 (7.4e8) 1430 and 1988; 100,000 x 8 (9e7) 853
-# and 240. The next ones: 171 and 383, 295 and 764, 740 and 1998, 111 and 228.
+# Pairs times columns from which a block product takes the tiles, also when it has to lay them out first. First product
+# on a fresh matrix, with the layout against the cluster layout at hand: 20,000 atoms x 64 columns (1.4e8) 583 and 358
+# us, 40,000 x 64 (2.9e8) 742 and 733, 100,000 x 64 (7.4e8) 1430 and 1988; 100,000 x 8 (9e7) 853 and 240. The next ones
+# are faster on the tiles at every size and column count (171 and 383, 295 and 764, 740 and 1998, 111 and 228; one
+# column of 100,003 atoms 74 and 117, of 2.4M 1716 and 2488), but the line asks for nothing but the matrix and the
+# call, so that a product's bits do not depend on what was called before.
 TILE_APPLY_TERMS = 2.5e8
 
 
@@ -246,8 +248,10 @@ class BlockHessian:
         """FP64 (H + PlusI I) X recomputed from coordinates (X [3n] or [3n, r])."""
         Y = torch.empty_like(X)
         columns = X.numel() // max(1, 3 * self.n_atoms)
-        tiled = "_tiles" in self.__dict__ or self.nnzb * columns >= TILE_APPLY_TERMS
+        tiled = self.nnzb * columns >= self.__dict__.get("_apply_line", TILE_APPLY_TERMS)
         if tiled and self.tiles() is not None and X.numel() and X.dtype == torch.float64 and Y.is_contiguous():
+            # a later change of the module's line does not move products that took the tiles
+            self.__dict__.setdefault("_apply_line", TILE_APPLY_TERMS)
             self.tiles().apply(X.contiguous(), Y, self.plus_i)
         elif self.images is not None:
             ops.matfree_pbc(self.xyz, self.rowptr, self.col, self.images, self.box, self.plus_i, X.contiguous(), Y)
