@@ -23,3 +23,33 @@ def test_block_product_does_not_depend_on_earlier_calls(cuda, columns):
     Operator(A, "mf64", pol=CH.design_filter(1.0, 3.0, (1.0, 80.0), 5120, 5, 0.7))
     assert A.tiles() is not None
     assert torch.equal(A.matfree(X), first)
+
+
+@pytest.mark.parametrize("shape", [(1500, 3), (4500,), (1500, 3, 2), (4500, 2, 2), (1500, 6)])
+def test_block_product_takes_every_shape_on_both_forms(cuda, shape, monkeypatch):
+    """Shapes of 3 n x r values: the tile form takes what the cluster layout takes. Row sums of at most 200 terms."""
+    from inching_amd import hessian
+    print("case: matfree %s" % (shape,), flush=True)
+    A = _matrix()
+    X = torch.randn(shape, dtype=torch.float64, device="cuda")
+    want = A.matfree(X)
+    assert "_tiles" not in A.__dict__
+    monkeypatch.setattr(hessian, "TILE_APPLY_TERMS", 0)
+    got = A.matfree(X)
+    assert A.tiles() is not None and got.shape == want.shape
+    assert float((got - want).abs().max()) <= 1e-12 * float(want.abs().max())
+
+
+def test_block_product_refuses_wrong_sizes_on_both_forms(cuda, monkeypatch):
+    from inching_amd import hessian
+    print("case: matfree of wrong sizes", flush=True)
+    A = _matrix()
+    bad = torch.randn(4501, dtype=torch.float64, device="cuda")
+    for line in (float("inf"), 0):
+        monkeypatch.setattr(hessian, "TILE_APPLY_TERMS", line)
+        with pytest.raises((ValueError, RuntimeError)):
+            A.matfree(bad)
+        with pytest.raises((ValueError, RuntimeError)):
+            A.matfree(torch.randn(4500, 2, device="cuda"))
+        with pytest.raises((ValueError, RuntimeError)):
+            A.matfree(torch.empty(4500, 0, dtype=torch.float64, device="cuda"))
