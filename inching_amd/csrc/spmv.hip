@@ -920,21 +920,22 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
 // third of its pairs outside the cutoff, 44 gathers per atom) took 1.83 ms; this takes 0.63, of
 // which the packing 0.05.
 constexpr int kBlockCols = 4;
+constexpr int kBlockPass = 64;   // columns packed and multiplied at a time: the workspace stays at 1.5 KB a slot
 constexpr size_t kTileBlockLds = 160 * 1024;
 
 // P[(group * slots + q) * 12 + 4 k + c] = X[3 a + k, 4 group + c], a the atom of slot q; zeros on
-// padding slots and past the last column. 16 slots per workgroup, 64 columns at a time through LDS.
+// padding slots and past the last of nc <= 64 columns. 16 slots per workgroup, through LDS.
 __global__ void __launch_bounds__(192) k_block_pack(int64_t slots, const int32_t *__restrict__ atoms,
-                                                    const double *__restrict__ X, int nrhs, double *__restrict__ P) {
-  __shared__ double tile[16][3][65];
+                                                    const double *__restrict__ X, int64_t ld, int nc,
+                                                    double *__restrict__ P) {
+  __shared__ double tile[16][3][kBlockPass + 1];
   const int64_t q0 = 16 * (int64_t)blockIdx.x;
-  const int c0 = 64 * (int)blockIdx.y, nc = nrhs - c0 < 64 ? nrhs - c0 : 64;
   const int t = threadIdx.x, col = t & 63, comp = t >> 6;
   double x[16];
 #pragma unroll
   for (int s = 0; s < 16; ++s) {   // 16 rows in flight
     const int32_t at = q0 + s < slots ? atoms[q0 + s] : -1;
-    x[s] = at >= 0 && col < nc ? X[(3 * (int64_t)at + comp) * nrhs + c0 + col] : 0.0;
+    x[s] = at >= 0 && col < nc ? X[(3 * (int64_t)at + comp) * ld + col] : 0.0;
   }
 #pragma unroll
   for (int s = 0; s < 16; ++s) tile[s][comp][col] = x[s];
@@ -942,7 +943,7 @@ __global__ void __launch_bounds__(192) k_block_pack(int64_t slots, const int32_t
   const int s = t / 12, u = t % 12, k = u >> 2, c = u & 3;
   if (q0 + s >= slots) return;
   const int groups = (nc + kBlockCols - 1) / kBlockCols;
-  double *out = P + ((int64_t)(c0 / kBlockCols) * slots + q0 + s) * 12 + u;
+  double *out = P + (q0 + s) * 12 + u;
 #pragma unroll 4
   for (int g = 0; g < groups; ++g) out[12 * slots * (int64_t)g] = tile[s][k][kBlockCols * g + c];
 }
@@ -952,7 +953,7 @@ __global__ void __launch_bounds__(TA *G)
 k_matfree_tile_block(int64_t slots, const double *__restrict__ rec, const int32_t *__restrict__ atoms,
                      const int32_t *__restrict__ ulen, const uint32_t *__restrict__ ulist, int ucap, int umax,
                      const int2 *__restrict__ waves, const u32x4 *__restrict__ pairs, double bx, double by,
-                     double plus_i, const double *__restrict__ P, double *__restrict__ Y, int nrhs) {
+                     double plus_i, const double *__restrict__ P, double *__restrict__ Y, int64_t ld, int nc) {
   extern __shared__ double lds[];   // the union's entries (3 x C each), then its coordinates
   constexpr int NW = TA * G / 64, C = kBlockCols, NT = TA * G;
   double2 *sx = (double2 *)lds;
@@ -1046,7 +1047,7 @@ k_matfree_tile_block(int64_t slots, const double *__restrict__ rec, const int32_
   for (int k = 0; k < 3; ++k)
 #pragma unroll
     for (int c = 0; c < C; ++c) s[k][c] = group_sum<G>(s[k][c]);
-  if (at >= 0 && l < C && c0 + l < nrhs) {   // lane l of the atom's writes column c0 + l
+  if (at >= 0 && l < C && c0 + l < nc) {   // lane l of the atom's writes column c0 + l
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       double y = s[k][0], x = v[k][0];
@@ -1056,7 +1057,7 @@ k_matfree_tile_block(int64_t slots, const double *__restrict__ rec, const int32_
           y = s[k][c];
           x = v[k][c];
         }
-      Y[(3 * (int64_t)at + k) * nrhs + c0 + l] = y + plus_i * x;
+      Y[(3 * (int64_t)at + k) * ld + c0 + l] = y + plus_i * x;
     }
   }
 }
@@ -2155,7 +2156,8 @@ inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, 
 }
 
 int64_t inch_anm_tile_apply_work_size(int64_t ntile, int32_t tile, int32_t nrhs) {
-  return 12 * ntile * tile * ((nrhs + kBlockCols - 1) / kBlockCols);
+  const int32_t nc = nrhs < kBlockPass ? nrhs : kBlockPass;
+  return 12 * ntile * tile * ((nc + kBlockCols - 1) / kBlockCols);
 }
 
 inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lanes, const double *rec,
@@ -2168,23 +2170,23 @@ inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lan
   INCH_REQUIRE(inch_tile_shape_ok(tile, lanes), "inch_anm_matfree_tile_apply: no tile shape of %d atoms x %d lanes",
                tile, lanes);
   INCH_REQUIRE(umax >= 0 && umax <= ucap && ucap <= inch_tile_max_union(tile), "inch_anm_matfree_tile_apply: bad union");
-  INCH_REQUIRE(nrhs <= kBlockCols * 65535, "inch_anm_matfree_tile_apply: nrhs too large");
   const size_t lds = (size_t)umax * (24 * kBlockCols + 24);
   if (lds > kTileBlockLds)
     INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_matfree_tile_apply: a tile's %d neighbours exceed the LDS", umax);
   hipStream_t st = (hipStream_t)stream;
   const int64_t slots = ntile * tile;
-  k_block_pack<<<dim3((unsigned)((slots + 15) / 16), (unsigned)((nrhs + 63) / 64)), 192, 0, st>>>(slots, tile_atoms, x,
-                                                                                                 nrhs, work);
-  HIP_TRY(hipGetLastError());
-  const dim3 grid((unsigned)ntile, (unsigned)((nrhs + kBlockCols - 1) / kBlockCols));
+  for (int64_t c0 = 0; c0 < nrhs; c0 += kBlockPass) {
+    const int nc = (int)(nrhs - c0 < kBlockPass ? nrhs - c0 : kBlockPass);
+    k_block_pack<<<(unsigned)((slots + 15) / 16), 192, 0, st>>>(slots, tile_atoms, x + c0, nrhs, nc, work);
+    HIP_TRY(hipGetLastError());
+    const dim3 grid((unsigned)ntile, (unsigned)((nc + kBlockCols - 1) / kBlockCols));
 #define INCH_TB(TA, GG, PB)                                                                                         \
   do {                                                                                                              \
     HIP_TRY(hipFuncSetAttribute((const void *)k_matfree_tile_block<TA, GG, PB>,                                     \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                             \
     k_matfree_tile_block<TA, GG, PB><<<grid, TA * GG, lds, st>>>(slots, rec, tile_atoms, ulen, ulist, ucap, umax,   \
                                                                  (const int2 *)waves, (const u32x4 *)pairs, box_x,  \
-                                                                 box_y, plus_i, work, y, nrhs);                     \
+                                                                 box_y, plus_i, work, y + c0, nrhs, nc);            \
   } while (0)
 #define INCH_TILE_BLOCK(TA, GG)        \
   if (tile == TA && lanes == GG) {     \
@@ -2193,12 +2195,13 @@ inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lan
     else                               \
       INCH_TB(TA, GG, false);          \
   }
-  INCH_TILE_BLOCK(64, 8)
-  INCH_TILE_BLOCK(32, 16)
-  INCH_TILE_BLOCK(16, 32)
+    INCH_TILE_BLOCK(64, 8)
+    INCH_TILE_BLOCK(32, 16)
+    INCH_TILE_BLOCK(16, 32)
 #undef INCH_TILE_BLOCK
 #undef INCH_TB
-  HIP_TRY(hipGetLastError());
+    HIP_TRY(hipGetLastError());
+  }
   return INCH_OK;
 }
 

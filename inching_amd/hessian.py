@@ -252,12 +252,17 @@ class BlockHessian:
         if tiled and self.tiles() is not None and X.numel() and X.dtype == torch.float64 and Y.is_contiguous():
             # a later change of the module's line does not move products that took the tiles
             self.__dict__.setdefault("_apply_line", TILE_APPLY_TERMS)
-            # any shape of 3 n_atoms x r values, as the cluster layout's product takes (the periodic one: [3n] or [3n, r])
-            if self.images is None:
-                self.tiles().apply(X.reshape(self.shape[0], -1).contiguous(), Y.view(self.shape[0], -1), self.plus_i)
-            else:
-                self.tiles().apply(X.contiguous(), Y, self.plus_i)
-        elif self.images is not None:
+            try:
+                # any shape of 3 n_atoms x r values, as the cluster layout's product takes (the periodic one: [3n] or
+                # [3n, r])
+                if self.images is None:
+                    self.tiles().apply(X.reshape(self.shape[0], -1).contiguous(), Y.view(self.shape[0], -1), self.plus_i)
+                else:
+                    self.tiles().apply(X.contiguous(), Y, self.plus_i)
+                return Y
+            except torch.OutOfMemoryError:
+                pass          # no room for the packed columns: the other forms need none
+        if self.images is not None:
             ops.matfree_pbc(self.xyz, self.rowptr, self.col, self.images, self.box, self.plus_i, X.contiguous(), Y)
         elif self.clusters() is not None:
             ops.matfree_cl_apply(self.xyz, self.clusters(), self.plus_i, X.contiguous(), Y)

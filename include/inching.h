@@ -346,7 +346,8 @@ inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, 
                                     double plus_i, double *acc, void *stream);
 /* inch_anm_matfree_apply on the tile form: Y = (H + plus_i I) X for nrhs row-major right-hand
  * sides (X, Y float64 [3n, nrhs]) in the matrix's order; rec: records with the layout's
- * coordinates (their vector parts are not read); work: inch_anm_tile_apply_work_size doubles.
+ * coordinates (their vector parts are not read); work: inch_anm_tile_apply_work_size doubles (the
+ * packed entries of up to 64 columns, which are multiplied at a time).
  * INCH_ERR_CAPACITY when the longest union does not fit the LDS with four columns (over 1,365). */
 int64_t inch_anm_tile_apply_work_size(int64_t ntile, int32_t tile, int32_t nrhs);
 inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lanes, const double *rec,

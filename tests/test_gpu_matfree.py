@@ -53,3 +53,37 @@ def test_block_product_refuses_wrong_sizes_on_both_forms(cuda, monkeypatch):
             A.matfree(torch.randn(4500, 2, device="cuda"))
         with pytest.raises((ValueError, RuntimeError)):
             A.matfree(torch.empty(4500, 0, dtype=torch.float64, device="cuda"))
+
+
+def test_block_product_workspace_is_bounded(cuda):
+    """The tile form packs 64 columns at a time: its workspace does not grow past them, and columns around the passes
+    are those of the narrower products."""
+    from inching_amd._lib import call
+    print("case: workspace of a wide block", flush=True)
+    A = _matrix()
+    T = A.tiles()
+    size = [int(call("inch_anm_tile_apply_work_size", T.ntile, T.shape[0], r)) for r in (1, 4, 5, 64, 65, 1000)]
+    assert size == [12 * T.slots * g for g in (1, 1, 2, 16, 16, 16)]
+    X = torch.randn(4500, 197, dtype=torch.float64, device="cuda")
+    Y = torch.full_like(X, float("nan"))
+    T.apply(X, Y, 1.0)
+    for c0, c1 in ((0, 64), (64, 128), (128, 192), (192, 197), (60, 70)):
+        part = torch.empty(4500, c1 - c0, dtype=torch.float64, device="cuda")
+        T.apply(X[:, c0:c1].contiguous(), part, 1.0)
+        assert torch.equal(Y[:, c0:c1], part)
+
+
+def test_block_product_without_room_for_its_workspace(cuda, monkeypatch):
+    from inching_amd import hessian, ops
+    print("case: no room for the packed columns", flush=True)
+    A = _matrix()
+    X = torch.randn(4500, 5, dtype=torch.float64, device="cuda")
+    want = A.matfree(X)
+    monkeypatch.setattr(hessian, "TILE_APPLY_TERMS", 0)
+
+    def full(*args):
+        raise torch.OutOfMemoryError("no room")
+
+    assert A.tiles() is not None
+    monkeypatch.setattr(ops, "_scratch", full)
+    assert torch.equal(A.matfree(X), want)
