@@ -249,6 +249,9 @@ class BlockHessian:
         Y = torch.empty_like(X)
         columns = X.numel() // max(1, 3 * self.n_atoms)
         tiled = self.nnzb * columns >= self.__dict__.get("_apply_line", TILE_APPLY_TERMS)
+        # a capture takes what is laid out: nothing can be laid out inside it
+        fixed = torch.cuda.is_current_stream_capturing()
+        tiled = tiled and ("_tiles" in self.__dict__ or not fixed)
         if tiled and self.tiles() is not None and X.numel() and X.dtype == torch.float64 and Y.is_contiguous():
             # a later change of the module's line does not move products that took the tiles
             self.__dict__.setdefault("_apply_line", TILE_APPLY_TERMS)
@@ -264,7 +267,7 @@ class BlockHessian:
                 pass          # no room for the packed columns: the other forms need none
         if self.images is not None:
             ops.matfree_pbc(self.xyz, self.rowptr, self.col, self.images, self.box, self.plus_i, X.contiguous(), Y)
-        elif self.clusters() is not None:
+        elif ("_clusters" in self.__dict__ or not fixed) and self.clusters() is not None:
             ops.matfree_cl_apply(self.xyz, self.clusters(), self.plus_i, X.contiguous(), Y)
         else:
             ops.matfree_apply(self.xyz, self.rowptr, self.col, self.plus_i, X.contiguous(), Y)

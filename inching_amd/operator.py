@@ -53,6 +53,8 @@ class Operator:
                   and (lanes is None or int(lanes) // 1000 & 4) and A.slot_form() is not None)
         if lanes is not None:
             self.lanes = int(lanes)
+            if rec_ok:
+                A.clusters()      # asked for by name: laid out here, not inside a caller's capture
         elif rec_ok:
             self.lanes = None     # plain products only: picked when the first one comes
         elif tune:
@@ -96,9 +98,15 @@ class Operator:
             e1 = torch.cuda.Event(enable_timing=True)
             e0.record()
         if self.vals is None:
-            if self.lanes is None:
-                self.lanes = 161 if self.A.images is not None or self.A.clusters() is None else 6001
-            self.A.matfree_spmv(x, y, config=self.lanes, **epi)
+            code = self.lanes
+            if code is None:
+                # the cluster layout (0.3 ms at 1,201 atoms, 16 at 2.4M) is laid out by the first product that can use
+                # it; a capture cannot lay out anything, and takes the rows where no product came before
+                code = 161
+                if self.A.images is None and ("_clusters" in self.A.__dict__
+                                              or not torch.cuda.is_current_stream_capturing()):
+                    code = self.lanes = 161 if self.A.clusters() is None else 6001
+            self.A.matfree_spmv(x, y, config=code, **epi)
         else:
             ops.bsr_spmv(self.A.n_atoms, self.A.rowptr, self.A.col, self.vals, x, y, lanes=self.blanes,
                          col16=self.c16, **epi)
