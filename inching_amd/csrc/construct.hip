@@ -901,14 +901,16 @@ __device__ __forceinline__ uint32_t tile_images(const double *__restrict__ xyz, 
   return keep;
 }
 
-// cnt[i] = terms of atom i (entries times their images); one 16-lane group per row. Flags:
+// cnt[i] = terms of atom i (entries times their images); one 16-lane group per row. Flags: bit 0 more than `most`
+// terms (so many different ones are more than a union holds; repeated columns would exceed k_tile_fill's places),
 // bit 3 a column outside [0, n), bit 4 a distance outside the float32 seed's range.
 template <bool PBC>
 __global__ void __launch_bounds__(256) k_tile_count(int64_t n, const double *__restrict__ xyz,
                                                     const int64_t *__restrict__ rowptr,
                                                     const int32_t *__restrict__ col,
                                                     const uint16_t *__restrict__ images, double bx, double by,
-                                                    int32_t *__restrict__ cnt, int32_t *__restrict__ flags) {
+                                                    int most, int32_t *__restrict__ cnt,
+                                                    int32_t *__restrict__ flags) {
   const int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 4;
   const int lane = threadIdx.x & 15;
   if (i >= n) return;
@@ -925,7 +927,10 @@ __global__ void __launch_bounds__(256) k_tile_count(int64_t n, const double *__r
   if (far) atomicOr(flags, 16);
 #pragma unroll
   for (int off = 8; off > 0; off >>= 1) c += __shfl_xor(c, off, 16);
-  if (lane == 0) cnt[i] = c;
+  if (lane == 0) {
+    cnt[i] = c;
+    if (c > most) atomicOr(flags, 1);
+  }
 }
 
 // One 64-thread block per tile: its atoms by falling term count (ties by place), the slot of
@@ -1014,8 +1019,8 @@ __global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, con
   __shared__ uint32_t hkey[kTileHash];
   __shared__ uint16_t hpos[kTileHash];
   __shared__ uint32_t list[2048];
-  __shared__ uint32_t taken[4][64];      // a wave's places in use: at most ucap + G < 2,048
-  __shared__ uint16_t spills[4][1408];   // at most ucap
+  __shared__ uint32_t taken[4][64];      // a wave's places in use: at most 1,349 terms (k_tile_count) + G < 2,048
+  __shared__ uint16_t spills[4][1408];   // at most its terms
   __shared__ int s_n;
   const int64_t t = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -2011,10 +2016,13 @@ extern "C" inch_status inch_anm_tiles(int64_t n, const double *xyz, const int64_
   HIP_TRY(hipMalloc(&blocks.p, nw * sizeof(int32_t)));
   HIP_TRY(hipMalloc(&ptr.p, (nw + 1) * sizeof(int32_t)));
   const unsigned cg = (unsigned)((16 * n + bs - 1) / bs);
+  const int most = inch_tile_max_union(tile);
   if (images)
-    k_tile_count<true><<<cg, bs, 0, st>>>(n, xyz, rowptr, col, images, box_x, box_y, (int32_t *)cnt.p, (int32_t *)flags.p);
+    k_tile_count<true><<<cg, bs, 0, st>>>(n, xyz, rowptr, col, images, box_x, box_y, most, (int32_t *)cnt.p,
+                                          (int32_t *)flags.p);
   else
-    k_tile_count<false><<<cg, bs, 0, st>>>(n, xyz, rowptr, col, images, 0.0, 0.0, (int32_t *)cnt.p, (int32_t *)flags.p);
+    k_tile_count<false><<<cg, bs, 0, st>>>(n, xyz, rowptr, col, images, 0.0, 0.0, most, (int32_t *)cnt.p,
+                                           (int32_t *)flags.p);
   HIP_TRY(hipGetLastError());
   k_tile_slots<<<(unsigned)ntile, 64, 0, st>>>(tile, lanes, order, tile_start, (const int32_t *)cnt.p, tile_atoms, slot_of,
                                                (int32_t *)passes.p, (int32_t *)blocks.p);

@@ -318,7 +318,8 @@ inch_status inch_anm_matfree_rec(int64_t ncl, const double *rec_in, const double
  * (pair_blocks >= *blocks_out) and the arrays of the first call it writes ulen, ulist, pairs,
  * rec float64 [6 tile ntile] (records as inch_anm_records: coordinates, zero vector part) and
  * *umax_out, the longest union (order and tile_start are then unused). INCH_ERR_CAPACITY when a
- * union exceeds ucap, a squared distance lies outside 1e-30 .. 1e30 or the slots exceed the
+ * union exceeds ucap, a row has more than 65536 / 48 - tile terms (a repeated column counts as
+ * often as it is listed), a squared distance lies outside 1e-30 .. 1e30 or the slots exceed the
  * 32-bit record offsets; syncs. */
 inch_status inch_anm_tile_order(int64_t n, const double *xyz, double side, int32_t tile, int32_t *order,
                                 int32_t *tile_start, int64_t *ntile_out, void *stream);
