@@ -31,3 +31,40 @@ def test_tile_rows_with_repeated_columns(cuda, times):
     ops.matfree_apply(xyz, ip, ix, 1.0, x, want)
     # row sums of at most 1,309 terms
     assert float((y - want).abs().max()) <= 1e-11 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("shape", [(64, 8), (32, 16), (16, 32)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 1e300])
+def test_tile_entries_that_are_not_finite(cuda, shape, value):
+    """An entry that is not finite reaches its own row and its neighbours' alone, as in the record form: an atom without
+    neighbours that shares its wave with others has plus_i times it, not a NaN from the wave's empty passes."""
+    from inching_amd import ops
+    from inching_amd.hessian import RecordForm, build_hessian
+    print("case: entries of %g, tiles %s" % (value, shape), flush=True)
+    r = np.random.default_rng(6)
+    X = np.concatenate([r.uniform(0.0, 4.0, (21, 3)), [[2.0, 2.0, 100.0 + 30.0 * k] for k in range(6)],
+                        [[2.0, 2.0, 300.0], [3.0, 1.0, 303.0], [2.5, 1.5, 306.0]]])
+    n = len(X)
+    A = build_hessian(X, 8.0, precision=(), reorder=False)
+    T = ops.Tiles(A.xyz, A.rowptr, A.col, 50.0, shape)
+    F = RecordForm(A)
+    for at in (3, 21, 23, 26, 27, 29):       # in the cloud, without neighbours, in the chain of three
+        x = r.standard_normal((n, 3))
+        x[at, at % 3] = value
+        x = torch.as_tensor(x.reshape(-1), device="cuda")
+        out = []
+        for form in (T, F):
+            rec = form.buffers(1)[0]
+            ops.rec_pack(form.atoms, x, rec)
+            y = torch.empty(3 * form.slots, dtype=torch.float64, device="cuda")
+            u = torch.empty_like(x)
+            form.product(rec, None, None, 2.0, y=y)
+            ops.rec_unpack(form.atoms, y, u)
+            out.append(u.cpu().numpy())
+        a, b = out
+        kind = lambda v: np.where(np.isnan(v), 2, np.where(np.isinf(v), np.sign(v), 0))    # noqa: E731
+        assert np.array_equal(kind(a), kind(b)), at
+        ok = np.isfinite(b)
+        assert np.all(np.abs(a[ok] - b[ok]) <= 1e-12 * np.abs(b[ok]).max())
+        if 21 <= at < 27:
+            assert np.array_equal(a.reshape(n, 3)[at], 2.0 * x.cpu().numpy().reshape(n, 3)[at], equal_nan=True)
