@@ -1385,12 +1385,9 @@ extern "C" inch_status inch_cells_fill(int64_t n, double rc, const double *plan,
   INCH_REQUIRE(work_bytes >= k.bytes, "inch_cells_fill: work too small");
   hipStream_t st = (hipStream_t)stream;
   const inch_status s = cell_fill(n, rc, g, k, indptr, indices, st);
-  if (s != INCH_OK) return s;
-  if (sorted) {
-    k_sort_rows<<<(unsigned)n, 64, 0, st>>>(n, indptr, indices, k.longest);
-    HIP_TRY(hipGetLastError());
-  }
-  HIP_TRY(hipStreamSynchronize(st));   // the rows may be read on any stream, and work reused, from here on
+  if (s != INCH_OK || !sorted) return s;
+  k_sort_rows<<<(unsigned)n, 64, 0, st>>>(n, indptr, indices, k.longest);
+  HIP_TRY(hipGetLastError());
   return INCH_OK;
 }
 

@@ -353,16 +353,16 @@ def build_hessian(X, rc, plus_i=1.0, reorder=True, precision=("f32",), seed_orde
     xyz = _to_device_xyz(X, device)
     n = xyz.shape[0]
 
-    def pattern(xyz_, ascending=True):
+    def pattern(xyz_, ordering=False):
         if box is None:
-            return ops.neighbours(xyz_, rc, ascending=ascending) + (None,)
+            # the device ordering takes rows in any order, on this stream, and the renumbering sorts them
+            return ops.neighbours(xyz_, rc, ascending=not ordering, wait=not ordering) + (None,)
         return ops.neighbours_pbc(xyz_, rc, box, origin)
 
     comps = None                     # connected components (offsets in the RCM order)
     permuted = None                  # the search's CSR renumbered into the RCM order
     if reorder:
-        # the device ordering reads rows in any order, and the renumbering sorts them
-        indptr, indices, _ = pattern(xyz, ascending=rcm != "device")
+        indptr, indices, _ = pattern(xyz, ordering=rcm == "device")
         if rcm == "device":
             order_d, undo_d, comps = ops.rcm_device(indptr, indices, seed_order=seed_order, components=True)
             xyz = xyz[order_d.long()].contiguous()

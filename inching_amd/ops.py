@@ -121,10 +121,10 @@ def batch_head(n, maxleaf):
 
 # ---------------------------------------------------------------- device ----
 
-def neighbours(xyz, rc, stream=None, ascending=True):
+def neighbours(xyz, rc, stream=None, ascending=True, wait=True):
     """Cell-list neighbour CSR of device float64 coordinates [n,3] -> (indptr, indices).
     ``ascending=False`` leaves each row's columns in an unspecified order. Both are whole on
-    return, for any stream."""
+    return, for any stream; ``wait=False`` leaves that to the order of ``stream``."""
     require_gpu()
     _check_dev(xyz)
     if xyz.dtype != torch.float64 or xyz.dim() != 2 or xyz.shape[1] != 3:
@@ -147,6 +147,8 @@ def neighbours(xyz, rc, stream=None, ascending=True):
     call("inch_cells_count", n, P(xyz), rc, plan, P(work), size.value, P(indptr), C.byref(nnz), sp)
     indices = result(max(1, nnz.value), torch.int32)
     call("inch_cells_fill", n, rc, plan, P(work), size.value, P(indptr), P(indices), 1 if ascending else 0, sp)
+    if wait:
+        (torch.cuda.current_stream(dev) if stream is None else stream).synchronize()
     return indptr, indices[:nnz.value]
 
 

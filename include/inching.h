@@ -114,7 +114,7 @@ inch_status inch_neighbors_celllist(int64_t n, const double *xyz, double rc, int
  * *work_bytes: the scratch of the other two) and syncs; inch_cells_count writes indptr and
  * *nnz_out and syncs (INCH_ERR_CAPACITY for rows over 2048 entries); inch_cells_fill writes the
  * rows (indices int32 [nnz]) from the lists that inch_cells_count left in work, ascending when
- * sorted != 0, else in an unspecified order, and syncs. */
+ * sorted != 0, else in an unspecified order, without a sync: work stays in use until the stream has run them. */
 inch_status inch_cells_plan(int64_t n, const double *xyz, double rc, double *plan, int64_t *work_bytes,
                             double *scratch, void *stream);
 inch_status inch_cells_count(int64_t n, const double *xyz, double rc, const double *plan, void *work,
