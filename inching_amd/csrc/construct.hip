@@ -1912,6 +1912,9 @@ extern "C" inch_status inch_anm_tile_order(int64_t n, const double *xyz, double 
       hi[a] = std::max(hi[a], hp[b * 6 + 3 + a]);
     }
     if (nan || !std::isfinite(g.lo[a]) || !std::isfinite(hi[a])) INCH_FAIL(INCH_ERR_NAN, "inch_anm_tile_order: non-finite coordinates");
+    // an infinite span has no finite number of columns, however wide they are
+    if (a < 2 && !std::isfinite(hi[a] - g.lo[a]))
+      INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tile_order: the coordinates' span overflows");
   }
   // columns (coarser ones where their numbers would not fit 31 bits)
   for (double s = side;; s *= 2.0) {

@@ -68,3 +68,28 @@ def test_tile_entries_that_are_not_finite(cuda, shape, value):
         assert np.all(np.abs(a[ok] - b[ok]) <= 1e-12 * np.abs(b[ok]).max())
         if 21 <= at < 27:
             assert np.array_equal(a.reshape(n, 3)[at], 2.0 * x.cpu().numpy().reshape(n, 3)[at], equal_nan=True)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("far,status", [(1.5e308, -3), (float("inf"), -5), (float("nan"), -5), (1e300, 0)])
+def test_tile_order_of_far_coordinates(cuda, axis, far, status):
+    """Columns widen until their numbers fit; a span that overflows has none (and is refused; along z it only loses the
+    order), a huge one has."""
+    import ctypes as C
+    from inching_amd import ops
+    print("case: tile order, span %g along %d" % (far, axis), flush=True)
+    X = np.random.default_rng(1).uniform(0.0, 5.0, (40, 3))
+    X[0, axis], X[1, axis] = -far, far
+    xyz = torch.as_tensor(X, device="cuda")
+    order, start = (torch.empty(41, dtype=torch.int32, device="cuda") for _ in range(2))
+    nt = C.c_int64(0)
+    args = (40, ops.P(xyz), 6.0, 16, ops.P(order), ops.P(start), C.byref(nt), ops.stream_ptr())
+    if status and (status == -5 or axis < 2):
+        with pytest.raises(ops.InchingError) as e:
+            ops.call("inch_anm_tile_order", *args)
+        assert e.value.status == status
+        return
+    ops.call("inch_anm_tile_order", *args)
+    cut = start.cpu().numpy()[:nt.value + 1]
+    assert np.array_equal(np.sort(order.cpu().numpy()[:40]), np.arange(40))
+    assert cut[0] == 0 and cut[-1] == 40 and np.all(np.diff(cut) >= 1) and np.all(np.diff(cut) <= 16)
