@@ -1764,11 +1764,10 @@ namespace {
 constexpr int kBsrTileWords = 8192;   // 262,144 columns from the smallest to the largest of a tile's rows
 
 // A workgroup per tile of rows order[start[t]] ..: the columns its rows name, each once and ascending, as set bits
-// from the smallest column on. ulen[t] their number (raised into *umax; -1 there when their span exceeds the bits);
-// with FILL ulist[t ustride ..] these columns, uidx[b] the place of col[b] among them, and per place of the tile
+// from the smallest column on. Their number goes to *umax (0x7fffffff when their span exceeds the bits) and ulen[t];
+// with FILL ulist[t ustride ..] are these columns, uidx[b] the place of col[b] among them, and per place of the tile
 // slots: its row (-1: none), the row's length and first block (low and high half). LDS atomics and one
-// scan bound it; the lists of 150,000 atoms, their order and both
-// passes take 0.9 ms.
+// scan bound it; the lists of 150,000 atoms, their order and both passes take 0.9 ms.
 template <bool FILL>
 __global__ void __launch_bounds__(256) k_bsr_tiles(const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col,
                                                     const int32_t *__restrict__ order,
@@ -1823,13 +1822,12 @@ __global__ void __launch_bounds__(256) k_bsr_tiles(const int64_t *__restrict__ r
     __syncthreads();
   }
   const int total = sums[255];
+  if (tid == 0) atomicMax(umax, total);
   if constexpr (!FILL) {
-    if (tid == 0) {
-      ulen[t] = total;
-      atomicMax(umax, total);
-    }
+    if (tid == 0) ulen[t] = total;
     return;
   }
+  if (total > ustride) return;   // the caller's stride is of other rows: refused by *umax
   if (tid < tile) {
     const int row = r0 + tid < r1 ? order[r0 + tid] : -1;
     const int32_t len = row < 0 ? 0 : (int32_t)(rowptr[row + 1] - rowptr[row]);
@@ -1844,7 +1842,7 @@ __global__ void __launch_bounds__(256) k_bsr_tiles(const int64_t *__restrict__ r
   for (int i = w0; i < w1; ++i) {
     before[i] = (uint16_t)at;
     for (uint32_t m = bits[i]; m; m &= m - 1) {
-      if (at < ustride) ulist[(int64_t)t * ustride + at] = c0 + 32 * i + __ffs(m) - 1;
+      ulist[(int64_t)t * ustride + at] = c0 + 32 * i + __ffs(m) - 1;
       ++at;
     }
   }
@@ -1867,22 +1865,23 @@ extern "C" inch_status inch_bsr_tiles(int64_t n, const int64_t *rowptr, const in
   INCH_REQUIRE(ulist ? slots && uidx && tile > 0 && tile <= 256 && ustride > 0 && ustride <= 65536 : umax_out != nullptr,
                "inch_bsr_tiles: bad lists");
   hipStream_t st = (hipStream_t)stream;
-  if (ulist) {
-    k_bsr_tiles<true><<<(unsigned)ntile, 256, 0, st>>>(rowptr, col, order, tile_start, ustride, tile, slots, ulen, ulist,
-                                                       uidx, nullptr);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(st));   // the lists may be read on any stream from here on
-    return INCH_OK;
-  }
   DevBuf um;
   HIP_TRY(hipMalloc(&um.p, sizeof(int32_t)));
   HIP_TRY(hipMemsetAsync(um.p, 0, sizeof(int32_t), st));
-  k_bsr_tiles<false><<<(unsigned)ntile, 256, 0, st>>>(rowptr, col, order, tile_start, 0, tile, nullptr, ulen, nullptr,
-                                                      nullptr, (int32_t *)um.p);
+  if (ulist)
+    k_bsr_tiles<true><<<(unsigned)ntile, 256, 0, st>>>(rowptr, col, order, tile_start, ustride, tile, slots, ulen, ulist,
+                                                       uidx, (int32_t *)um.p);
+  else
+    k_bsr_tiles<false><<<(unsigned)ntile, 256, 0, st>>>(rowptr, col, order, tile_start, 0, tile, nullptr, ulen, nullptr,
+                                                        nullptr, (int32_t *)um.p);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(umax_out, um.p, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  if (*umax_out > 65536) INCH_FAIL(INCH_ERR_CAPACITY, "inch_bsr_tiles: a tile's columns span too far or are too many");
+  int32_t umax = 0;
+  HIP_TRY(hipMemcpyAsync(&umax, um.p, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));   // the lists may be read on any stream from here on
+  if (umax_out) *umax_out = umax;
+  if (umax > 65536) INCH_FAIL(INCH_ERR_CAPACITY, "inch_bsr_tiles: a tile's columns span too far or are too many");
+  if (ulist && umax > ustride)
+    INCH_FAIL(INCH_ERR_CAPACITY, "inch_bsr_tiles: a list of %d columns, room for %d", umax, ustride);
   return INCH_OK;
 }
 

@@ -217,10 +217,10 @@ inch_status inch_bsr_spmv16(int64_t n, const int64_t *rowptr, const int32_t *row
  * inch_anm_tile_order writes them (at most `tile` rows each). inch_bsr_tiles lists the columns of every tile's
  * rows, each once and ascending: with ulist NULL it writes ulen [ntile] and *umax_out, the longest list (both calls
  * sync; INCH_ERR_CAPACITY when a tile's columns span more than 262,144 or a list exceeds 65,536); with ulist
- * [ntile * ustride], ustride >= *umax_out, it writes the lists, uidx [nnz], the place of col[b] in its tile's list,
- * and slots [4 * ntile * tile] (16-byte aligned): per place of a tile its row (-1: none), the row's length and first
- * block. inch_bsr_spmv_tile: other arguments as inch_bsr_spmv; lanes 8, 16 or 32 per row, tile * lanes a multiple
- * of 64 up to 512; three values per list entry must fit 64 KiB (ustride of them). */
+ * [ntile * ustride], ustride >= *umax_out (else INCH_ERR_CAPACITY), it writes the lists, uidx [nnz], the place of
+ * col[b] in its tile's list, and slots [4 * ntile * tile] (16-byte aligned): per place of a tile its row (-1: none),
+ * the row's length and first block. inch_bsr_spmv_tile: other arguments as inch_bsr_spmv; lanes 8, 16 or 32 per row,
+ * tile * lanes a multiple of 64 up to 512; three values per list entry must fit 64 KiB (ustride of them). */
 inch_status inch_bsr_tiles(int64_t n, const int64_t *rowptr, const int32_t *col, int64_t ntile, const int32_t *order,
                            const int32_t *tile_start, int32_t tile, int32_t ustride, int32_t *slots, int32_t *ulen,
                            int32_t *ulist, uint16_t *uidx, int32_t *umax_out, void *stream);

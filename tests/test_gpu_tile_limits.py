@@ -93,3 +93,31 @@ def test_tile_order_of_far_coordinates(cuda, axis, far, status):
     cut = start.cpu().numpy()[:nt.value + 1]
     assert np.array_equal(np.sort(order.cpu().numpy()[:40]), np.arange(40))
     assert cut[0] == 0 and cut[-1] == 40 and np.all(np.diff(cut) >= 1) and np.all(np.diff(cut) <= 16)
+
+
+@pytest.mark.parametrize("case", ["stride", "span"])
+def test_row_tiles_refuse_lists_without_room(cuda, case):
+    """The second call finds longer lists, or columns further apart, than the first call's stride allows."""
+    import ctypes as C
+    from inching_amd import ops
+    print("case: row tiles, %s" % case, flush=True)
+    n = 40 if case == "stride" else 300000
+    i32 = dict(dtype=torch.int32, device="cuda")
+    per = 20 if case == "stride" else 2
+    rowptr = torch.arange(0, per * n + 1, per, dtype=torch.int64, device="cuda")
+    cols = torch.arange(20, **i32) if case == "stride" else torch.tensor([0, n - 1], **i32)
+    col = cols.repeat(n)
+    order, start = torch.arange(n, **i32), torch.arange(0, n + 1, 10, **i32)
+    nt = n // 10
+    slots, ulen, uidx = torch.empty(64 * nt, **i32), torch.empty(nt, **i32), torch.empty(per * n, dtype=torch.int16, device="cuda")
+    for stride, ok in ((19, False),) + (((20, True),) if case == "stride" else ()):
+        ulist = torch.empty(stride * nt, **i32)
+        args = (n, ops.P(rowptr), ops.P(col), nt, ops.P(order), ops.P(start), 16, stride, ops.P(slots), ops.P(ulen),
+                ops.P(ulist), ops.P(uidx), None, ops.stream_ptr())
+        if ok:
+            ops.call("inch_bsr_tiles", *args)
+            assert torch.equal(ulist.view(nt, 20), cols.repeat(nt, 1))
+        else:
+            with pytest.raises(ops.InchingError) as e:
+                ops.call("inch_bsr_tiles", *args)
+            assert e.value.status == -3
