@@ -1196,10 +1196,14 @@ struct DevBuf {
 
 }  // namespace
 
+// Out of device memory is INCH_ERR_CAPACITY (a caller may fall back on a form that needs less), and leaves no error
+// behind for the next launch to report.
 #define HIP_TRY(expr)                                                                      \
   do {                                                                                     \
     hipError_t _e = (expr);                                                                \
-    if (_e != hipSuccess) INCH_FAIL(INCH_ERR_HIP, "%s: %s", #expr, hipGetErrorString(_e)); \
+    if (_e == hipErrorOutOfMemory) (void)hipGetLastError();                                \
+    if (_e != hipSuccess)                                                                  \
+      INCH_FAIL(_e == hipErrorOutOfMemory ? INCH_ERR_CAPACITY : INCH_ERR_HIP, "%s: %s", #expr, hipGetErrorString(_e)); \
   } while (0)
 
 namespace {

@@ -158,30 +158,37 @@ class BlockHessian:
 
     def tiles(self):
         """Tile form of the matrix-free operator (ops.Tiles; built once, immutable), or None when
-        the neighbours of every tile shape's tiles exceed the LDS."""
+        the neighbours of every tile shape's tiles exceed the LDS, or without memory for it."""
         if "_tiles" not in self.__dict__:
-            self._tiles = None
+            tiles = None
             for shape in tile_shapes(self.n_atoms):
                 # cubes of the tile's atoms, at the density that the mean row length shows
                 side = self.rc * (shape[0] * 4.0 * np.pi / 3.0 / max(1.0, self.nnzb / self.n_atoms)) ** (1.0 / 3.0)
                 try:
-                    self._tiles = ops.Tiles(self.xyz, self.rowptr, self.col, side, shape, images=self.images,
-                                            box=self.box)
+                    tiles = ops.Tiles(self.xyz, self.rowptr, self.col, side, shape, images=self.images, box=self.box)
+                    break
+                except torch.OutOfMemoryError:
                     break
                 except ops.InchingError as e:
                     if e.status != ERR_CAPACITY:
-                        break
+                        raise
+            self._tiles = tiles       # once it is known: another thread builds its own until then
         return self._tiles
 
     def bsr_tiles(self):
         """Tiles of rows for the stored-block product (ops.BsrTiles; built once, immutable), or None
-        when a tile's columns are too many or too far apart."""
+        when a tile's columns are too many or too far apart, or without memory for them."""
         if "_bsr_tiles" not in self.__dict__:
             side = self.rc * (ops.BsrTiles.TILE * 4.0 * np.pi / 3.0 / max(1.0, self.nnzb / self.n_atoms)) ** (1.0 / 3.0)
+            tiles = None
             try:
-                self._bsr_tiles = ops.BsrTiles(self.xyz, self.rowptr, self.col, side)
-            except (ops.InchingError, torch.OutOfMemoryError):
-                self._bsr_tiles = None
+                tiles = ops.BsrTiles(self.xyz, self.rowptr, self.col, side)
+            except torch.OutOfMemoryError:
+                pass
+            except ops.InchingError as e:
+                if e.status != ERR_CAPACITY:
+                    raise
+            self._bsr_tiles = tiles
         return self._bsr_tiles
 
     def slot_form(self):

@@ -49,7 +49,7 @@ enum {
   INCH_OK = 0,
   INCH_ERR_INVALID = -1,      /* bad argument / shape */
   INCH_ERR_HIP = -2,          /* a HIP runtime call failed */
-  INCH_ERR_CAPACITY = -3,     /* an output buffer or a fixed capacity is too small */
+  INCH_ERR_CAPACITY = -3,     /* an output buffer, a fixed capacity or device memory (construction) is too small */
   INCH_ERR_NOT_CONVERGED = -4,
   INCH_ERR_NAN = -5
 };
