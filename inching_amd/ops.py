@@ -350,6 +350,10 @@ class Tiles:
         self.rec = torch.empty(6 * self.slots, dtype=torch.float64, device=dev)
         call("inch_anm_tiles", *head, ucap, P(self.ulen), P(self.ulist), P(self.pairs), max(1, blocks.value),
              P(self.rec), C.byref(umax), stream_ptr(stream))
+        # the lists at the longest union's stride (a quarter to three quarters of the room they were made in)
+        ucap, full = max(1, umax.value), self.ulist
+        self.ulist = full.view(nt, -1)[:, :ucap].contiguous()
+        torch.cuda.current_stream(dev).synchronize()     # whole on every stream from here on, as the others are
         self._lists = (P(self.ulen), P(self.ulist), ucap, umax.value, P(self.waves), P(self.pairs), bx, by)
 
     def buffers(self, count):

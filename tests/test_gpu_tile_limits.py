@@ -121,3 +121,10 @@ def test_row_tiles_refuse_lists_without_room(cuda, case):
             with pytest.raises(ops.InchingError) as e:
                 ops.call("inch_bsr_tiles", *args)
             assert e.value.status == -3
+
+
+def test_tile_lists_keep_no_spare_room(cuda):
+    from inching_amd.hessian import build_hessian
+    print("case: tile lists' stride", flush=True)
+    T = build_hessian(small_globule(2000, seed=3), 8.0, precision=()).tiles()
+    assert T.ulist.numel() == T.ntile * int(T.ulen.max())
