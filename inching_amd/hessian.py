@@ -33,6 +33,15 @@ def tile_shapes(n):
     return shapes[2 if n < 4000 else (1 if n < 40000 else 0):]
 
 
+def tile_slots(n):
+    """Most slots of the tiles of n atoms that pay. Every column of tiles ends in padding, and structures spread thin over
+    the columns (dimers in a plane, a chain along x) are mostly that: at 200,000 atoms 2.4 / 8.1 / 30 slots an atom
+    took 26 / 94 / 358 us a product, the record form 25 for all of them; a globule has 1.04. Up to 100,000 slots the
+    chip holds all tiles at once, and they are never slower (10,000 atoms in 81,000 slots 6.3 us, 6.9 on records;
+    20,000 in 162,000 slots 9.7 and 7.9)."""
+    return max(100000, int(2.5 * n))
+
+
 class RecordForm:
     """The record form of the cluster layout behind the interface of ``ops.Tiles``."""
 
@@ -158,16 +167,18 @@ class BlockHessian:
 
     def tiles(self):
         """Tile form of the matrix-free operator (ops.Tiles; built once, immutable), or None when
-        the neighbours of every tile shape's tiles exceed the LDS, or without memory for it."""
+        the neighbours of every tile shape's tiles exceed the LDS, where most of the slots would be padding, or without
+        memory for it."""
         if "_tiles" not in self.__dict__:
             tiles = None
             for shape in tile_shapes(self.n_atoms):
                 # cubes of the tile's atoms, at the density that the mean row length shows
                 side = self.rc * (shape[0] * 4.0 * np.pi / 3.0 / max(1.0, self.nnzb / self.n_atoms)) ** (1.0 / 3.0)
                 try:
-                    tiles = ops.Tiles(self.xyz, self.rowptr, self.col, side, shape, images=self.images, box=self.box)
+                    tiles = ops.Tiles(self.xyz, self.rowptr, self.col, side, shape, images=self.images, box=self.box,
+                                      most_slots=tile_slots(self.n_atoms))
                     break
-                except torch.OutOfMemoryError:
+                except (ops.SparseTiles, torch.OutOfMemoryError):     # (smaller tiles pad less and take longer)
                     break
                 except ops.InchingError as e:
                     if e.status != ERR_CAPACITY:

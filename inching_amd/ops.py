@@ -317,12 +317,16 @@ def matfree_rec(rec_in, rec_z, rec_out, cl_ptr, rec_entries, plus_i, s1=1.0, c0=
          float(plus_i), float(s1), float(c0), float(c2), P(acc), float(mu), 1 if xcd else 0, stream_ptr(stream))
 
 
+class SparseTiles(InchingError):
+    """More slots than a Tiles' caller allows: most would be padding."""
+
+
 class Tiles:
     """Tile form of the matrix-free operator (inch_anm_tiles): the slots' atoms, every tile's
     union of neighbours and its atoms' lists into it. Holds the arrays and the launch's fixed
     arguments; the record buffers of a recurrence are the caller's (``buffers``)."""
 
-    def __init__(self, xyz, rowptr, col, side, shape, images=None, box=None, stream=None):
+    def __init__(self, xyz, rowptr, col, side, shape, images=None, box=None, stream=None, most_slots=None):
         require_gpu()
         _check_dev(xyz, rowptr, col)
         n, dev = xyz.shape[0], xyz.device
@@ -335,6 +339,8 @@ class Tiles:
         call("inch_anm_tile_order", n, P(xyz), float(side), tile, P(order), P(start), C.byref(nt), stream_ptr(stream))
         nt = nt.value
         self.shape, self.ntile, self.slots, self.nd = (tile, lanes), nt, nt * tile, 3 * n
+        if most_slots is not None and self.slots > most_slots:
+            raise SparseTiles("inch_anm_tile_order", -3, "%d slots for %d atoms" % (self.slots, n))
         ucap = 65536 // 48 - tile
         self.atoms = torch.empty(self.slots, **i32)
         slot_of = torch.empty(n, **i32)

@@ -128,3 +128,31 @@ def test_tile_lists_keep_no_spare_room(cuda):
     print("case: tile lists' stride", flush=True)
     T = build_hessian(small_globule(2000, seed=3), 8.0, precision=()).tiles()
     assert T.ulist.numel() == T.ntile * int(T.ulen.max())
+
+
+@pytest.mark.parametrize("what", ["dimers", "chain", "globule", "few_dimers"])
+def test_tiles_that_would_be_padding_are_left_out(cuda, what):
+    """Structures spread thin keep the record form; dense ones, and as many slots as the chip holds at once, the tiles."""
+    from inching_amd import chebyshev as CH
+    from inching_amd.hessian import RecordForm, build_hessian
+    from inching_amd.operator import Operator
+    print("case: sparse structure %s" % what, flush=True)
+    r = np.random.default_rng(2)
+    if what == "globule":
+        X = small_globule(4000, seed=3)
+    elif what == "chain":
+        t = 3.8 * np.arange(20000)
+        X = np.stack([t, np.sin(t), np.cos(t)], 1)
+    else:
+        k = 5000 if what == "dimers" else 500
+        d = r.uniform(0.0, 1.0, (k, 3)) * [80.0 * k ** 0.5, 80.0 * k ** 0.5, 5.0]
+        X = np.concatenate([d, d + 1.5])
+    A = build_hessian(X, 8.0, precision=())
+    assert (A.tiles() is None) == (what in ("dimers", "chain"))
+    assert isinstance(A.slot_form(), RecordForm) == (A.tiles() is None)
+    v = torch.randn(A.shape[0], dtype=torch.float64, device="cuda")
+    a, b = torch.empty_like(v), torch.empty_like(v)
+    pol = CH.design_filter(1.0, 3.0, (1.0, 80.0), 5120, 5, 0.7)
+    Operator(A, "mf64", pol=pol).apply(v, a)
+    Operator(A, "mf64", pol=pol, records=False).apply(v, b)
+    assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
