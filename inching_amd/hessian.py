@@ -34,8 +34,8 @@ def tile_shapes(n):
 
 
 def tile_slots(n):
-    """Most slots of the tiles of n atoms that pay. Every column of tiles ends in padding, and structures spread thin over
-    the columns (dimers in a plane, a chain along x) are mostly that: at 200,000 atoms 2.4 / 8.1 / 30 slots an atom
+    """Most slots of the tiles of n atoms that pay. Every column of tiles ends in padding, and structures spread thin
+    over the columns (dimers in a plane, a chain along x) are mostly that: at 200,000 atoms 2.4 / 8.1 / 30 slots an atom
     took 26 / 94 / 358 us a product, the record form 25 for all of them; a globule has 1.04. Up to 100,000 slots the
     chip holds all tiles at once, and they are never slower (10,000 atoms in 81,000 slots 6.3 us, 6.9 on records;
     20,000 in 162,000 slots 9.7 and 7.9)."""
@@ -262,22 +262,25 @@ class BlockHessian:
             raise ValueError("config %d asks for 16-bit column offsets, which this matrix cannot use" % config)
         ops.matfree_spmv(self.xyz, self.rowptr, self.col, self.plus_i, x, y, config=abi, col16=c16, **epi)
 
+    def _at_hand(self, layout):
+        """A layout is there, or can be made: a capture takes what there is, nothing can be laid out inside it."""
+        return layout in self.__dict__ or not torch.cuda.is_current_stream_capturing()
+
     def matfree(self, X):
         """FP64 (H + PlusI I) X recomputed from coordinates (X [3n] or [3n, r])."""
         Y = torch.empty_like(X)
         columns = X.numel() // max(1, 3 * self.n_atoms)
-        tiled = self.nnzb * columns >= self.__dict__.get("_apply_line", TILE_APPLY_TERMS)
-        # a capture takes what is laid out: nothing can be laid out inside it
-        fixed = torch.cuda.is_current_stream_capturing()
-        tiled = tiled and ("_tiles" in self.__dict__ or not fixed)
-        if tiled and self.tiles() is not None and X.numel() and X.dtype == torch.float64 and Y.is_contiguous():
+        tiled = (self.nnzb * columns >= self.__dict__.get("_apply_line", TILE_APPLY_TERMS) and X.numel() > 0
+                 and X.dtype == torch.float64 and Y.is_contiguous())
+        if tiled and self._at_hand("_tiles") and self.tiles() is not None:
             # a later change of the module's line does not move products that took the tiles
             self.__dict__.setdefault("_apply_line", TILE_APPLY_TERMS)
             try:
                 # any shape of 3 n_atoms x r values, as the cluster layout's product takes (the periodic one: [3n] or
                 # [3n, r])
                 if self.images is None:
-                    self.tiles().apply(X.reshape(self.shape[0], -1).contiguous(), Y.view(self.shape[0], -1), self.plus_i)
+                    nd = self.shape[0]
+                    self.tiles().apply(X.reshape(nd, -1).contiguous(), Y.view(nd, -1), self.plus_i)
                 else:
                     self.tiles().apply(X.contiguous(), Y, self.plus_i)
                 return Y
@@ -285,7 +288,7 @@ class BlockHessian:
                 pass          # no room for the packed columns: the other forms need none
         if self.images is not None:
             ops.matfree_pbc(self.xyz, self.rowptr, self.col, self.images, self.box, self.plus_i, X.contiguous(), Y)
-        elif ("_clusters" in self.__dict__ or not fixed) and self.clusters() is not None:
+        elif self._at_hand("_clusters") and self.clusters() is not None:
             ops.matfree_cl_apply(self.xyz, self.clusters(), self.plus_i, X.contiguous(), Y)
         else:
             ops.matfree_apply(self.xyz, self.rowptr, self.col, self.plus_i, X.contiguous(), Y)

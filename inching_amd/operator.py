@@ -103,8 +103,7 @@ class Operator:
                 # the cluster layout (0.3 ms at 1,201 atoms, 16 at 2.4M) is laid out by the first product that can use
                 # it; a capture cannot lay out anything, and takes the rows where no product came before
                 code = 161
-                if self.A.images is None and ("_clusters" in self.A.__dict__
-                                              or not torch.cuda.is_current_stream_capturing()):
+                if self.A.images is None and self.A._at_hand("_clusters"):
                     code = self.lanes = 161 if self.A.clusters() is None else 6001
             self.A.matfree_spmv(x, y, config=code, **epi)
         else:
