@@ -124,6 +124,8 @@ __global__ void __launch_bounds__(256) k_bsr_spmv(int64_t n, const int64_t *__re
   }
 }
 
+constexpr int kBsrTileLanes = 32;
+
 // The product on tiles of rows (inch_bsr_tiles): a workgroup takes a tile of neighbouring atoms, gathers the x
 // entries that its rows meet once into LDS, and the rows read them from there by 16-bit places (as much index
 // traffic as 16-bit columns). What bounded k_bsr_spmv was the gather through L1: 0.8 lines from L2 per block, while
@@ -132,9 +134,9 @@ __global__ void __launch_bounds__(256) k_bsr_spmv(int64_t n, const int64_t *__re
 // and 96 against 123 in float64 at 50,000 atoms (0.42 GB). What is left above the stream: rows of a tile lie
 // apart in memory (rows one after the other took 131 and 79), and the gather (10 and 3). Tiles of 8, 32 and 64
 // rows took 158, 155 and 163; tiles of consecutive rows share few entries (1,745 per 16 rows) and took 179.
-// G lanes per row; U blocks per lane at a time, all of their loads in flight, the first ones while x is gathered
+// 32 lanes per row; U blocks per lane at a time, all of their loads in flight, the first ones while x is gathered
 // (U = 4 takes 162 and 108: fewer waves).
-template <typename MT, typename VT, int G>
+template <typename MT, typename VT>
 __global__ void __launch_bounds__(512) k_bsr_spmv_tile(int64_t n, const int4 *__restrict__ slots, int ustride,
                                                         const int32_t *__restrict__ ulen,
                                                         const int32_t *__restrict__ ulist,
@@ -144,7 +146,7 @@ __global__ void __launch_bounds__(512) k_bsr_spmv_tile(int64_t n, const int4 *__
                                                         MT c2, VT *__restrict__ acc, MT mu,
                                                         const double *__restrict__ Q,
                                                         const double *__restrict__ qcoef, int mq) {
-  constexpr int U = 2;
+  constexpr int U = 2, G = kBsrTileLanes;
   extern __shared__ __align__(16) char tile_x[];
   MT *xs = (MT *)tile_x;
   const int64_t t = xcd_block(true);
@@ -1523,7 +1525,6 @@ constexpr int kDcgsChunks = 512;     // most chunks of the dot products
 constexpr int kDcgsChunk = 1024;     // fewest dofs of one: two pairs per thread
 constexpr int kDcgsUpdates = 1024;   // most workgroups of the update
 constexpr int64_t dcgs2_words(int64_t J) { return kDcgsChunks * 2 * J + 4 * J + kDcgsUpdates; }
-constexpr int64_t kDcgsNarrow = 524288;
 
 // part[c*2J + j] = V_j . u (j < J), part[c*2J + J + j] = V_j . w (j < J), w = V[J-1], over dofs
 // [c per, (c + 1) per), 8 rows per workgroup. Memory or, for short
@@ -1894,35 +1895,24 @@ inch_status inch_bsr_spmv_tile(int64_t n, int64_t ntile, int32_t tile, const int
                "inch_bsr_spmv_tile: bad args");
   INCH_REQUIRE(!qcoef || (Q && m_q > 0), "inch_bsr_spmv_tile: qcoef needs Q and m_q > 0");
   INCH_REQUIRE(x != y, "inch_bsr_spmv_tile: x and y must not alias");
-  INCH_REQUIRE(tile > 0 && lanes > 0 && tile <= 512 / lanes && tile * lanes % 64 == 0 && ustride > 0,
-               "inch_bsr_spmv_tile: bad tile");
+  INCH_REQUIRE(lanes == kBsrTileLanes, "inch_bsr_spmv_tile: lanes must be %d (got %d)", kBsrTileLanes, lanes);
+  INCH_REQUIRE(tile > 0 && tile <= 512 / lanes && tile * lanes % 64 == 0 && ustride > 0, "inch_bsr_spmv_tile: bad tile");
   const size_t lds = 3 * (size_t)ustride * (mdt == INCH_F64 ? 8 : 4);
   INCH_REQUIRE(lds <= 65536, "inch_bsr_spmv_tile: the union exceeds the LDS");
   hipStream_t st = (hipStream_t)stream;
-#define INCH_TILE_CASE(MT, VT, G)                                                                                      \
-  case G:                                                                                                              \
-    k_bsr_spmv_tile<MT, VT, G><<<(unsigned)ntile, tile * G, lds, st>>>(                                                \
-        n, (const int4 *)slots, ustride, ulen, ulist, uidx, (const MT *)vals, (const VT *)x, (VT *)y, (MT)s1, (MT)c0,  \
-        (const VT *)z, (MT)c2, (VT *)acc, (MT)mu, Q, qcoef, m_q);                                                      \
-    break;
-#define INCH_TILE_TYPES(MT, VT)                                                                                        \
-  switch (lanes) {                                                                                                     \
-    INCH_TILE_CASE(MT, VT, 8)                                                                                          \
-    INCH_TILE_CASE(MT, VT, 16)                                                                                         \
-    INCH_TILE_CASE(MT, VT, 32)                                                                                         \
-    default: INCH_FAIL(INCH_ERR_INVALID, "inch_bsr_spmv_tile: lanes must be 8, 16 or 32 (got %d)", lanes);             \
-  }
-  if (mdt == INCH_F32 && vdt == INCH_F32) {
-    INCH_TILE_TYPES(float, float)
-  } else if (mdt == INCH_F32 && vdt == INCH_F64) {
-    INCH_TILE_TYPES(float, double)
-  } else if (mdt == INCH_F64 && vdt == INCH_F64) {
-    INCH_TILE_TYPES(double, double)
-  } else {
+#define INCH_BSR_TILE(MT, VT)                                                                                        \
+  k_bsr_spmv_tile<MT, VT><<<(unsigned)ntile, tile * lanes, lds, st>>>(                                               \
+      n, (const int4 *)slots, ustride, ulen, ulist, uidx, (const MT *)vals, (const VT *)x, (VT *)y, (MT)s1, (MT)c0,  \
+      (const VT *)z, (MT)c2, (VT *)acc, (MT)mu, Q, qcoef, m_q)
+  if (mdt == INCH_F32 && vdt == INCH_F32)
+    INCH_BSR_TILE(float, float);
+  else if (mdt == INCH_F32 && vdt == INCH_F64)
+    INCH_BSR_TILE(float, double);
+  else if (mdt == INCH_F64 && vdt == INCH_F64)
+    INCH_BSR_TILE(double, double);
+  else
     INCH_FAIL(INCH_ERR_INVALID, "inch_bsr_spmv_tile: unsupported dtype pair (%d,%d)", mdt, vdt);
-  }
-#undef INCH_TILE_TYPES
-#undef INCH_TILE_CASE
+#undef INCH_BSR_TILE
   HIP_TRY(hipGetLastError());
   return INCH_OK;
 }
@@ -2192,9 +2182,9 @@ inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lan
   INCH_REQUIRE(inch_tile_shape_ok(tile, lanes), "inch_anm_matfree_tile_apply: no tile shape of %d atoms x %d lanes",
                tile, lanes);
   INCH_REQUIRE(umax >= 0 && umax <= ucap && ucap <= inch_tile_max_union(tile), "inch_anm_matfree_tile_apply: bad union");
+  // the longest union that a tile may have (16 atoms: 65536 / 48 - 16) fits the LDS
+  static_assert((65536 / 48 - 16) * (24 * kBlockCols + 24) <= kTileBlockLds, "kBlockCols");
   const size_t lds = (size_t)umax * (24 * kBlockCols + 24);
-  if (lds > kTileBlockLds)
-    INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_matfree_tile_apply: a tile's %d neighbours exceed the LDS", umax);
   hipStream_t st = (hipStream_t)stream;
   const int64_t slots = ntile * tile;
   for (int64_t c0 = 0; c0 < nrhs; c0 += kBlockPass) {

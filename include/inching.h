@@ -219,8 +219,8 @@ inch_status inch_bsr_spmv16(int64_t n, const int64_t *rowptr, const int32_t *row
  * sync; INCH_ERR_CAPACITY when a tile's columns span more than 262,144 or a list exceeds 65,536); with ulist
  * [ntile * ustride], ustride >= *umax_out (else INCH_ERR_CAPACITY), it writes the lists, uidx [nnz], the place of
  * col[b] in its tile's list, and slots [4 * ntile * tile] (16-byte aligned): per place of a tile its row (-1: none),
- * the row's length and first block. inch_bsr_spmv_tile: other arguments as inch_bsr_spmv; lanes 8, 16 or 32 per row,
- * tile * lanes a multiple of 64 up to 512; three values per list entry must fit 64 KiB (ustride of them). */
+ * the row's length and first block. inch_bsr_spmv_tile: other arguments as inch_bsr_spmv; 32 lanes per row, tile even
+ * and at most 16; three values per list entry must fit 64 KiB (ustride of them). */
 inch_status inch_bsr_tiles(int64_t n, const int64_t *rowptr, const int32_t *col, int64_t ntile, const int32_t *order,
                            const int32_t *tile_start, int32_t tile, int32_t ustride, int32_t *slots, int32_t *ulen,
                            int32_t *ulist, uint16_t *uidx, int32_t *umax_out, void *stream);
@@ -348,8 +348,7 @@ inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, 
 /* inch_anm_matfree_apply on the tile form: Y = (H + plus_i I) X for nrhs row-major right-hand
  * sides (X, Y float64 [3n, nrhs]) in the matrix's order; rec: records with the layout's
  * coordinates (their vector parts are not read); work: inch_anm_tile_apply_work_size doubles (the
- * packed entries of up to 64 columns, which are multiplied at a time).
- * INCH_ERR_CAPACITY when the longest union does not fit the LDS with four columns (over 1,365). */
+ * packed entries of up to 64 columns, which are multiplied at a time). */
 int64_t inch_anm_tile_apply_work_size(int64_t ntile, int32_t tile, int32_t nrhs);
 inch_status inch_anm_matfree_tile_apply(int64_t ntile, int32_t tile, int32_t lanes, const double *rec,
                                         const int32_t *tile_atoms, const int32_t *ulen, const uint32_t *ulist,
