@@ -111,3 +111,14 @@ def test_fused_layer_equals_its_parts(cuda, Din, Dout):
         _call("inch_gnn_aggregate", N, Din, ip, ix, dagg, 0, back, 0, 1)
         for x, y in zip(got, (dh + back, dWs, dWn, db)):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 4096 * 256 + 3])
+def test_relu_backward(cuda, n):
+    from inching_amd import ops
+    print("case: relu backward %d" % n, flush=True)
+    pre, dy = torch.randn(n, device="cuda"), torch.randn(n, device="cuda")
+    pre[0] = 0.0
+    out = torch.full((n,), float("nan"), device="cuda")
+    ops.call("inch_gnn_relu_bwd", n, ops.P(pre), ops.P(dy), ops.P(out), ops.stream_ptr())
+    assert torch.equal(out, torch.where(pre > 0, dy, torch.zeros_like(dy)))

@@ -93,3 +93,36 @@ def test_pairs_at_the_cutoff_across_rounded_cells(cuda, rc, lo, step, axis):
     ip, ix = ops.neighbours(torch.as_tensor(X, device="cuda"), rc)
     for i, row in enumerate(_rows(ip, ix)):
         assert np.array_equal(row, np.nonzero(want[i])[0]), i
+
+
+@pytest.mark.parametrize("case", ["one", "run_edge_33", "one_cell_two_stages", "globule"])
+def test_one_call_search_equals_the_steps(cuda, case):
+    """inch_neighbors_celllist: the count pass, the fill pass, a buffer one short, and rows over 2,048 entries."""
+    import ctypes as C
+    from inching_amd import ops
+    print("case: one-call search %s" % case, flush=True)
+    X = CASES[case](np.random.default_rng(8))
+    xyz = torch.as_tensor(X, device="cuda")
+    n = len(X)
+    want = ops.neighbours(xyz, 8.0)
+    ip = torch.full((n + 1,), -1, dtype=torch.int64, device="cuda")
+    nnz = C.c_int64(-1)
+    call = lambda ix, cap: ops.call("inch_neighbors_celllist", n, ops.P(xyz), 8.0, ops.P(ip), ops.P(ix), cap,    # noqa: E731
+                                    C.byref(nnz), ops.stream_ptr())
+    call(None, 0)
+    assert nnz.value == want[1].numel() and torch.equal(ip, want[0])
+    ix = torch.full((nnz.value + 1,), -7, dtype=torch.int32, device="cuda")
+    with pytest.raises(ops.InchingError) as e:
+        call(ix, nnz.value - 1)
+    assert e.value.status == -3 and bool((ix == -7).all())
+    call(ix, nnz.value)
+    assert torch.equal(ix[:-1], want[1]) and int(ix[-1]) == -7
+    if case == "one":
+        xyz, n = torch.rand((2049, 3), dtype=torch.float64, device="cuda"), 2049
+        ip = torch.empty(n + 1, dtype=torch.int64, device="cuda")
+        call(None, 0)
+        assert nnz.value == 2049 * 2049
+        ix = torch.empty(nnz.value, dtype=torch.int32, device="cuda")
+        with pytest.raises(ops.InchingError) as e:
+            call(ix, nnz.value)
+        assert e.value.status == -3
