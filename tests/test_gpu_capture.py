@@ -4,14 +4,14 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import small_globule
+from inching_amd.synth import globule
 
 pytestmark = pytest.mark.gpu
 
 
 def _matrix():
     from inching_amd.hessian import build_hessian
-    return build_hessian(small_globule(1500, seed=7), 8.0, precision=())
+    return build_hessian(globule(1500, seed=7), 8.0, precision=())
 
 
 def _replays(graph, x, y, reference):

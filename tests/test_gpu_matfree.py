@@ -2,14 +2,14 @@
 import pytest
 import torch
 
-from helpers import small_globule
+from inching_amd.synth import globule
 
 pytestmark = pytest.mark.gpu
 
 
 def _matrix(n=1500, seed=3):
     from inching_amd.hessian import build_hessian
-    return build_hessian(small_globule(n, seed=seed), 8.0, precision=())
+    return build_hessian(globule(n, seed=seed), 8.0, precision=())
 
 
 @pytest.mark.parametrize("columns", [1, 7])

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import small_globule
+from inching_amd.synth import globule
 
 pytestmark = pytest.mark.gpu
 
@@ -59,7 +59,7 @@ def test_neighbours_wait_for_a_reused_block(cuda):
 def test_build_without_ordering_on_another_stream(cuda):
     from inching_amd.hessian import build_hessian
     print("case: build_hessian on one stream, product on another", flush=True)
-    X = small_globule(3000, seed=4)
+    X = globule(3000, seed=4)
     x = torch.randn(9000, dtype=torch.float64, device="cuda")
     ref = build_hessian(X, 8.0, reorder=False, precision=()).matfree(x)
     s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
@@ -78,7 +78,7 @@ def test_block_product_keeps_its_scratch(cuda, monkeypatch):
     from inching_amd import ops
     from inching_amd.hessian import build_hessian
     print("case: block product's scratch", flush=True)
-    A = build_hessian(small_globule(3000, seed=5), 8.0, precision=())
+    A = build_hessian(globule(3000, seed=5), 8.0, precision=())
     T = A.tiles()
     X = torch.randn(9000, 16, dtype=torch.float64, device="cuda")
     Y, want = torch.empty_like(X), torch.empty_like(X)
@@ -109,7 +109,7 @@ def test_filter_on_another_stream_than_its_operator(cuda):
     from inching_amd.hessian import build_hessian
     from inching_amd.operator import Operator
     print("case: operator made on one stream, applied on another", flush=True)
-    A = build_hessian(small_globule(3000, seed=5), 8.0, precision=())
+    A = build_hessian(globule(3000, seed=5), 8.0, precision=())
     pol = CH.design_filter(1.0, 3.0, (1.0, 80.0), 5120, 5, 0.7)
     v = torch.randn(9000, dtype=torch.float64, device="cuda")
     u, want = torch.empty_like(v), torch.empty_like(v)

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import small_globule
+from inching_amd.synth import globule
 
 pytestmark = pytest.mark.gpu
 
@@ -15,7 +15,7 @@ def test_tile_rows_with_repeated_columns(cuda, times):
     from inching_amd import ops
     print("case: columns repeated %d times" % times, flush=True)
     n = 120
-    xyz = torch.as_tensor(small_globule(n, seed=2), device="cuda")
+    xyz = torch.as_tensor(globule(n, seed=2), device="cuda")
     rows = [np.repeat(np.arange(n), times) if i % 7 == 0 else np.arange(n) for i in range(n)]
     ip = torch.as_tensor(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), device="cuda")
     ix = torch.as_tensor(np.concatenate(rows).astype(np.int32), device="cuda")
@@ -126,7 +126,7 @@ def test_row_tiles_refuse_lists_without_room(cuda, case):
 def test_tile_lists_keep_no_spare_room(cuda):
     from inching_amd.hessian import build_hessian
     print("case: tile lists' stride", flush=True)
-    T = build_hessian(small_globule(2000, seed=3), 8.0, precision=()).tiles()
+    T = build_hessian(globule(2000, seed=3), 8.0, precision=()).tiles()
     assert T.ulist.numel() == T.ntile * int(T.ulen.max())
 
 
@@ -139,7 +139,7 @@ def test_tiles_that_would_be_padding_are_left_out(cuda, what):
     print("case: sparse structure %s" % what, flush=True)
     r = np.random.default_rng(2)
     if what == "globule":
-        X = small_globule(4000, seed=3)
+        X = globule(4000, seed=3)
     elif what == "chain":
         t = 3.8 * np.arange(20000)
         X = np.stack([t, np.sin(t), np.cos(t)], 1)
