@@ -2152,7 +2152,7 @@ inch_status inch_anm_chebyshev_tile(int64_t ntile, int32_t tile, int32_t lanes, 
                                     const int32_t *ulen, const uint32_t *ulist, int32_t ucap, int32_t umax,
                                     const int32_t *waves, const uint16_t *pairs, double box_x, double box_y,
                                     double plus_i, double *acc, void *stream) {
-  INCH_REQUIRE(degree >= 1 && mu && dd != 0.0 && acc && rec0 && rec1 && rec2, "inch_anm_chebyshev_tile: bad args");
+  INCH_REQUIRE(degree >= 0 && mu && dd != 0.0 && acc && rec0 && rec1 && rec2, "inch_anm_chebyshev_tile: bad args");
   double *cur = rec0, *prev = nullptr, *out = rec1, *spare = rec2;
   for (int32_t k = 1; k <= degree; ++k) {
     const inch_status s =

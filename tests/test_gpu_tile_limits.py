@@ -156,3 +156,23 @@ def test_tiles_that_would_be_padding_are_left_out(cuda, what):
     Operator(A, "mf64", pol=pol).apply(v, a)
     Operator(A, "mf64", pol=pol, records=False).apply(v, b)
     assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("degree", [0, 1, 2])
+@pytest.mark.parametrize("shift", [0.0, -40.0])
+def test_filters_of_the_smallest_degrees(cuda, degree, shift):
+    """A filter without a product is its constant, on the tiles as in the matrix's order."""
+    from types import SimpleNamespace
+    from inching_amd.hessian import build_hessian, rigid_body_basis
+    from inching_amd.operator import Operator
+    print("case: filter of degree %d, shift %g" % (degree, shift), flush=True)
+    A = build_hessian(globule(300, seed=3), 8.0, precision=())
+    pol = SimpleNamespace(AdjustedCoefficients=np.array([0.3, -0.7, 0.2]), AdjustedDegree=degree, cc=40.0, dd=39.0)
+    Q = rigid_body_basis(A.xyz)
+    v = torch.randn(900, dtype=torch.float64, device="cuda")
+    a, b = torch.empty_like(v), torch.empty_like(v)
+    op = Operator(A, "mf64", pol=pol, Q=Q, shift=shift)
+    assert op.rec is A.tiles() is not None
+    op.apply(v, a)
+    Operator(A, "mf64", pol=pol, Q=Q, shift=shift, records=False).apply(v, b)
+    assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
