@@ -267,7 +267,7 @@ class KPMMoments:
     def _step(self):
         k = len(self.mom)
         if self.precision == "mf64":
-            W = self.A.matfree(self.tcur)
+            W = getattr(self.A, "_matfree", self.A.matfree)(self.tcur)
         else:
             W = self.A.matmat(self.tcur, precision=self.precision)
         self.n_spmv += self.tcur.shape[1]

@@ -268,13 +268,18 @@ class BlockHessian:
 
     def matfree(self, X):
         """FP64 (H + PlusI I) X recomputed from coordinates (X [3n] or [3n, r])."""
-        Y = torch.empty_like(X)
         columns = X.numel() // max(1, 3 * self.n_atoms)
-        tiled = (self.nnzb * columns >= self.__dict__.get("_apply_line", TILE_APPLY_TERMS) and X.numel() > 0
-                 and X.dtype == torch.float64 and Y.is_contiguous())
-        if tiled and self._at_hand("_tiles") and self.tiles() is not None:
-            # a later change of the module's line does not move products that took the tiles
+        tiled = self.nnzb * columns >= self.__dict__.get("_apply_line", TILE_APPLY_TERMS)
+        if tiled:     # a later change of the module's line does not move products that took the tiles
             self.__dict__.setdefault("_apply_line", TILE_APPLY_TERMS)
+        return self._matfree(X, tiled)
+
+    def _matfree(self, X, tiled=True):
+        """matfree with the choice of the tiles left to the caller: solvers, whose filters and bounds lay them out
+        anyway, take them at every size."""
+        Y = torch.empty_like(X)
+        tiled = tiled and X.numel() > 0 and X.dtype == torch.float64 and Y.is_contiguous()
+        if tiled and self._at_hand("_tiles") and self.tiles() is not None:
             try:
                 # any shape of 3 n_atoms x r values, as the cluster layout's product takes (the periodic one: [3n] or
                 # [3n, r])

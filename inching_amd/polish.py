@@ -47,7 +47,7 @@ def apply_fp64(A, X, operator="matfree"):
     """Y = A X for a row block X [k, n] in float64."""
     Xc = X.T.contiguous()
     if operator == "matfree":
-        Yc = A.matfree(Xc)
+        Yc = getattr(A, "_matfree", A.matfree)(Xc)
     else:
         Yc = A.matmat(Xc, precision="f64")
     return Yc.T.contiguous()

@@ -87,3 +87,13 @@ def test_block_product_without_room_for_its_workspace(cuda, monkeypatch):
     assert A.tiles() is not None
     monkeypatch.setattr(ops, "_scratch", full)
     assert torch.equal(A.matfree(X), want)
+
+
+def test_solver_keeps_to_one_layout(cuda):
+    """A filtered matrix-free solve counts, filters and checks on the tiles, without a second layout for its blocks."""
+    from inching_amd.hessian import rigid_body_basis
+    from inching_amd.pipeline import lowest_modes
+    print("case: layouts of a solve", flush=True)
+    A = _matrix(900)
+    r = lowest_modes(A, 8, Q=rigid_body_basis(A.xyz), precision="mf64")
+    assert r.converged and A.tiles() is not None and "_clusters" not in A.__dict__
