@@ -55,6 +55,13 @@ def _scratch(k, dtype, device, stream):
         return torch.empty(k, dtype=dtype, device=device)
 
 
+def _after_current(stream, device):
+    """``stream`` follows what the current stream runs by now, which may still use a block that has since been handed
+    out again for a result of ``stream``'s kernels."""
+    if stream is not None:
+        stream.wait_stream(torch.cuda.current_stream(device))
+
+
 # ------------------------------------------------------------------ host ----
 
 def synth_globule(n, radius, dmin, seed, max_attempts=0):
@@ -133,19 +140,14 @@ def neighbours(xyz, rc, stream=None, ascending=True, wait=True):
     rc = float(rc)
     plan, size, nnz = (C.c_double * 7)(), C.c_int64(0), C.c_int64(0)
 
-    def result(k, dtype):
-        # the caller's memory, from the current stream: what still runs there on a reused block goes before ``stream``
-        t = torch.empty(k, dtype=dtype, device=dev)
-        if stream is not None:
-            stream.wait_stream(torch.cuda.current_stream(dev))
-        return t
-
-    indptr = result(n + 1, torch.int64)
+    indptr = torch.empty(n + 1, dtype=torch.int64, device=dev)
+    _after_current(stream, dev)
     part = _scratch(256 * 6, torch.float64, dev, stream)
     call("inch_cells_plan", n, P(xyz), rc, plan, C.byref(size), P(part), sp)
     work = _scratch(size.value, torch.uint8, dev, stream)
     call("inch_cells_count", n, P(xyz), rc, plan, P(work), size.value, P(indptr), C.byref(nnz), sp)
-    indices = result(max(1, nnz.value), torch.int32)
+    indices = torch.empty(max(1, nnz.value), dtype=torch.int32, device=dev)
+    _after_current(stream, dev)
     call("inch_cells_fill", n, rc, plan, P(work), size.value, P(indptr), P(indices), 1 if ascending else 0, sp)
     if wait:
         (torch.cuda.current_stream(dev) if stream is None else stream).synchronize()
@@ -336,6 +338,7 @@ class Tiles:
         i32 = dict(dtype=torch.int32, device=dev)
         order, start = torch.empty(n, **i32), torch.empty(n + 1, **i32)
         nt = C.c_int64(0)
+        _after_current(stream, dev)
         call("inch_anm_tile_order", n, P(xyz), float(side), tile, P(order), P(start), C.byref(nt), stream_ptr(stream))
         nt = nt.value
         self.shape, self.ntile, self.slots, self.nd = (tile, lanes), nt, nt * tile, 3 * n
@@ -349,11 +352,13 @@ class Tiles:
         blocks, umax = C.c_int64(0), C.c_int32(0)
         head = (n, P(xyz), P(rowptr), P(col), P(images), bx, by, nt, tile, lanes, P(order), P(start), P(self.atoms),
                 P(slot_of), P(self.waves), C.byref(blocks))
+        _after_current(stream, dev)
         call("inch_anm_tiles", *head, ucap, None, None, None, 0, None, None, stream_ptr(stream))
         self.pairs = torch.empty(1024 * max(1, blocks.value), dtype=torch.uint8, device=dev)
         self.ulen = torch.empty(nt, **i32)
         self.ulist = torch.empty(nt * ucap, **i32)
         self.rec = torch.empty(6 * self.slots, dtype=torch.float64, device=dev)
+        _after_current(stream, dev)
         call("inch_anm_tiles", *head, ucap, P(self.ulen), P(self.ulist), P(self.pairs), max(1, blocks.value),
              P(self.rec), C.byref(umax), stream_ptr(stream))
         # the lists at the longest union's stride (a quarter to three quarters of the room they were made in)
@@ -482,10 +487,12 @@ class BsrTiles:
         self.n, self.nnz = n, col.numel()
         order, start = torch.empty(n, **i32), torch.empty(n + 1, **i32)
         nt, umax = C.c_int64(0), C.c_int32(0)
+        _after_current(stream, dev)
         call("inch_anm_tile_order", n, P(xyz), float(side), tile, P(order), P(start), C.byref(nt), stream_ptr(stream))
         self.ntile = nt.value
         self.ulen = torch.empty(self.ntile, **i32)
         head = (n, P(rowptr), P(col), self.ntile, P(order), P(start), tile)
+        _after_current(stream, dev)
         call("inch_bsr_tiles", *head, 0, None, P(self.ulen), None, None, C.byref(umax), stream_ptr(stream))
         self.stride = max(1, umax.value)
         if 24 * self.stride > 65536:
@@ -493,6 +500,7 @@ class BsrTiles:
         self.slots = torch.empty(4 * self.ntile * tile, **i32)
         self.ulist = torch.empty(self.ntile * self.stride, **i32)
         self.uidx = torch.empty(max(1, self.nnz), dtype=torch.int16, device=dev)
+        _after_current(stream, dev)
         call("inch_bsr_tiles", *head, self.stride, P(self.slots), P(self.ulen), P(self.ulist), P(self.uidx), None,
              stream_ptr(stream))
 

@@ -124,3 +124,36 @@ def test_filter_on_another_stream_than_its_operator(cuda):
         op.apply(v, u)
     torch.cuda.synchronize()
     assert torch.equal(u, want)
+
+
+@pytest.mark.parametrize("layout", ["Tiles", "BsrTiles"])
+def test_layouts_wait_for_reused_blocks(cuda, layout):
+    """The layouts' arrays come from the current stream's pool too, with writes to their former tensors still queued."""
+    from inching_amd import ops
+    from inching_amd.hessian import build_hessian
+    print("case: %s after reused blocks" % layout, flush=True)
+    A = build_hessian(globule(3000, seed=5), 8.0, precision=())
+    names = {"Tiles": ["atoms", "waves", "pairs", "ulen", "ulist", "rec"], "BsrTiles": ["slots", "ulen", "ulist", "uidx"]}
+
+    def make(stream):
+        args = ((32, 16),) if layout == "Tiles" else ()
+        return getattr(ops, layout)(A.xyz, A.rowptr, A.col, 10.0, *args, stream=stream)
+
+    want = make(None)
+    want = {k: getattr(want, k).clone() for k in names[layout]}
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    old = make(None)
+    torch.cuda._sleep(LONG)
+    for k in names[layout]:
+        getattr(old, k).fill_(0)
+    del old
+    got = make(s)
+    torch.cuda.synchronize()
+    n = getattr(got, "ntile")
+    for k in names[layout]:
+        a, b = getattr(got, k), want[k]
+        if k == "ulist":          # entries past a tile's union are not written
+            keep = torch.arange(a.numel() // n, device="cuda")[None, :] < want["ulen"][:, None]
+            a, b = a.view(n, -1)[keep], b.view(n, -1)[keep]
+        assert torch.equal(a, b), k
