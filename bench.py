@@ -571,7 +571,7 @@ def kernel_key(kind, A):
                                                        "true" if f & 2 else "false")
     t = "float" if kind == "f32" else "double"
     if cfg == BSR_TILE:
-        return "k_bsr_spmv_tile<%s,%s,%d>" % (t, t, cfg - 3000)
+        return "k_bsr_spmv_tile<%s,%s>" % (t, t)
     if cfg >= 1200:
         return "k_bsr_spmv<%s,%s,%d,unsigned short,true>" % (t, t, cfg - 1200)
     if cfg >= 200:
