@@ -1175,12 +1175,14 @@ __global__ void __launch_bounds__(256) k_tile_fill(int64_t n, int TA, int G, con
   }
 }
 
-// rec[6 q .. 6 q + 2] = coordinates of slot q (zeros for a padding slot), rec[6 q + 3 ..] = 0
+// rec[6 q .. 6 q + 2] = coordinates of slot q (zeros for a padding slot), rec[6 q + 3 ..] = 0. Flags bit 4: an x whose
+// square overflows (the product's dummy records lie as far off).
 __global__ void k_tile_coords(int64_t slots, const int32_t *__restrict__ tile_atoms, const double *__restrict__ xyz,
-                              double *__restrict__ rec) {
+                              double *__restrict__ rec, int32_t *__restrict__ flags) {
   const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (q >= slots) return;
   const int32_t at = tile_atoms[q];
+  if (at >= 0 && !(fabs(xyz[3 * (int64_t)at]) < 1e150)) atomicOr(flags, 16);
   for (int k = 0; k < 3; ++k) {
     rec[6 * q + k] = at >= 0 ? xyz[3 * (int64_t)at + k] : 0.0;
     rec[6 * q + 3 + k] = 0.0;
@@ -1988,7 +1990,7 @@ extern "C" inch_status inch_anm_tiles(int64_t n, const double *xyz, const int64_
     HIP_TRY(hipMemcpyAsync(fl, flags.p, sizeof(fl), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     if (fl[0] & 8) INCH_FAIL(INCH_ERR_INVALID, "inch_anm_tiles: a column lies outside [0, n)");
-    if (fl[0] & 16) INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tiles: squared distances outside 1e-30 .. 1e30");
+    if (fl[0] & 16) INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tiles: squared distances outside 1e-30 .. 1e30, or x beyond 1e150");
     if (fl[0] & 1) INCH_FAIL(INCH_ERR_CAPACITY, "inch_anm_tiles: a tile's neighbours exceed %d", ucap);
     return INCH_OK;
   };
@@ -1996,7 +1998,7 @@ extern "C" inch_status inch_anm_tiles(int64_t n, const double *xyz, const int64_
     INCH_REQUIRE(ulen && ulist && rec && umax_out && ucap > 0 && ucap <= inch_tile_max_union(tile),
                  "inch_anm_tiles: bad args of the fill call");
     INCH_REQUIRE(blocks_out && *blocks_out <= pair_blocks, "inch_anm_tiles: pairs too small");
-    k_tile_coords<<<(unsigned)((slots + bs - 1) / bs), bs, 0, st>>>(slots, tile_atoms, xyz, rec);
+    k_tile_coords<<<(unsigned)((slots + bs - 1) / bs), bs, 0, st>>>(slots, tile_atoms, xyz, rec, (int32_t *)flags.p);
     HIP_TRY(hipGetLastError());
     if (images)
       k_tile_fill<true><<<(unsigned)ntile, 256, 0, st>>>(n, tile, lanes, xyz, rowptr, col, images, box_x, box_y,

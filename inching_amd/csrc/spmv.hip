@@ -12,7 +12,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cfloat>
 #include <mutex>
 
 #include "common.h"
@@ -885,8 +884,7 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
     term(q0, q1, q2);
   };
   // an infinite entry less itself is no zero: such waves skip the dummy's passes
-  const bool odd = !(fabs(v0) <= DBL_MAX && fabs(v1) <= DBL_MAX && fabs(v2) <= DBL_MAX && fabs(p0) < 1e150);
-  if (__any(odd)) {
+  if (__any(!(isfinite(v0) && isfinite(v1) && isfinite(v2)))) {
     const uint32_t lim = 48u * (uint32_t)ul;
     auto one = [&](uint32_t off) {
       const double2 *r = (const double2 *)((const char *)lds + off);

@@ -319,8 +319,8 @@ inch_status inch_anm_matfree_rec(int64_t ncl, const double *rec_in, const double
  * rec float64 [6 tile ntile] (records as inch_anm_records: coordinates, zero vector part) and
  * *umax_out, the longest union (order and tile_start are then unused). INCH_ERR_CAPACITY when a
  * union exceeds ucap, a row has more than 65536 / 48 - tile terms (a repeated column counts as
- * often as it is listed), a squared distance lies outside 1e-30 .. 1e30 or the slots exceed the
- * 32-bit record offsets; syncs. */
+ * often as it is listed), a squared distance lies outside 1e-30 .. 1e30, an x coordinate beyond
+ * 1e150 or the slots exceed the 32-bit record offsets; syncs. */
 inch_status inch_anm_tile_order(int64_t n, const double *xyz, double side, int32_t tile, int32_t *order,
                                 int32_t *tile_start, int64_t *ntile_out, void *stream);
 inch_status inch_anm_tiles(int64_t n, const double *xyz, const int64_t *rowptr, const int32_t *col,

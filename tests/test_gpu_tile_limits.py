@@ -176,3 +176,30 @@ def test_filters_of_the_smallest_degrees(cuda, degree, shift):
     op.apply(v, a)
     Operator(A, "mf64", pol=pol, Q=Q, shift=shift, records=False).apply(v, b)
     assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("x,ok", [(1e149, True), (1e151, False)])
+def test_tiles_of_an_atom_out_of_range(cuda, x, ok):
+    """An atom by itself so far out that its empty passes would overflow leaves the tiles to the other forms."""
+    from inching_amd import ops
+    print("case: an atom at x = %g" % x, flush=True)
+    X = np.random.default_rng(6).uniform(0.0, 4.0, (20, 3))
+    X[7, 0] = x
+    xyz = torch.as_tensor(X, device="cuda")
+    keep = [i for i in range(20) if i != 7]
+    rows = [keep if i != 7 else [7] for i in range(20)]
+    ip = torch.as_tensor(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), device="cuda")
+    ix = torch.as_tensor(np.concatenate(rows).astype(np.int32), device="cuda")
+    if not ok:
+        with pytest.raises(ops.InchingError) as e:
+            ops.Tiles(xyz, ip, ix, 1e160, (32, 16))
+        assert e.value.status == -3
+        return
+    T = ops.Tiles(xyz, ip, ix, 1e160, (32, 16))
+    v = torch.randn(60, dtype=torch.float64, device="cuda")
+    rec, y, u = T.buffers(1)[0], torch.empty(3 * T.slots, dtype=torch.float64, device="cuda"), torch.empty_like(v)
+    ops.rec_pack(T.atoms, v, rec)
+    T.product(rec, None, None, 2.0, y=y)
+    ops.rec_unpack(T.atoms, y, u)
+    assert T.ntile == 1 and torch.equal(u.view(20, 3)[7], 2.0 * v.view(20, 3)[7])
+    assert bool(torch.isfinite(u).all())
