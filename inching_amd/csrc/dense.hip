@@ -27,8 +27,8 @@ constexpr int kGramGrid = 1024;    // most column blocks of a Gram product (at l
 // through LDS with coalesced row loads, the next chunk's in flight while the current one is used;
 // when X and Y are the same rows (SAME) they are staged once. The contraction dimension is the
 // column index i of X and Y. Memory bounds it: 64 x 64 over 900,000 columns took 289 us with both
-// operands staged and a wait on memory per chunk, 164 with the loads ahead (the matrix cores busy for three
-// quarters of it) and 135 without the tiles that mirror others (0.46 GB, 3.4 TB/s); 64 x 6 with its sum took 247, now 94.
+// operands staged and a wait on memory per chunk, 164 with the loads ahead and 134 without the tiles that mirror
+// others (0.46 GB, 3.4 TB/s, the matrix cores busy in 56% of the cycles); 64 x 6 took 247 with its sum, now 94 to 126.
 // v_mfma_f64_16x16x4f64 operand layout: A (16x4): lane l holds A[l%16][l/16];
 // B (4x16): lane l holds B[l/16][l%16]; D (16x16): lane l, element r holds
 // D[(l/16) + 4*r][l%16] (checked on gfx950 with one-hot operands).

@@ -764,13 +764,14 @@ k_matfree_rec(int64_t ncl, const double *__restrict__ rin, const double *__restr
 // entry for all 4) no lane idles on a pair outside the cutoff (0.61 of them are inside) or in a
 // list's last chunk, nothing is masked or branched on, and a neighbour's record is gathered 9
 // instead of 45 times per atom. Measured per product, record form -> tile form: 2.4M-atom
-// assembly 676 -> 419 us, 300,000-atom globule 73 -> 55 us, 1,200 atoms 3.7 -> 3.3 us; a periodic
+// assembly 629 -> 415 us, 300,000-atom globule 73 -> 49 us, 1,200 atoms 3.7 -> 3.3 us; a periodic
 // slab of 60,000 atoms (per-row kernel before) 92 -> 12.5 us. FP64 issue bounds it: 19 FP64
 // operations per pair at the measured rate of three-register FMAs (2.5 ns per wave and SIMD) are
-// 0.21 ms on the assembly; the same kernel without its LDS reads or without staging takes 0.92 of
-// its time. The order of an atom's terms (inch_anm_tiles) keeps the LDS reads of a half wave on
-// different banks: in list order 57% of the LDS cycles were conflicts and the products took 60 us
-// at 300,000 atoms (now 55), 14.2 in the periodic slab (now 12.5) and 432 on the assembly (now 419).
+// 0.21 ms on the assembly; the vector units are busy in 82% of a CU's cycles (478 instructions a wave
+// for 117 neighbours an atom: 19 FP64 operations, two conversions and a reciprocal a pair), the LDS
+// in 57%. The order of an atom's terms (inch_anm_tiles) keeps the LDS reads of a half wave on
+// different banks: in list order 57% of the LDS cycles were conflicts, now 31%, and the products
+// took 3% (assembly) to 14% (periodic slab) longer.
 // Periodic images: a union entry names its image in its low 4 bits, and the shift is added as
 // the record is staged, so the inner loop is the same.
 // The reciprocal: a float32 seed (about 22 bits; the layout keeps r2 inside float32's normal
@@ -937,10 +938,11 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
 // stages the union's coordinates and entries in LDS, and G lanes per atom walk the atom's list,
 // each forming a pair's geometry (12 FP64 operations and the reciprocal's seed) once for the 9 per
 // column. The halves of a component's four entries change places with bit 3 of 3 x the record's
-// number, so that the reads of 16 lanes spread over all banks. FP64 issue bounds it (VALU busy 82%
-// of the time). 100,003 atoms, 64 columns: the kernel on the cluster layout (one column per lane, a
-// third of its pairs outside the cutoff, 44 gathers per atom) took 1.83 ms; this takes 0.63, of
-// which the packing 0.05.
+// number, so that the reads of 16 lanes spread over all banks. Vector issue bounds it (the units are
+// busy in 82% of a CU's cycles), then the LDS (71%, two fifths of that bank conflicts). 100,003
+// atoms, 64 columns: the kernel on the cluster layout (one column per lane, a third of its pairs
+// outside the cutoff, 44 gathers per atom) took 1.83 ms; this takes 0.64, of which the packing 0.05.
+// The first product of a matrix lays the tiles out besides: 1.4 ms.
 constexpr int kBlockCols = 4;
 constexpr int kBlockPass = 64;   // columns packed and multiplied at a time: the workspace stays at 1.5 KB a slot
 constexpr size_t kTileBlockLds = 160 * 1024;
@@ -2252,10 +2254,6 @@ int64_t inch_dcgs2_work_size(int32_t J) { return dcgs2_words(J); }
 
 namespace {
 
-// The kernels of one delayed-CGS2 step on the scratch `work` (inch_dcgs2_work_size(J) doubles:
-// per-block partial dots, the reduced dots, the coefficients, the norm partials). Every word
-// of `work` that a kernel reads was written earlier in the same step, so the scratch needs no
-// clearing between steps.
 template <bool SUB>
 inch_status launch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V, int64_t ld, const double *W,
                               double *out, int64_t ld_out, hipStream_t st) {
@@ -2275,6 +2273,10 @@ inch_status launch_rr_combine(int64_t len, int32_t m, int32_t k, const double *V
   return INCH_OK;
 }
 
+// The kernels of one delayed-CGS2 step on the scratch `work` (inch_dcgs2_work_size(J) doubles:
+// per-block partial dots, the reduced dots, the coefficients, the norm partials). Every word
+// of `work` that a kernel reads was written earlier in the same step, so the scratch needs no
+// clearing between steps.
 inch_status dcgs2_launch(int64_t len, int32_t J, double *V, int64_t ld, double *u, double *alpha,
                          const double *beta, double *beta_out, double *vnext, double *work, hipStream_t st) {
   const int tiles = (J + 7) / 8;
