@@ -1291,8 +1291,9 @@ inch_status cell_grid(int64_t n, const double *xyz, double rc, double *part, Gri
   ncell = 1;
   for (int a = 0; a < 3; ++a) {
     const double d = std::floor((hi[a] - g.lo[a]) * g.inv) + 1.0;
-    if (!(d < 1.1e9)) INCH_FAIL(INCH_ERR_CAPACITY, "%s: %g cells along one axis", who, d);
-    g.dim[a] = std::max<int64_t>(1, (int64_t)d);
+    // beyond what cells can be numbered by: one for all (cell_coord cuts there), as long as the other axes have few
+    if (d >= 1.1e9 && d < 9.2e18) INCH_FAIL(INCH_ERR_CAPACITY, "%s: %g cells along one axis", who, d);
+    g.dim[a] = d < 1.1e9 ? std::max<int64_t>(1, (int64_t)d) : 1;
     if (ncell > ((int64_t)1 << 30) / g.dim[a]) INCH_FAIL(INCH_ERR_CAPACITY, "%s: more than 2^30 cells", who);
     ncell *= g.dim[a];
   }

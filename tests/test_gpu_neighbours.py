@@ -126,3 +126,21 @@ def test_one_call_search_equals_the_steps(cuda, case):
         with pytest.raises(ops.InchingError) as e:
             call(ix, nnz.value)
         assert e.value.status == -3
+
+
+@pytest.mark.parametrize("far", [1e5, 1e25, 1e300, 1.5e308])
+@pytest.mark.parametrize("axis", [0, 2])
+def test_neighbours_across_any_span(cuda, far, axis):
+    """Atoms a few cells or any distance apart, the span's overflow included: brute force, and built either way."""
+    from inching_amd import ops
+    from inching_amd.hessian import build_hessian
+    print("case: atoms %g apart along %d" % (far, axis), flush=True)
+    X = np.random.default_rng(4).uniform(0.0, 6.0, (40, 3))
+    X[3, axis], X[20, axis] = far, -far
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = _brute(X, 8.0)
+    ip, ix = ops.neighbours(torch.as_tensor(X, device="cuda"), 8.0)
+    for i, row in enumerate(_rows(ip, ix)):
+        assert np.array_equal(row, np.nonzero(want[i])[0]), i
+    A = build_hessian(X, 8.0, precision=())
+    assert A.nnzb == int(want.sum())
