@@ -49,12 +49,12 @@ class Operator:
         self.shift = float(shift)
         use_rec = RECORDS if records is None else bool(records)
         # a launch code for the matrix's order (other than the cluster layout's) asks for that order
+        # (a code of the cluster layout's lays it out here, not inside a caller's capture)
         rec_ok = (pol is not None and precision == "mf64" and use_rec
-                  and (lanes is None or int(lanes) // 1000 & 4) and A.slot_form() is not None)
+                  and (lanes is None or (int(lanes) // 1000 & 4 and A.clusters() is not None))
+                  and A.slot_form() is not None)
         if lanes is not None:
             self.lanes = int(lanes)
-            if rec_ok:
-                A.clusters()      # asked for by name: laid out here, not inside a caller's capture
         elif rec_ok:
             self.lanes = None     # plain products only: picked when the first one comes
         elif tune:
