@@ -775,12 +775,11 @@ k_matfree_rec(int64_t ncl, const double *__restrict__ rin, const double *__restr
 // Periodic images: a union entry names its image in its low 4 bits, and the shift is added as
 // the record is staged, so the inner loop is the same.
 // The reciprocal: a float32 seed (about 22 bits; the layout keeps r2 inside float32's normal
-// range) and one third-order step, inv + inv (e + e^2) with e = 1 - r2 inv, whose error e^3 is
-// below 2^-64 before its rounding. The step is taken on the reciprocal, not on the product with
-// it: an infinite entry would meet a factor e of either sign.
+// range) and one third-order step, s = q + q (e + e^2) with q = dw inv, e = 1 - r2 inv, whose
+// error e^3 is below 2^-64: two roundings, as in the product with the rounded reciprocal.
 // Passes that a row does not fill read the atom's dummy record, at the atom's own vector
-// entries and another place, so that its term is exactly zero; with an entry that is not finite
-// these passes are skipped.
+// entries and another place, so that its term is exactly zero (sums that are not finite are
+// formed again without them).
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double v) {
   const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
@@ -808,7 +807,7 @@ __device__ __forceinline__ double group_sum(double v) {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <int TA, int G, bool PBC>
-__global__ void __launch_bounds__(TA *G)
+__global__ void __launch_bounds__(TA *G) __attribute__((amdgpu_waves_per_eu(8)))   // 64 registers
 k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__restrict__ rz, double *__restrict__ rout,
                double *__restrict__ yout, const int32_t *__restrict__ ulen, const uint32_t *__restrict__ ulist,
                int ucap, const int2 *__restrict__ waves, const u32x4 *__restrict__ pairs, double bx, double by,
@@ -872,7 +871,8 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
     const double dw = __builtin_fma(d2, w2, __builtin_fma(d1, w1, d0 * w0));
     const double inv = (double)__builtin_amdgcn_rcpf((float)rr2);
     const double e = __builtin_fma(-rr2, inv, 1.0);
-    const double s = dw * __builtin_fma(inv, __builtin_fma(e, e, e), inv);
+    const double q = dw * inv;
+    const double s = __builtin_fma(q, __builtin_fma(e, e, e), q);
     a0 = __builtin_fma(d0, s, a0);
     a1 = __builtin_fma(d1, s, a1);
     a2 = __builtin_fma(d2, s, a2);
@@ -884,35 +884,34 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
     term(r0, r1, r2);
     term(q0, q1, q2);
   };
-  // an infinite entry less itself is no zero: such waves skip the dummy's passes
-  if (__any(!(isfinite(v0) && isfinite(v1) && isfinite(v2)))) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (2 * q < passes) two(ix[q]);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (8 + 2 * q < passes) two(iy[q]);
+  for (int k = 16; k < passes; k += 8) {
+    const u32x4 iz = pl[8 * k];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (k + 2 * q < passes) two(iz[q]);
+  }
+  // sums that are not finite: an infinite entry less itself is a NaN in the empty passes, and q's correction has either
+  // sign. Such waves sum again, without the empty passes and with the step on the reciprocal.
+  if (__any(!(isfinite(a0) && isfinite(a1) && isfinite(a2)))) {
     const uint32_t lim = 48u * (uint32_t)ul;
-    auto one = [&](uint32_t off) {
-      const double2 *r = (const double2 *)((const char *)lds + off);
-      if (off < lim) term(r[0], r[1], r[2]);
-    };
-    for (int k = 0; k < passes; k += 8) {
-      const u32x4 iz = pl[8 * k];
-#pragma unroll 1
-      for (int q = 0; q < 4; ++q)
-        if (k + 2 * q < passes) {
-          const uint32_t pair = q < 2 ? (q ? iz[1] : iz[0]) : (q < 3 ? iz[2] : iz[3]);
-          one(pair & 0xffffu);
-          one(pair >> 16);
-        }
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (2 * q < passes) two(ix[q]);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (8 + 2 * q < passes) two(iy[q]);
-    for (int k = 16; k < passes; k += 8) {
-      const u32x4 iz = pl[8 * k];
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (k + 2 * q < passes) two(iz[q]);
+    a0 = a1 = a2 = 0.0;
+    for (int k = 0; k < passes; ++k) {
+      const uint32_t off = ((const uint16_t *)(pl + 64 * (k >> 3)))[k & 7];
+      if (off >= lim) continue;
+      const double *r = (const double *)((const char *)lds + off);
+      const double d0 = r[0] - p0, d1 = r[1] - p1, d2 = r[2] - p2;
+      const double w0 = v0 - r[3], w1 = v1 - r[4], w2 = v2 - r[5];
+      const double s = __builtin_fma(d2, w2, __builtin_fma(d1, w1, d0 * w0)) *
+                       recip_r2(__builtin_fma(d2, d2, __builtin_fma(d1, d1, d0 * d0)));
+      a0 = __builtin_fma(d0, s, a0);
+      a1 = __builtin_fma(d1, s, a1);
+      a2 = __builtin_fma(d2, s, a2);
     }
   }
   a0 = group_sum<G>(a0);
