@@ -764,12 +764,12 @@ k_matfree_rec(int64_t ncl, const double *__restrict__ rin, const double *__restr
 // entry for all 4) no lane idles on a pair outside the cutoff (0.61 of them are inside) or in a
 // list's last chunk, nothing is masked or branched on, and a neighbour's record is gathered 9
 // instead of 45 times per atom. Measured per product, record form -> tile form: 2.4M-atom
-// assembly 629 -> 415 us, 300,000-atom globule 73 -> 49 us, 1,200 atoms 3.7 -> 3.3 us; a periodic
+// assembly 629 -> 412 us, 300,000-atom globule 73 -> 48 us, 1,200 atoms 3.7 -> 3.3 us; a periodic
 // slab of 60,000 atoms (per-row kernel before) 92 -> 12.5 us. FP64 issue bounds it: 19 FP64
 // operations per pair at the measured rate of three-register FMAs (2.5 ns per wave and SIMD) are
-// 0.21 ms on the assembly; the vector units are busy in 82% of a CU's cycles (478 instructions a wave
+// 0.21 ms on the assembly; the vector units are busy in 85% of a CU's cycles (479 instructions a wave
 // for 117 neighbours an atom: 19 FP64 operations, two conversions and a reciprocal a pair), the LDS
-// in 57%. The order of an atom's terms (inch_anm_tiles) keeps the LDS reads of a half wave on
+// in 59%. The order of an atom's terms (inch_anm_tiles) keeps the LDS reads of a half wave on
 // different banks: in list order 57% of the LDS cycles were conflicts, now 31%, and the products
 // took 3% (assembly) to 14% (periodic slab) longer.
 // Periodic images: a union entry names its image in its low 4 bits, and the shift is added as
