@@ -896,9 +896,13 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
     for (int q = 0; q < 4; ++q)
       if (k + 2 * q < passes) two(iz[q]);
   }
-  // sums that are not finite: an infinite entry less itself is a NaN in the empty passes, and q's correction has either
-  // sign. Such waves sum again, without the empty passes and with the step on the reciprocal.
-  if (__any(!(isfinite(a0) && isfinite(a1) && isfinite(a2)))) {
+  a0 = group_sum<G>(a0);
+  a1 = group_sum<G>(a1);
+  a2 = group_sum<G>(a2);
+  double sum = l == 0 ? a0 : (l == 1 ? a1 : a2);
+  // a sum that is not finite: an infinite entry less itself is a NaN in the empty passes, and q's correction has either
+  // sign. Such waves sum again, without the empty passes and with the reciprocal of the record form.
+  if (__any(!isfinite(sum))) {
     const uint32_t lim = 48u * (uint32_t)ul;
     a0 = a1 = a2 = 0.0;
     for (int k = 0; k < passes; ++k) {
@@ -913,13 +917,14 @@ k_matfree_tile(int64_t slots, const double *__restrict__ rin, const double *__re
       a1 = __builtin_fma(d1, s, a1);
       a2 = __builtin_fma(d2, s, a2);
     }
+    a0 = group_sum<G>(a0);
+    a1 = group_sum<G>(a1);
+    a2 = group_sum<G>(a2);
+    sum = l == 0 ? a0 : (l == 1 ? a1 : a2);
   }
-  a0 = group_sum<G>(a0);
-  a1 = group_sum<G>(a1);
-  a2 = group_sum<G>(a2);
   if (l >= 3) return;
   const double xv = l == 0 ? v0 : (l == 1 ? v1 : v2);
-  double out = (l == 0 ? a0 : (l == 1 ? a1 : a2)) + plus_i * xv;
+  double out = sum + plus_i * xv;
   if (c0 != 0.0) out -= c0 * xv;
   out *= s1;
   if (rz) out -= c2 * zv;
